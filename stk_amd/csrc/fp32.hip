@@ -3,11 +3,15 @@
 // The reference's launchers pass whatever dtype the tensors have to kernels that accumulate in fp32
 // (stk/backend/triton_kernels.py:250, 306, 358; ACC_TYPE :248): float32 operands are legal there.  The 16-bit
 // tile engine (gemm_core.h) does not take them, so stk_sdd / stk_dsd / stk_dds hand STK_F32 problems to the
-// kernels here: one workgroup of four wavefronts per BLK x BLK output tile, v_mfma_f32_32x32x2_f32 on operand
-// tiles staged through LDS as [k][m] and [k][n], 16 k at a time, the next K-tile on its way in registers while
-// the current one is multiplied.  Operands are read with their element strides as they are (row-major, .t()
-// views or anything else), so nothing is copied or converted; ragged dense extents are predicated.  The walks
-// are those of the 16-bit kernels.  A plan, a workspace or a block order are ignored: results never depend on them.
+// kernels here, all on v_mfma_f32_32x32x2_f32 (256 FLOP per cycle and compute unit, a sixteenth of the bf16 rate: it is
+// the matrix pipe that bounds them, and what is left to choose is how many compute units get work).  Two sets:
+//   Fast     operands with a unit stride, 16-byte aligned, extents that are whole tiles: operand tiles go from memory
+//            to LDS without passing through registers, in a ring of two to four K-tiles of 32; output tiles of
+//            128x128, 64x64 or 32x32 (fast_tile).
+//   generic  any strides and ragged dense extents: one BLK x BLK tile per workgroup of four wavefronts, 16 k at a time
+//            through registers, predicated.
+// The walks are those of the 16-bit kernels.  A plan, a workspace or a block order are ignored: results never depend
+// on them.
 #include "common.h"
 #include "gemm_core.h"
 
@@ -198,6 +202,245 @@ __global__ __launch_bounds__(kThreads) void walk_kernel(WalkArgs g) {
   else t.store(g.out + (int64_t)f0 * g.ldc + (int64_t)line * BLK, g.ldc, valid, BLK, kNoActivation, nullptr);
 }
 
+// ---------------------------------------------------------------------------
+// Fast set.
+//
+// An operand tile is EXT (m or n extent) x kFastKT k, in LDS as it lies in memory: K-major [EXT][32 k], 128-byte rows,
+// or MN-major [32 k][EXT].  A wavefront's 1 KiB transfer fills consecutive LDS bytes, so the swizzles that keep the
+// reads free of bank conflicts are applied by choosing which 16-byte piece a lane fetches.  In a group of eight k the
+// lanes of the lower half hold k 0..3 and those of the upper half k 4..7: a K-major operand is then read as one
+// 16-byte piece per lane for four MFMAs, an MN-major one as a 4-byte word per MFMA.
+// ---------------------------------------------------------------------------
+constexpr int kFastKT = 32;
+
+template <int EXT, bool KMAJOR>
+struct FastOperand {
+  static constexpr int kBytes = EXT * kFastKT * 4;
+  static constexpr int kSlices = kBytes / 1024;
+  static constexpr int kPerWave = kSlices / 4;
+  static_assert(kSlices % 4 == 0, "whole transfers per wavefront");
+  // Byte offset from the tile's origin of what lane `lane` fetches for slice `slice`; ld in elements.
+  __device__ __forceinline__ static uint32_t source(int slice, int lane, int64_t ld) {
+    if constexpr (KMAJOR) {
+      const int row = slice * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+      return (uint32_t)((row * ld + piece * 4) * 4);
+    } else {
+      constexpr int kPieces = EXT / 4;  // per k row
+      const int k = slice * (64 / kPieces) + lane / kPieces;
+      const int byte = ((lane % kPieces) << 4) ^ swizzle(k);
+      return (uint32_t)(k * ld * 4 + byte);
+    }
+  }
+  // Rows k and k + 4 are read together, 128 bytes of each: when the rows are multiples of the 256 bytes of banks apart
+  // the second one is kept with its 128-byte halves swapped.
+  __device__ __forceinline__ static int swizzle(int k) { return EXT >= 64 ? ((k >> 2) & 1) << 7 : 0; }
+  // f[j] = element (mn + lane % 32, k = 8 group + 4 (lane / 32) + j)
+  __device__ __forceinline__ static void frag(const char* s, int mn, int group, int lane, float (&f)[4]) {
+    if constexpr (KMAJOR) {
+      const int row = mn + (lane & 31), piece = (2 * group + (lane >> 5)) ^ ((row >> 1) & 7);
+      const f32x4 v = *reinterpret_cast<const f32x4*>(s + row * 128 + piece * 16);
+#pragma unroll
+      for (int j = 0; j < 4; j++) f[j] = v[j];
+    } else {
+      const int k = 8 * group + 4 * (lane >> 5);
+      const char* at = s + k * (EXT * 4) + ((4 * (mn + (lane & 31))) ^ swizzle(k));
+#pragma unroll
+      for (int j = 0; j < 4; j++) f[j] = *reinterpret_cast<const float*>(at + j * (EXT * 4));
+    }
+  }
+};
+
+// T x T output tile of four wavefronts: 2 x 2 of (T / 2) x (T / 2), or for T = 32 one tile whose K-tiles are split over
+// the wavefronts (8 k each) and added up at the end, in the order of the wavefronts.
+template <int T, bool AK, bool BK>
+struct Fast {
+  static constexpr int kStages = T == 128 ? 2 : T == 64 ? 3 : 4;
+  static constexpr int kW = T == 128 ? 2 : 1;  // 32x32 MFMA tiles per wavefront in each direction
+  static constexpr bool kSplit = T == 32;
+  using OpA = FastOperand<T, AK>;
+  using OpB = FastOperand<T, BK>;
+  static constexpr int kStageBytes = OpA::kBytes + OpB::kBytes;
+  static constexpr int kLds = kStages * kStageBytes;  // (T = 32: 32 KiB, of which the partial sums use 16)
+  static constexpr int kLoads = OpA::kPerWave + OpB::kPerWave;
+  f32x16_t acc[kW][kW];
+
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < kW; i++)
+#pragma unroll
+      for (int j = 0; j < kW; j++) acc[i][j] = f32x16_t{};
+  }
+
+  // acc += the `ntiles` K-tiles whose origins tile_fn(t, a, b) gives (called once per t, in increasing order)
+  template <class TileFn>
+  __device__ __forceinline__ void accumulate(int ntiles, int64_t lda, int64_t ldb, char* smem, TileFn&& tile_fn) {
+    const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)((STK_LDS char*)smem);
+    uint32_t offa[OpA::kPerWave], offb[OpB::kPerWave];
+#pragma unroll
+    for (int i = 0; i < OpA::kPerWave; i++) offa[i] = OpA::source(i * 4 + wave, lane, lda);
+#pragma unroll
+    for (int i = 0; i < OpB::kPerWave; i++) offb[i] = OpB::source(i * 4 + wave, lane, ldb);
+    auto issue = [&](int t) {
+      const float *a, *b;
+      tile_fn(t, a, b);
+      const gptr_t ga = uniform_global(a), gb = uniform_global(b);
+      const uint32_t stage = lds0 + (uint32_t)(t % kStages) * kStageBytes;
+#pragma unroll
+      for (int i = 0; i < OpA::kPerWave; i++) dma16(ga, offa[i], stage + (i * 4 + wave) * 1024);
+#pragma unroll
+      for (int i = 0; i < OpB::kPerWave; i++) dma16(gb, offb[i], stage + OpA::kBytes + (i * 4 + wave) * 1024);
+    };
+#pragma unroll
+    for (int t = 0; t < kStages - 1; t++)
+      if (t < ntiles) issue(t);
+    const int m0 = kSplit ? 0 : (wave & 1) * (T / 2), n0 = kSplit ? 0 : (wave >> 1) * (T / 2);
+    for (int t = 0; t < ntiles; t++) {
+      // K-tile t has landed; up to kStages - 2 younger ones may stay in flight
+      const int younger = ntiles - 1 - t;
+      if (kStages >= 4 && younger >= 2) wait_vmcnt<2 * kLoads>();
+      else if (kStages >= 3 && younger >= 1) wait_vmcnt<1 * kLoads>();
+      else wait_vmcnt<0>();
+      __syncthreads();  // every wavefront's part of K-tile t is there, and K-tile t - 1, whose stage is refilled, has been read
+      if (t + kStages - 1 < ntiles) issue(t + kStages - 1);
+      const char* sa = smem + (t % kStages) * kStageBytes;
+      const char* sb = sa + OpA::kBytes;
+#pragma unroll
+      for (int g = 0; g < (kSplit ? 1 : 4); g++) {
+        const int group = kSplit ? wave : g;
+        float fa[kW][4], fb[kW][4];
+#pragma unroll
+        for (int i = 0; i < kW; i++) OpA::frag(sa, m0 + 32 * i, group, lane, fa[i]);
+#pragma unroll
+        for (int j = 0; j < kW; j++) OpB::frag(sb, n0 + 32 * j, group, lane, fb[j]);
+        // operands swapped, as in the 16-bit engine: a lane then owns four consecutive columns of one output row
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+          for (int i = 0; i < kW; i++)
+#pragma unroll
+            for (int j = 0; j < kW; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j][q], fa[i][q], acc[i][j], 0, 0, 0);
+      }
+    }
+    __syncthreads();  // the ring has been read: it is filled again, or used for the partial sums
+  }
+
+  // out[m * ldc + n] = act(acc) (* mul[m * ldc + n]); out and mul 16-byte aligned with rows at multiples of 16 bytes
+  __device__ __forceinline__ void store(float* out, int64_t ldc, int activation, const float* mul, char* smem) {
+    const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+    auto put = [&](int m, int n, f32x4 v) {
+      const int64_t at = (int64_t)m * ldc + n;
+      if (mul) v *= *reinterpret_cast<const f32x4*>(mul + at);
+      *reinterpret_cast<f32x4*>(out + at) = v;
+    };
+    if constexpr (kSplit) {
+      // wavefront w finishes the columns 8 w + 0..7: values 4 w .. 4 w + 3 of every lane
+      float* part = reinterpret_cast<float*>(smem);
+#pragma unroll
+      for (int r = 0; r < 16; r++) part[(wave * 16 + r) * 64 + lane] = acc[0][0][r];
+      __syncthreads();
+      f32x16_t v = {};
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        float sum = part[(4 * wave + q) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < 4; w++) sum += part[(w * 16 + 4 * wave + q) * 64 + lane];
+        v[q] = sum;
+      }
+      if (activation != kNoActivation) activate_all(v, activation);
+      put(lane & 31, 8 * wave + 4 * (lane >> 5), f32x4{v[0], v[1], v[2], v[3]});
+    } else {
+      const int m0 = (wave & 1) * (T / 2), n0 = (wave >> 1) * (T / 2);
+#pragma unroll
+      for (int i = 0; i < kW; i++)
+#pragma unroll
+        for (int j = 0; j < kW; j++) {
+          if (activation != kNoActivation) activate_all(acc[i][j], activation);
+#pragma unroll
+          for (int g = 0; g < 4; g++)
+            put(m0 + 32 * i + (lane & 31), n0 + 32 * j + 8 * g + 4 * (lane >> 5),
+                f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]});
+        }
+    }
+  }
+};
+
+template <int BLK, int T, bool AK, bool BK>
+__global__ __launch_bounds__(kThreads, 2) void sdd_fast_kernel(SddArgs g, int nnz) {
+  __shared__ __align__(16) char smem[Fast<T, AK, BK>::kLds];
+  constexpr int kSide = BLK / T, kPerBlock = kSide * kSide;
+  const int item = xcd_chunked(blockIdx.x, nnz * kPerBlock);
+  const int p = item / kPerBlock, m0 = item % kPerBlock / kSide * T, n0 = item % kSide * T;
+  const int64_t r = uniform(load_index(g.row_indices, p, g.idx32)), c = uniform(load_index(g.column_indices, p, g.idx32));
+  const float* a0 = g.lhs + (r * BLK + m0) * g.lsm;
+  const float* b0 = g.rhs + (c * BLK + n0) * g.rsn;
+  Fast<T, AK, BK> t;
+  t.clear();
+  t.accumulate(g.k / kFastKT, AK ? g.lsm : g.lsk, BK ? g.rsn : g.rsk, smem, [&](int i, const float*& a, const float*& b) {
+    a = a0 + (int64_t)i * kFastKT * g.lsk;
+    b = b0 + (int64_t)i * kFastKT * g.rsk;
+  });
+  const int64_t at = (int64_t)p * BLK * BLK + m0 * BLK + n0;
+  t.store(g.out + at, BLK, g.activation, g.multiplier ? g.multiplier + at : nullptr, smem);
+}
+
+// One T-wide stretch of a line of op(S) against a T-wide tile of the dense operand.
+template <int BLK, int T, bool SPARSE_LHS, bool AK, bool BK>
+__global__ __launch_bounds__(kThreads, 2) void walk_fast_kernel(WalkArgs g, int items) {
+  __shared__ __align__(16) char smem[Fast<T, AK, BK>::kLds];
+  constexpr int kSide = BLK / T, kPer = BLK / kFastKT;
+  const int tiles = g.free_extent / T;
+  const int item = xcd_chunked(blockIdx.x, items);
+  // (the stretches of a line next to each other: they share the tile of the dense operand)
+  const int stretch = item % kSide, line = item / (kSide * tiles), f0 = item / kSide % tiles * T, l0 = stretch * T;
+  const int lane = threadIdx.x & 63;
+  const int begin = uniform(g.walk_offsets[line]), end = uniform(g.walk_offsets[line + 1]);
+  const float* dense0 = g.dense + (int64_t)f0 * g.ds_outer;
+  const float* data0 = g.data + (int64_t)l0 * g.bs_mn;
+  Fast<T, AK, BK> t;
+  t.clear();
+  for (int s0 = begin; s0 < end; s0 += 64) {
+    const int count = end - s0 < 64 ? end - s0 : 64;
+    // lane i holds the place and the block of walk entry s0 + i: the K loop gets them with a lane read
+    const int e = s0 + (lane < count ? lane : count - 1);
+    const int seg_k = load_index(g.walk_positions, e, g.idx32), seg_block = g.walk_blocks ? g.walk_blocks[e] : e;
+    auto origins = [&](int i, const float*& a, const float*& b) {
+      const int sub = i % kPer * kFastKT;
+      const float* block = data0 + (int64_t)__builtin_amdgcn_readlane(seg_block, i / kPer) * BLK * BLK + sub * g.bs_k;
+      const float* dense = dense0 + ((int64_t)__builtin_amdgcn_readlane(seg_k, i / kPer) * BLK + sub) * g.ds_k;
+      a = SPARSE_LHS ? block : dense;
+      b = SPARSE_LHS ? dense : block;
+    };
+    const int64_t ld_block = BLK, ld_dense = g.ds_k == 1 ? g.ds_outer : g.ds_k;
+    t.accumulate(count * kPer, SPARSE_LHS ? ld_block : ld_dense, SPARSE_LHS ? ld_dense : ld_block, smem, origins);
+  }
+  const int64_t row = SPARSE_LHS ? (int64_t)line * BLK + l0 : f0, col = SPARSE_LHS ? f0 : (int64_t)line * BLK + l0;
+  t.store(g.out + row * g.ldc + col, g.ldc, kNoActivation, nullptr, smem);
+}
+
+// Side of the output tiles for a problem of `area` tiles of 32 x 32 whose extents are multiples of `most`.  The matrix pipe
+// is the bound, so a tile that leaves compute units without work, or with a second tile while others have none, costs in
+// proportion, while a smaller tile than needed moves more operand bytes per FLOP.  Kernel times in us with tiles of 128 /
+// 64 / 32:
+//   sdd, 32 blocks of 128, k = 1024 (32 / 128 / 512 tiles)            66 / 23 / 15
+//   dsd, 1024 x 1024 half full x 1024 (64 / 256 / 1024 tiles)         69 / 26 / 27
+//   dds, 3072 x 3072 half full, 2048 rows (384 / 1536 / 6144 tiles)  254 / 175 / 213
+//   dsd, 4096 x 4096 half full x 4096 (1024 / 4096 / 16384 tiles)    546 / 587 / 728
+// so 64 as soon as every unit gets a tile, 128 from four of them for every unit on.  (Before these kernels, with a 128 x 128
+// tile per block in all of these cases: sdd 69, dsd 68, and 990 for the dsd of 4096 x 4096.)
+inline int fast_tile(int64_t area, int most) {
+  const int64_t units = compute_units() > 0 ? compute_units() : 256;
+  if (most >= 128 && area / 16 >= 4 * units) return 128;
+  return most >= 64 && area / 4 >= units ? 64 : 32;
+}
+
+// A float32 array that the transfers can read: unit stride in one dimension, the other one and the base multiples of 16
+// bytes, and rows of a tile within 32-bit byte offsets of its origin.
+inline bool fast_layout(const void* p, int64_t s0, int64_t s1) {
+  const int64_t ld = s1 == 1 ? s0 : s1;
+  return aligned16(p) && (s0 == 1 || s1 == 1) && ld > 0 && ld % 4 == 0 && ld < (1 << 22);
+}
+
 }  // namespace f32
 
 int sdd_f32(const void* lhs, int64_t lhs_stride_m, int64_t lhs_stride_k, const void* rhs, int64_t rhs_stride_k, int64_t rhs_stride_n,
@@ -216,6 +459,21 @@ int sdd_f32(const void* lhs, int64_t lhs_stride_m, int64_t lhs_stride_k, const v
   const f32::SddArgs g{static_cast<const float*>(lhs), lhs_stride_m, lhs_stride_k, static_cast<const float*>(rhs), rhs_stride_k, rhs_stride_n,
                        (int)k, static_cast<float*>(out), row_indices, column_indices, index_dtype == STK_I32, activation,
                        static_cast<const float*>(multiplier)};
+  if (f32::fast_layout(lhs, lhs_stride_m, lhs_stride_k) && f32::fast_layout(rhs, rhs_stride_k, rhs_stride_n) && aligned16(out) && (!multiplier || aligned16(multiplier))) {
+    const int t = f32::fast_tile(nnz * (blocking / 32) * (blocking / 32), blocking);
+    const bool ak = lhs_stride_k == 1, bk = rhs_stride_n != 1;
+    const int64_t grid = nnz * (blocking / t) * (blocking / t);
+    if (grid <= INT32_MAX) {
+#define STK_F32_SDD(BLK, T, AK, BK)                                                                                              \
+  if (blocking == BLK && t == T && ak == AK && bk == BK)                                                                         \
+    hipLaunchKernelGGL((f32::sdd_fast_kernel<BLK, T, AK, BK>), dim3((unsigned)grid), dim3(f32::kThreads), 0, stream, g, (int)nnz);
+#define STK_F32_SDD_LAYOUTS(BLK, T) STK_F32_SDD(BLK, T, true, true) STK_F32_SDD(BLK, T, true, false) STK_F32_SDD(BLK, T, false, true) STK_F32_SDD(BLK, T, false, false)
+      STK_F32_SDD_LAYOUTS(128, 128) STK_F32_SDD_LAYOUTS(128, 64) STK_F32_SDD_LAYOUTS(128, 32) STK_F32_SDD_LAYOUTS(64, 64) STK_F32_SDD_LAYOUTS(64, 32)
+#undef STK_F32_SDD_LAYOUTS
+#undef STK_F32_SDD
+      return check_launch("stk_sdd");
+    }
+  }
   if (blocking == 128) hipLaunchKernelGGL(f32::sdd_kernel<128>, dim3((unsigned)nnz), dim3(f32::kThreads), 0, stream, g);
   else hipLaunchKernelGGL(f32::sdd_kernel<64>, dim3((unsigned)nnz), dim3(f32::kThreads), 0, stream, g);
   return check_launch("stk_sdd");
@@ -237,6 +495,25 @@ int walk_f32(bool sparse_lhs, const char* who, int64_t lines, int64_t free_exten
   const f32::WalkArgs g{static_cast<const float*>(data), walk_offsets, walk_positions, walk_blocks, static_cast<const float*>(dense),
                         dense_stride_free, dense_stride_k, line_major ? b : 1, line_major ? 1 : b,
                         static_cast<float*>(out), out_stride_m, (int)free_extent, index_dtype == STK_I32};
+  const int side = free_extent % 128 == 0 ? 128 : free_extent % 64 == 0 ? 64 : free_extent % 32 == 0 ? 32 : 0;
+  if (side && f32::fast_layout(dense, dense_stride_free, dense_stride_k) && aligned16(data) && aligned16(out) && out_stride_m % 4 == 0) {
+    const int t = f32::fast_tile(lines * (b / 32) * (free_extent / 32), side < blocking ? side : blocking);
+    const int64_t items = lines * (b / t) * (free_extent / t);
+    if (items <= INT32_MAX) {
+      // K-major operands: stored blocks whose rows run along the line, a dense operand with unit stride along k
+      const bool sk = line_major, dk = dense_stride_k == 1;
+#define STK_F32_WALK(BLK, T, SL, SK, DK)                                                                                               \
+  if (blocking == BLK && t == T && sparse_lhs == SL && sk == SK && dk == DK)                                                           \
+    hipLaunchKernelGGL((f32::walk_fast_kernel<BLK, T, SL, SL ? SK : DK, SL ? DK : SK>), dim3((unsigned)items), dim3(f32::kThreads), 0, stream, g, (int)items);
+#define STK_F32_WALK_LAYOUTS(BLK, T, SL) STK_F32_WALK(BLK, T, SL, true, true) STK_F32_WALK(BLK, T, SL, true, false) STK_F32_WALK(BLK, T, SL, false, true) STK_F32_WALK(BLK, T, SL, false, false)
+#define STK_F32_WALKS(BLK, T) STK_F32_WALK_LAYOUTS(BLK, T, true) STK_F32_WALK_LAYOUTS(BLK, T, false)
+      STK_F32_WALKS(128, 128) STK_F32_WALKS(128, 64) STK_F32_WALKS(128, 32) STK_F32_WALKS(64, 64) STK_F32_WALKS(64, 32)
+#undef STK_F32_WALKS
+#undef STK_F32_WALK_LAYOUTS
+#undef STK_F32_WALK
+      return check_launch(who);
+    }
+  }
   const dim3 grid((unsigned)(lines * tiles));
   if (sparse_lhs) {
     if (blocking == 128) hipLaunchKernelGGL((f32::walk_kernel<128, true>), grid, dim3(f32::kThreads), 0, stream, g);
