@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define STK_AMD_ABI_VERSION 16
+#define STK_AMD_ABI_VERSION 17
 
 /* status codes */
 #define STK_OK 0
@@ -406,6 +406,18 @@ int stk_dmoe_topology(const int32_t* padded_bins, int64_t num_experts, int block
                       int32_t* offsets, void* row_indices, void* column_indices,
                       int32_t* offsets_t, void* column_indices_t, int32_t* block_offsets_t,
                       stk_stream_t stream);
+
+/*
+ * stk_dmoe_topology that also builds the fusion plan of the topology (for both directions), in the same launch: plan
+ * holds stk_plan_bytes(block_rows, num_experts * blocks_per_row, nnz) bytes, 4-byte aligned.  The tiles, lists and hints
+ * are those of stk_build_plan; the role arrays, which no product reads, are left as they are.  Blocking 64 or 128, at
+ * most 1024 experts and at least one block (STK_ERR_UNSUPPORTED otherwise; plan == NULL: stk_dmoe_topology).
+ */
+int stk_dmoe_topology_plan(const int32_t* padded_bins, int64_t num_experts, int blocking, int64_t block_rows,
+                           int64_t blocks_per_row, int index_dtype,
+                           int32_t* offsets, void* row_indices, void* column_indices,
+                           int32_t* offsets_t, void* column_indices_t, int32_t* block_offsets_t,
+                           uint8_t* plan, size_t plan_bytes, stk_stream_t stream);
 
 /*
  * Token routing of a dropless mixture-of-experts layer: the producer of the rows that

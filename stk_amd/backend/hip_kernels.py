@@ -143,8 +143,8 @@ def _plan_cache_get(tensors, blocking):
 
 def _plan_cache_put(tensors, blocking, plan, stream_handle, built, capture):
     """Remembers `plan` on tensors[0]; tensors without a version counter (made under inference mode)
-    cannot be watched for in-place changes and are not cached.  `capture`: the graph capture the plan was built in
-    (0: none)."""
+    cannot be watched for in-place changes and are not cached.  `built`: the torch stream whose handle is
+    stream_handle, on which the plan was built; `capture`: the graph capture it was built in (0: none)."""
     versions = tuple(_version_of(t) for t in tensors)
     if None in versions:
         return False
@@ -178,7 +178,7 @@ def fusion_plan(offsets, column_indices, offsets_t=None, column_indices_t=None, 
         if built_in in (0, capture):
             if cached[3] != handle and (built_in != 0 or capture == 0):
                 # built on another stream: what this one launches next comes after the build
-                torch.cuda.current_stream(offsets.device).wait_event(cached[4])
+                torch.cuda.current_stream(offsets.device).wait_stream(cached[4])
             return cached[1]
     else:
         capture = _capture_id(offsets.device)
@@ -196,9 +196,7 @@ def fusion_plan(offsets, column_indices, offsets_t=None, column_indices_t=None, 
             _offsets(offsets_t).data_ptr() if want_cols else None, cit.data_ptr() if want_cols else None, block_cols,
             nnz, blocking, _INDEX_DTYPES[ci.dtype], plan.data_ptr(), nbytes, _stream()))
     stream = torch.cuda.current_stream(offsets.device)
-    built = torch.cuda.Event()
-    built.record(stream)
-    _plan_cache_put(tensors, blocking, plan, stream.cuda_stream, built, capture)
+    _plan_cache_put(tensors, blocking, plan, stream.cuda_stream, stream, capture)
     return plan
 
 
@@ -537,10 +535,14 @@ def transpose_meta(size, data, row_indices, column_indices, offsets):
     return column_indices_t, offsets_t, block_offsets_t
 
 
+DMOE_PLAN_EXPERTS = 1024   # up to this many experts stk_dmoe_topology_plan builds the plan (their shares fit in LDS)
+
+
 def dmoe_topology(padded_bins, blocking, block_rows, blocks_per_row, index_dtype=torch.int16):
     """(offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t) of the
     block-diagonal dropless-MoE pattern, one launch, no sort.  padded_bins: int32 device tensor,
-    inclusive prefix sum of the per-expert row counts (each a multiple of `blocking`)."""
+    inclusive prefix sum of the per-expert row counts (each a multiple of `blocking`).  The launch also
+    builds the fusion plan, which the products on the topology then find on `offsets`."""
     _need_gpu(padded_bins)
     assert padded_bins.dim() == 1 and padded_bins.numel() > 0
     bins = _offsets(padded_bins)
@@ -553,11 +555,20 @@ def dmoe_topology(padded_bins, blocking, block_rows, blocks_per_row, index_dtype
     column_indices = torch.empty(nnz, dtype=index_dtype, device=dev)
     column_indices_t = torch.empty(nnz, dtype=index_dtype, device=dev)
     block_offsets_t = torch.empty(nnz, dtype=torch.int32, device=dev)
+    lib = _lib.load()
+    plan, nbytes = None, 0
+    if FUSION and blocking in (64, 128) and nnz > 0 and experts <= DMOE_PLAN_EXPERTS:
+        nbytes = lib.stk_plan_bytes(block_rows, experts * blocks_per_row, nnz)
+        plan = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     with _on_device(dev):
-        _lib.check(_lib.load().stk_dmoe_topology(
+        _lib.check(lib.stk_dmoe_topology_plan(
             bins.data_ptr(), experts, blocking, block_rows, blocks_per_row, _INDEX_DTYPES[index_dtype],
             offsets.data_ptr(), row_indices.data_ptr(), column_indices.data_ptr(),
-            offsets_t.data_ptr(), column_indices_t.data_ptr(), block_offsets_t.data_ptr(), _stream()))
+            offsets_t.data_ptr(), column_indices_t.data_ptr(), block_offsets_t.data_ptr(),
+            plan.data_ptr() if plan is not None else None, nbytes, _stream()))
+    if plan is not None:
+        stream = torch.cuda.current_stream(dev)
+        _plan_cache_put((offsets, column_indices, offsets_t, column_indices_t), blocking, plan, stream.cuda_stream, stream, _capture_id(dev))
     return offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t
 
 

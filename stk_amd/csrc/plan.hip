@@ -38,89 +38,12 @@
 //   list 2 (tall 1's place)  of pairs                           list 4 (tall 0's place)  lone lines
 // with list 1 empty.
 #include "common.h"
+#include "plan_sim.h"
 #include "wave_scan.h"
 
 namespace stk {
 
-// When the tiles of a launch fill the compute units a few times only, the last round
-// leaves most of them idle.  Cutting the tiles of that round into k slices along the
-// contraction (workgroups add the partial tiles up) fills the round better, at the price of
-// the partial tiles' round trip through memory.  Which k pays is found by playing the
-// hardware's dispatch through: workgroups start in order, each on the compute unit that
-// is free first.  Tiles of one kind take equally long here (the lines' average length), so
-// the compute units are kept as a few groups (free time, how many) in ascending order.
-constexpr int kSortCapacity = 4096;  // lone lines that are put in order of their lengths (more: left as they are)
-constexpr int kSimGroups = 24;    // groups alive at a time
-constexpr int kSimCapacity = 48;  // room for the queue to move along before it is shifted back
-struct DispatchSim {
-  float* time;  // kSimCapacity entries each, private to the thread
-  int* count;
-  int head, tail;  // the groups are entries [head, tail), ascending in time
-  __host__ __device__ void reset(int units) { time[0] = 0.f, count[0] = units, head = 0, tail = 1; }
-  // n work items of the same duration
-  __host__ __device__ void run(int n, float duration) {
-    while (n > 0) {
-      const int m = n < count[head] ? n : count[head];
-      const float t = time[head] + duration;
-      n -= m;
-      count[head] -= m;
-      if (count[head] == 0) head++;
-      if (tail == kSimCapacity) {
-        for (int i = head; i < tail; i++) time[i - head] = time[i], count[i - head] = count[i];
-        tail -= head, head = 0;
-      }
-      int at = tail;
-      while (at > head && time[at - 1] > t) at--;
-      if (at > head && time[at - 1] == t) {
-        count[at - 1] += m;
-      } else if (tail - head == kSimGroups) {
-        // out of groups: join a neighbour (a small error in a rare case)
-        count[at < tail ? at : tail - 1] += m;
-      } else {
-        for (int i = tail; i > at; i--) time[i] = time[i - 1], count[i] = count[i - 1];
-        time[at] = t, count[at] = m, tail++;
-      }
-    }
-  }
-  __host__ __device__ float end() const { return time[tail - 1]; }
-};
-
-// Simulated end of a launch whose last round is cut into k slices.  tiles[]: pairs, threes, lone lines;
-// length: average blocks per line.
-__host__ __device__ inline float simulate_launch(DispatchSim& sim, const int (&tiles)[3], float length, int units, int k) {
-  // Durations in units of one block of k of a 256x256 tile (about 5 us).  Measured on an MI355X: a workgroup
-  // spends about 4 such units outside its K loop (start, first loads, store), and 2 more when its tile is a
-  // slice (partial tile out to memory and back in, the counter); 384x128 and 128x256 tiles take 0.75 and 0.58
-  // of a 256x256 tile's time per block.
-  const float start = 4.f, seam = 2.f;
-  const float duration[3] = {length, 0.75f * length, 0.58f * length};
-  const int total = tiles[0] + tiles[1] + tiles[2];
-  const int whole = (total - 1) / units * units;
-  sim.reset(units);
-  int left = whole, tail[3];
-  for (int kind = 0; kind < 3; kind++) {
-    const int n = tiles[kind] < left ? tiles[kind] : left;
-    sim.run(n, duration[kind] + start);
-    left -= n;
-    tail[kind] = tiles[kind] - n;
-  }
-  for (int slice = 0; slice < k; slice++)
-    for (int kind = 0; kind < 3; kind++) sim.run(tail[kind], k == 1 ? duration[kind] + start : duration[kind] / k + start + seam);
-  return sim.end();
-}
-
-// With more than four rounds of tiles the last one matters too little to be worth the simulation.
-__host__ __device__ inline bool tail_slices_considered(int64_t tiles, int units) { return tiles > 0 && units > 0 && tiles <= 4 * (int64_t)units; }
-
-// Slices for the tiles of the last round, given the simulated ends for k = 1 .. kMaxTailSlices: the k with the
-// shortest launch, 1 unless k > 1 saves 2 %.
-__host__ __device__ inline int choose_tail_slices(const float (&end)[kMaxTailSlices]) {
-  int best = 1;
-  float best_end = end[0];
-  for (int k = 2; k <= kMaxTailSlices; k++)
-    if (end[k - 1] < best_end && end[k - 1] < 0.98f * end[0]) best = k, best_end = end[k - 1];
-  return best;
-}
+constexpr int kSortCapacity = 4096;  // lines that are put in order of their lengths (longer lists: left as they are)
 
 // Step 1, one wavefront per line (both directions in one launch): same[i] = line i + 1
 // repeats line i.  The flags go to the scratch half of the plan.
@@ -209,8 +132,6 @@ __global__ __launch_bounds__(1024) void plan_roles_kernel(const int32_t* __restr
   __shared__ int sort_line[kSortCapacity];
   __shared__ uint8_t sort_key[kSortCapacity];
   __shared__ uint16_t sort_wave[16 * 256];  // per wavefront and key: a count, then the place of the first such entry
-  __shared__ float sim_time[kTailSliceColumns * kMaxTailSlices][kSimCapacity];
-  __shared__ int sim_count[kTailSliceColumns * kMaxTailSlices][kSimCapacity];
   const bool cols = blockIdx.x == 1;
   const int lines = cols ? block_cols : block_rows;
   uint8_t* tail_slices = plan + plan_slices_offset(block_rows, block_cols) + (cols ? kPlanHintBytes : 0);
@@ -446,35 +367,34 @@ __global__ __launch_bounds__(1024) void plan_roles_kernel(const int32_t* __restr
       }
     }
   }
-  // slices for the last round of stk_dsd: one thread per (width of the dense operand, slice count) simulates
-  // the launch; the first of each four picks
-  static_assert(kTailSliceColumns * kMaxTailSlices == 64 && kMaxTailSlices == 4, "one wavefront");
-  if (tid < 64) {
+  // slices for the last round of stk_dsd: every wavefront simulates the launches for one width of the dense operand
+  static_assert(kTailSliceColumns == 16, "one wavefront each");
+  {
     const int32_t* offs = cols ? offsets_t : offsets;
-    const int ntn = tid / kMaxTailSlices + 1;  // column tiles of 256
+    const int ntn = wave + 1;  // column tiles of 256
     const int tiles[3] = {totals[kTallPairs] * ntn, totals[kTallTriples] * 2 * ntn, totals[kTallSingles] * ntn};
-    DispatchSim sim{sim_time[tid], sim_count[tid], 0, 0};
-    float end = 0.f;
-    if (tail_slices_considered(tiles[0] + tiles[1] + tiles[2], compute_units) && offs)
-      end = simulate_launch(sim, tiles, (float)offs[lines] / (float)lines, compute_units, tid % kMaxTailSlices + 1);
-    float ends[kMaxTailSlices];
-#pragma unroll
-    for (int k = 0; k < kMaxTailSlices; k++) ends[k] = __shfl(end, (tid & ~3) + k, 64);
-    if (tid % kMaxTailSlices == 0) tail_slices[tid / kMaxTailSlices] = (uint8_t)choose_tail_slices(ends);
+    float ends[kMaxTailSlices] = {0.f, 0.f, 0.f, 0.f};
+    if (tail_slices_considered(tiles[0] + tiles[1] + tiles[2], compute_units) && offs) {
+      const float length = (float)offs[lines] / (float)lines;
+      for (int k = 1; k <= kMaxTailSlices; k++) {
+        WaveSim sim;
+        ends[k - 1] = simulate_launch(sim, tiles, length, compute_units, k);
+      }
+    }
+    if (lane == 0) tail_slices[wave] = (uint8_t)choose_tail_slices(ends);
   }
   // Do equal eighths of the lines hold about equal numbers of blocks?  If not (one share 25 % above the mean),
   // the products spread the list over the XCDs in small groups instead of eight contiguous shares.
-  if (tid == 64) {
+  if (wave == 0) {
     const int32_t* offs = cols ? offsets_t : offsets;
-    int spread = 0;
-    if (offs) {
+    bool heavy = false;
+    if (offs && lane < 8) {
       const int64_t total = offs[lines];
-      for (int c = 0; c < 8; c++) {
-        const int64_t share = offs[(int64_t)(c + 1) * lines / 8] - offs[(int64_t)c * lines / 8];
-        if (share * 32 > total * 5) spread = 1;  // > 1.25 / 8 of the blocks
-      }
+      const int64_t share = offs[(int64_t)(lane + 1) * lines / 8] - offs[(int64_t)lane * lines / 8];
+      heavy = share * 32 > total * 5;  // > 1.25 / 8 of the blocks
     }
-    tail_slices[kSpreadHint] = (uint8_t)spread;
+    const uint64_t any = __ballot(heavy);
+    if (lane == 0) tail_slices[kSpreadHint] = any != 0;
   }
 }
 
@@ -489,9 +409,7 @@ extern "C" int stk_dsd_tail_slices(int64_t pair_tiles, int64_t triple_tiles, int
   using namespace stk;
   if (pair_tiles < 0 || triple_tiles < 0 || single_tiles < 0 || pair_tiles + triple_tiles + single_tiles > INT32_MAX) return 1;
   if (!tail_slices_considered(pair_tiles + triple_tiles + single_tiles, compute_units)) return 1;
-  float time[kSimCapacity];
-  int count[kSimCapacity];
-  DispatchSim sim{time, count, 0, 0};
+  HostSim sim;
   const int tiles[3] = {(int)pair_tiles, (int)triple_tiles, (int)single_tiles};
   float ends[kMaxTailSlices];
   for (int k = 1; k <= kMaxTailSlices; k++) ends[k - 1] = simulate_launch(sim, tiles, (float)blocks_per_line, compute_units, k);

@@ -439,65 +439,6 @@ __global__ __launch_bounds__(256) void block_coordinates_kernel(const uint8_t* _
   }
 }
 
-// ------------------------------------------------------------ dMoE topology
-// Block-diagonal pattern of a dropless mixture-of-experts layer: expert e owns the
-// block rows [first_e, first_e + R_e) given by the padded bins and the `width` block
-// columns starting at e * width.  Everything is a closed form of (block row, expert):
-//   block p = i * width + j          row_indices[p] = i, column_indices[p] = e(i) * width + j
-//   offsets[i] = i * width
-//   column c = e * width + j         offsets_t[c] = first_e * width + j * R_e
-//   entry r of that column           column_indices_t = first_e + r, block_offsets_t = (first_e + r) * width + j
-// which is also what a stable sort by column of the (row, column) pairs gives.
-// Expert of a block row: the first bin that ends beyond it (rows past the last bin go to the last expert).
-__device__ __forceinline__ int expert_of_row(const int32_t* __restrict__ bins, int experts, int64_t row_end_exclusive_probe) {
-  int lo = 0, hi = experts - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (bins[mid] > row_end_exclusive_probe) hi = mid;
-    else lo = mid + 1;
-  }
-  return lo;
-}
-
-template <typename IDX>
-__global__ __launch_bounds__(256) void dmoe_topology_kernel(
-    const int32_t* __restrict__ bins, int experts, int blocking, int block_rows, int width,
-    int32_t* __restrict__ offsets, IDX* __restrict__ row_indices, IDX* __restrict__ column_indices,
-    int32_t* __restrict__ offsets_t, IDX* __restrict__ column_indices_t, int32_t* __restrict__ block_offsets_t) {
-  const int64_t nnz = (int64_t)block_rows * width;
-  const int64_t columns = (int64_t)experts * width;
-  const int64_t work = nnz > columns + 1 ? nnz : columns + 1;
-  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < work; p += (int64_t)gridDim.x * blockDim.x) {
-    if (p < nnz) {
-      const int i = (int)(p / width), j = (int)(p % width);
-      const int e = expert_of_row(bins, experts, (int64_t)i * blocking);
-      int first = e == 0 ? 0 : bins[e - 1] / blocking;
-      int last = e == experts - 1 ? block_rows : bins[e] / blocking;  // rows past the last bin stay with the last expert
-      if (first > block_rows) first = block_rows;  // bins that claim more rows than exist: stay inside the arrays
-      if (last > block_rows) last = block_rows;
-      row_indices[p] = (IDX)i;
-      column_indices[p] = (IDX)(e * width + j);
-      if (j == 0) offsets[i] = i * width;
-      const int64_t q = (int64_t)first * width + (int64_t)j * (last - first) + (i - first);
-      column_indices_t[q] = (IDX)i;
-      block_offsets_t[q] = (int32_t)p;
-    }
-    if (p <= columns) {
-      if (p == columns) {
-        offsets_t[p] = (int32_t)nnz;
-        offsets[block_rows] = (int32_t)nnz;
-      } else {
-        const int e = (int)(p / width), j = (int)(p % width);
-        int first = e == 0 ? 0 : bins[e - 1] / blocking;
-        int last = e == experts - 1 ? block_rows : bins[e] / blocking;
-        if (first > block_rows) first = block_rows;
-        if (last > block_rows) last = block_rows;
-        offsets_t[p] = (int32_t)((int64_t)first * width + (int64_t)j * (last - first));
-      }
-    }
-  }
-}
-
 static thread_local char g_error[kErrorBufferBytes] = "";
 char* error_buffer() { return g_error; }
 
@@ -651,33 +592,4 @@ extern "C" int stk_to_sparse_fill(const void* x, int64_t rows, int64_t cols, int
   const int rc = stk_to_sparse_coordinates(rows, cols, blocking, mask, offsets, row_indices, column_indices, index_dtype, stream);
   if (rc != STK_OK) return rc;
   return stk_to_sparse_gather(x, rows, cols, x_stride, blocking, elem_bytes, row_indices, column_indices, nnz, index_dtype, data, stream);
-}
-
-extern "C" int stk_dmoe_topology(const int32_t* padded_bins, int64_t num_experts, int blocking, int64_t block_rows,
-                                 int64_t blocks_per_row, int index_dtype, int32_t* offsets, void* row_indices,
-                                 void* column_indices, int32_t* offsets_t, void* column_indices_t, int32_t* block_offsets_t,
-                                 stk_stream_t stream) {
-  if (index_dtype != STK_I16 && index_dtype != STK_I32) return fail(STK_ERR_UNSUPPORTED, "stk_dmoe_topology: index dtype %d", index_dtype);
-  if (num_experts <= 0 || blocking <= 0 || block_rows < 0 || blocks_per_row <= 0)
-    return fail(STK_ERR_DIMS, "stk_dmoe_topology: %lld experts, blocking %d, %lld block rows of %lld blocks", (long long)num_experts,
-                blocking, (long long)block_rows, (long long)blocks_per_row);
-  const int64_t nnz = block_rows * blocks_per_row, columns = num_experts * blocks_per_row;
-  if (nnz > INT32_MAX || columns >= INT32_MAX || block_rows * blocking > INT32_MAX)
-    return fail(STK_ERR_UNSUPPORTED, "stk_dmoe_topology: size exceeds 32-bit range");
-  if (index_dtype == STK_I16 && (block_rows > 32767 || columns > 32767))
-    return fail(STK_ERR_DIMS, "stk_dmoe_topology: %lld block rows x %lld block columns do not fit 16-bit indices", (long long)block_rows, (long long)columns);
-  if (!padded_bins || !offsets || !offsets_t || (nnz > 0 && (!row_indices || !column_indices || !column_indices_t || !block_offsets_t)))
-    return fail(STK_ERR_DIMS, "stk_dmoe_topology: missing pointer");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t work = nnz > columns + 1 ? nnz : columns + 1;
-  const int grid = (int)((work + 255) / 256 < 65536 ? (work + 255) / 256 : 65536);
-  if (index_dtype == STK_I32)
-    hipLaunchKernelGGL((dmoe_topology_kernel<int32_t>), dim3(grid), dim3(256), 0, s, padded_bins, (int)num_experts, blocking, (int)block_rows,
-                       (int)blocks_per_row, offsets, static_cast<int32_t*>(row_indices), static_cast<int32_t*>(column_indices), offsets_t,
-                       static_cast<int32_t*>(column_indices_t), block_offsets_t);
-  else
-    hipLaunchKernelGGL((dmoe_topology_kernel<int16_t>), dim3(grid), dim3(256), 0, s, padded_bins, (int)num_experts, blocking, (int)block_rows,
-                       (int)blocks_per_row, offsets, static_cast<int16_t*>(row_indices), static_cast<int16_t*>(column_indices), offsets_t,
-                       static_cast<int16_t*>(column_indices_t), block_offsets_t);
-  return check_launch("stk_dmoe_topology");
 }
