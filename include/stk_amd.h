@@ -260,7 +260,7 @@ int stk_dds(int64_t m, int64_t k, int64_t n,
  * Replaces the pair of backend calls in SDD.backward, stk/backend/sputnik.py:274-299 (dsd at :280-288, dds at
  * :289-297), which read dS twice in two launches.  With blocking 128, a plan, rhs as a .t() view of a row-major
  * [n_dsd, k] and lhs as a .t() view of a row-major [m, m_dds] (what the backward pass of a product of two
- * row-major operands passes), n_dsd and m_dds multiples of 256, both products run as one grid: the long tiles of
+ * row-major operands passes), n_dsd and m_dds at least 256 and multiples of 64, both products run as one grid: the long tiles of
  * the dsd first, the short tiles of the dds behind them.  Any other case runs stk_dsd (without a workspace) and
  * then stk_dds.  Either way the results are those of stk_dsd without a workspace and of stk_dds, bit for bit.
  * Arguments as for stk_dsd and stk_dds with transpose flags 0.
@@ -278,7 +278,7 @@ int stk_dsd_dds(int64_t m, int64_t k,
  *   out   [m, n]    = S [m, k] * rhs [k, n]            the gradient with respect to lhs (rhs here = the row-major tensor)
  *   out_t [k, n_t]  = S^T [k, m] * rhs_t [m, n_t]      the gradient with respect to the row-major tensor (rhs_t here = lhs there)
  * two dsd products on the same values, which SDD.backward (stk/backend/sputnik.py:274-299) issues as two backend
- * calls.  With blocking 128, a plan, row-major rhs and rhs_t and n, n_t multiples of 256 they run as one grid (the tiles
+ * calls.  With blocking 128, a plan, row-major rhs and rhs_t and n, n_t of at least 256 and multiples of 64 they run as one grid (the tiles
  * of the first, then of the second); any other case runs stk_dsd twice (without a workspace).  Either way the results
  * are those of the two stk_dsd calls without a workspace, bit for bit.
  */
@@ -297,7 +297,7 @@ int stk_dsd_dsd(int64_t m, int64_t k,
  * op(S) = S^T lhs = rhs, rhs_sdd = dy^T, transpose_a = 0 and rhs_dsd = dy.  Replaces the pair of backend calls in
  * DSD.backward, stk/backend/sputnik.py:131-155 (sdd at :139-145, dsd at :146-154), which are two launches.  With
  * blocking 128, a plan, more nonzero blocks than compute units, a row-major lhs and rhs_sdd as a .t() view of a
- * row-major [n, k_sdd] with k_sdd a multiple of 64, and a row-major rhs_dsd with n_dsd a multiple of 256, both
+ * row-major [n, k_sdd] with k_sdd a multiple of 64, and a row-major rhs_dsd with n_dsd at least 256 and a multiple of 64, both
  * products run as one grid: the tiles of the sdd first, the tiles of the dsd behind them.  Any other case runs stk_sdd
  * and then stk_dsd (without a workspace).  Either way the results are those of stk_sdd and of stk_dsd without a
  * workspace, bit for bit.  Arguments as for stk_sdd (block_order = block_offsets_t) and stk_dsd.
@@ -526,7 +526,7 @@ int stk_sdd_gather(const void* tokens, int64_t num_tokens, int64_t token_stride,
  * The sums are rounded to dtype, then multiplied by the fp32 weight and rounded again (weights NULL: not at all),
  * which is what the two calls do; the results are theirs bit for bit.  Rows of `out` that no r names are not
  * written (stk_route with top_k = 1 names every token).  out is [num_tokens, n] with out_stride_m elements between
- * rows.  The other arguments are those of stk_dsd, workspace included.  128-blocks, n a multiple of 256 and a launch
+ * rows.  The other arguments are those of stk_dsd, workspace included.  128-blocks, n at least 256 and a multiple of 64 and a launch
  * that stk_dsd would run on its eight-wavefront tiles only; STK_ERR_UNSUPPORTED otherwise (callers then make the two
  * calls).  No counterpart in the reference (see stk_route); replaces its dsd, stk/backend/sputnik.py:51-120, for
  * this use.

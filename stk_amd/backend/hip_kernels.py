@@ -796,7 +796,7 @@ def dsd_scatter(shape, data, offsets, column_indices, offsets_t, column_indices_
     assert k == rhs.shape[0], "incompatible dimensions"
     _validate_matmul_dims(m, k, n, b)
     tokens = out.shape[0]
-    if b != 128 or n % 256 or not FUSION or data.shape[0] == 0 or tokens == 0:
+    if b != 128 or n < 256 or n % 64 or not FUSION or data.shape[0] == 0 or tokens == 0:
         return False
     rhs = _dense_operand(rhs)
     data = data.detach()

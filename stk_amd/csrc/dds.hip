@@ -15,7 +15,7 @@ __global__ __launch_bounds__(Cfg::kThreads, 2) void dds_kernel(DdsArgs g) {
   extern __shared__ __align__(16) char smem[];
   const int ntm = (g.m + Cfg::TM - 1) / Cfg::TM;
   const int item = xcd_grouped(blockIdx.x, g.block_cols * ntm);  // no plan, no hint about the lines: small groups
-  dds_tile<Cfg, BLK, TRANS_B, FULL, 1>(g, item / ntm, (item % ntm) * Cfg::TM, smem);
+  dds_tile<Cfg, BLK, TRANS_B, FULL, 1>(g, item / ntm, item % ntm, smem);
 }
 
 // Every block column on its own (four wavefronts), in the order of the plan's lists: the columns of the pairs,
@@ -31,7 +31,7 @@ __global__ __launch_bounds__(Cfg::kThreads, 2) void dds_lines_kernel(DdsArgs g, 
   const int item = xcd_lines(blockIdx.x, tiles, ntm, plan.stripe_from(false));   // (by stripes of lhs rows when the columns share little)
   const int l = item / ntm;
   const int line = l < 2 * pairs ? const_ints(plan.list(kPairs))[l >> 1] + (l & 1) : const_ints(plan.list(kSingles))[l - 2 * pairs];
-  dds_tile<Cfg, BLK, TRANS_B, true, 1>(g, line, (item % ntm) * Cfg::TM, smem);
+  dds_tile<Cfg, BLK, TRANS_B, true, 1>(g, line, item % ntm, smem);
 }
 
 // The lone block columns of a plan's list, one per workgroup (four wavefronts): what dds_fused64_kernel leaves.
@@ -42,7 +42,7 @@ __global__ __launch_bounds__(Cfg::kThreads, 2) void dds_singles_kernel(DdsArgs g
   const int tiles = const_ints(plan.counts)[kTallSingles] * ntm;
   if ((int)blockIdx.x >= tiles) return;
   const int item = xcd_grouped(blockIdx.x, tiles);
-  dds_tile<Cfg, BLK, TRANS_B, FULL, 1>(g, const_ints(plan.list(kTallSingles))[item / ntm], (item % ntm) * Cfg::TM, smem);
+  dds_tile<Cfg, BLK, TRANS_B, FULL, 1>(g, const_ints(plan.list(kTallSingles))[item / ntm], item % ntm, smem);
 }
 
 // 64-blocks with a plan built for them, eight wavefronts: groups of four identical block columns as 256x256
@@ -53,26 +53,26 @@ template <class Quad, class Pair, bool TRANS_B>
 __global__ __launch_bounds__(512, 2) void dds_fused64_kernel(DdsArgs g, PlanLists plan) {
   extern __shared__ __align__(16) char smem[];
   static_assert(Quad::TM == Pair::TM, "same row tiling");
-  const int ntm = g.m / Quad::TM;
+  const int ntm = (g.m + Quad::TM - 1) / Quad::TM;
   const int quad_tiles = const_ints(plan.counts)[kPairs] * ntm, triple_tiles = const_ints(plan.counts)[kTallTriples] * ntm;
   const int pair_tiles = const_ints(plan.counts)[kTallPairs] * ntm;
   int bid = blockIdx.x;
   // pairs first: they hold the lines that were too long for groups of four, the longest tiles of the launch
   if (bid < pair_tiles) {
     const int item = xcd_item(bid, pair_tiles, ntm, plan.group(kTallPairs));
-    dds_tile<Pair, 64, TRANS_B, true, 2>(g, const_ints(plan.list(kTallPairs))[item / ntm], (item % ntm) * Pair::TM, smem, 2);
+    dds_tile<Pair, 64, TRANS_B, true, 2>(g, const_ints(plan.list(kTallPairs))[item / ntm], item % ntm, smem, 2);
     return;
   }
   bid -= pair_tiles;
   if (bid < quad_tiles) {
     const int item = xcd_item(bid, quad_tiles, ntm, plan.group(kPairs));
-    dds_tile<Quad, 64, TRANS_B, true, 4>(g, const_ints(plan.list(kPairs))[item / ntm], (item % ntm) * Quad::TM, smem, 4);
+    dds_tile<Quad, 64, TRANS_B, true, 4>(g, const_ints(plan.list(kPairs))[item / ntm], item % ntm, smem, 4);
     return;
   }
   bid -= quad_tiles;
   if (bid < triple_tiles) {
     const int item = xcd_item(bid, triple_tiles, ntm, plan.group(kTallTriples));
-    dds_tile<Quad, 64, TRANS_B, true, 4>(g, const_ints(plan.list(kTallTriples))[item / ntm], (item % ntm) * Quad::TM, smem, 3);
+    dds_tile<Quad, 64, TRANS_B, true, 4>(g, const_ints(plan.list(kTallTriples))[item / ntm], item % ntm, smem, 3);
   }
 }
 
@@ -97,14 +97,14 @@ __device__ __forceinline__ int round_tile(int round) {
 }
 
 // The tiles [first, first + count) of the launch, all of LINES block columns, that this workgroup takes (round_tile);
-// locate(id) gives a tile's first block column and first output row.  `round` counts on from the call before.
+// locate(id) gives a tile's first block column and which tile of output rows it is.  `round` counts on from the call before.
 template <class Cfg, bool TRANS_B, int LINES, class Locate>
 __device__ __forceinline__ void dds_walk_tiles(const DdsArgs& g, int first, int count, Locate&& locate, char* smem, int& round, bool& used_lds) {
   int id = round_tile(round);
   while (id < first) id = round_tile(++round);
   if (id >= first + count) return;
-  int line, m0;
-  locate(id, line, m0);
+  int line, row_tile;
+  locate(id, line, row_tile);
   DdsWalk<LINES> walk;
   if (!dds_walk_scalar<LINES, TRANS_B>(g, line, LINES, walk)) walk = dds_walk<LINES, TRANS_B>(g, line, LINES);
   for (;;) {
@@ -112,21 +112,21 @@ __device__ __forceinline__ void dds_walk_tiles(const DdsArgs& g, int first, int 
     used_lds = true;
     const int next_id = round_tile(++round);
     const bool more = next_id < first + count;
-    int next_line = line, next_m0 = m0;
+    int next_line = line, next_row_tile = row_tile;
     DdsWalk<LINES> next_walk = walk;
     bool have_next = false;
     auto look_ahead = [&] {
       if (more) {
-        locate(next_id, next_line, next_m0);
+        locate(next_id, next_line, next_row_tile);
         have_next = dds_walk_scalar<LINES, TRANS_B>(g, next_line, LINES, next_walk);
       }
     };
     if (walk.nseg <= 0) look_ahead();  // (a column without blocks has no main loop to hide it behind)
-    dds_tile_of<Cfg, 128, TRANS_B, true, LINES>(g, walk, m0, smem, LINES, look_ahead);
+    dds_tile_of<Cfg, 128, TRANS_B, true, LINES>(g, walk, row_tile, smem, LINES, look_ahead);
     if (!more) return;
     id = next_id;
     line = next_line;
-    m0 = next_m0;
+    row_tile = next_row_tile;
     if (have_next) walk = next_walk;
     else walk = dds_walk<LINES, TRANS_B>(g, line, LINES);
   }
@@ -136,27 +136,27 @@ template <class Fused, class Single, bool TRANS_B>
 __global__ __launch_bounds__(512, 2) void dds_fused_kernel(DdsArgs g, PlanLists plan) {
   extern __shared__ __align__(16) char smem[];
   static_assert(Fused::TM == Single::TM, "same row tiling");
-  const int ntm = g.m / Fused::TM;
+  const int ntm = (g.m + Fused::TM - 1) / Fused::TM;
   bool used_lds = false;
   int round = 0;
   if (!plan.counts) {
     const int total = g.block_cols * ntm;
-    dds_walk_tiles<Single, TRANS_B, 1>(g, 0, total, [&](int id, int& line, int& m0) {
+    dds_walk_tiles<Single, TRANS_B, 1>(g, 0, total, [&](int id, int& line, int& row_tile) {
       const int item = xcd_grouped(id, total);
-      line = item / ntm, m0 = (item % ntm) * Single::TM;
+      line = item / ntm, row_tile = item % ntm;
     }, smem, round, used_lds);
     return;
   }
   const int pair_tiles = const_ints(plan.counts)[kPairs] * ntm, single_tiles = const_ints(plan.counts)[kSingles] * ntm;
-  dds_walk_tiles<Fused, TRANS_B, 2>(g, 0, pair_tiles, [&](int id, int& line, int& m0) {
+  dds_walk_tiles<Fused, TRANS_B, 2>(g, 0, pair_tiles, [&](int id, int& line, int& row_tile) {
     const int item = xcd_item(id, pair_tiles, ntm, plan.group(kPairs));
-    line = const_ints(plan.list(kPairs))[item / ntm], m0 = (item % ntm) * Fused::TM;
+    line = const_ints(plan.list(kPairs))[item / ntm], row_tile = item % ntm;
   }, smem, round, used_lds);
   // (in order of length: no contiguous shares; by stripes of the dense operand when the plan says so, in its 256-wide tiles)
   const int stripe_from = (plan.stripe_from(false) + 1) >> 1;
-  dds_walk_tiles<Single, TRANS_B, 1>(g, pair_tiles, single_tiles, [&](int id, int& line, int& m0) {
+  dds_walk_tiles<Single, TRANS_B, 1>(g, pair_tiles, single_tiles, [&](int id, int& line, int& row_tile) {
     const int item = xcd_lines(id - pair_tiles, id, single_tiles, ntm, stripe_from);
-    line = const_ints(plan.list(kSingles))[item / ntm], m0 = (item % ntm) * Single::TM;
+    line = const_ints(plan.list(kSingles))[item / ntm], row_tile = item % ntm;
   }, smem, round, used_lds);
 }
 
@@ -178,15 +178,15 @@ static void launch_dds(const DdsArgs& g, const PlanLists& plan, hipStream_t stre
     // eight wavefronts: 2x4... see dsd.hip; here 4x2 of 64x128 over two block columns, or 4x2 of 64x64 over one
     using Fused = TileCfg<4, 2, 2, 4, 1, 2, 2, AK, TRANS_B, BF16, KT, S, STREAM>;
     using Single = TileCfg<4, 2, 2, 2, 1, 2, 1, AK, TRANS_B, BF16, KT, S, STREAM>;
-    // four wavefronts, 128x128, for row counts that are not a multiple of 256
+    // four wavefronts, 128x128, for launches with little work and for 128 rows
     using Narrow = TileCfg<2, 2, 2, 2, 1, 1, 1, AK, TRANS_B, BF16, KT, S, STREAM>;
     using Reg = TileCfg<2, 2, 2, 2, 1, 1, 1, AK, TRANS_B, BF16, 64, 2>;
-    if (g.m % Fused::TM == 0 && !g.small) {
+    if (edge_tiles(g.m, Fused::TM) && !g.small) {
       constexpr int lds = Fused::kSmemBytes > Single::kSmemBytes ? Fused::kSmemBytes : Single::kSmemBytes;
       static const int once = (set_lds_limit(&dds_fused_kernel<Fused, Single, TRANS_B>, lds), 0);
       (void)once;
       // one workgroup per compute unit; the tiles are at most one per block column and row tile
-      const int units = compute_units(), tiles = g.block_cols * (g.m / Fused::TM);
+      const int units = compute_units(), tiles = g.block_cols * ((g.m + Fused::TM - 1) / Fused::TM);
       hipLaunchKernelGGL((dds_fused_kernel<Fused, Single, TRANS_B>), dim3(units > 0 && units < tiles ? units : tiles), dim3(512), lds, stream, g, plan);
     } else if (g.m % Narrow::TM == 0 && plan.counts) {
       static const int once = (set_lds_limit(&dds_lines_kernel<Narrow, BLK, TRANS_B>, Narrow::kSmemBytes), 0);
@@ -201,7 +201,7 @@ static void launch_dds(const DdsArgs& g, const PlanLists& plan, hipStream_t stre
   } else {
     // 64-blocks: 4x1 wavefronts of 64x64 (tile 256x64)
     using Dma = TileCfg<4, 1, 2, 2, 1, 1, 1, AK, TRANS_B, BF16, 64, 2, STREAM>;
-    if (plan.counts && g.m % 256 == 0 && !g.small) {
+    if (plan.counts && edge_tiles(g.m, 256) && !g.small) {
       // groups of identical block columns on eight wavefronts (4x2 of 64x128 over four block columns, 4x2 of 64x64
       // over two), then the lone columns one per four-wave workgroup; both grids are upper bounds
       using Quad = TileCfg<4, 2, 2, 4, 1, 2, 4, AK, TRANS_B, BF16, 64, 2, STREAM>;
@@ -209,12 +209,15 @@ static void launch_dds(const DdsArgs& g, const PlanLists& plan, hipStream_t stre
       constexpr int lds = Quad::kSmemBytes > Pair::kSmemBytes ? Quad::kSmemBytes : Pair::kSmemBytes;
       static const int once = (set_lds_limit(&dds_fused64_kernel<Quad, Pair, TRANS_B>, lds), set_lds_limit(&dds_singles_kernel<Dma, 64, TRANS_B, true>, Dma::kSmemBytes), 0);
       (void)once;
-      const int ntm = g.m / 256;
+      const int ntm = (g.m + 255) / 256;
       hipLaunchKernelGGL((dds_fused64_kernel<Quad, Pair, TRANS_B>), dim3((g.block_cols + 1) / 2 * ntm), dim3(512), lds, stream, g, plan);
       hipLaunchKernelGGL((dds_singles_kernel<Dma, 64, TRANS_B, true>), dim3(g.block_cols * ntm), dim3(Dma::kThreads), Dma::kSmemBytes, stream, g, plan);
       return;
     }
-    if (g.m % Dma::TM == 0) launch_one<Dma, BLK, TRANS_B, true>(g, stream);
+    // fewer than 256 rows: 64x64 tiles, the four wavefronts split each K-tile
+    using Few = TileCfg<1, 1, 2, 2, 4, 1, 1, AK, TRANS_B, BF16, 64, 4, STREAM>;
+    if (edge_tiles(g.m, Dma::TM)) launch_one<Dma, BLK, TRANS_B, true>(g, stream);
+    else if (edge_tiles(g.m, Few::TM)) launch_one<Few, BLK, TRANS_B, true>(g, stream);
     else launch_one<Dma, BLK, TRANS_B, false>(g, stream);
   }
 }

@@ -99,14 +99,16 @@ __device__ __forceinline__ bool dds_walk_scalar(const DdsArgs& g, int bj, int li
   return true;
 }
 
-// The tile of the LINES block columns of walk `w`, output rows [m0, m0 + Cfg::TM).  after_prologue: see mainloop_dma
+// The tile of the LINES block columns of walk `w`, the row_tile-th tile of Cfg::TM output rows (FULL: whole tiles, or the
+// last one is moved back, edge_start()).  after_prologue: see mainloop_dma
 // (called once, inside the first main loop; not at all for a walk without entries).
 template <class Cfg, int BLK, bool TRANS_B, bool FULL, int LINES, class Hook>
-__device__ __forceinline__ void dds_tile_of(const DdsArgs& g, DdsWalk<LINES> w, int m0, char* smem, int lines, Hook&& after_prologue) {
+__device__ __forceinline__ void dds_tile_of(const DdsArgs& g, DdsWalk<LINES> w, int row_tile, char* smem, int lines, Hook&& after_prologue) {
   static_assert(Cfg::TN == LINES * BLK && Cfg::B_PARTS == LINES && Cfg::B_KMAJOR == TRANS_B, "one operand part per block column");
   constexpr int KT = Cfg::KT;
   constexpr int kTilesPerBlock = BLK / KT;
   const int nseg = w.nseg, bj = w.bj;
+  const int m0 = FULL ? edge_start(row_tile, Cfg::TM, g.m) : row_tile * Cfg::TM;
   const elem_t* a0 = g.lhs + (int64_t)m0 * (Cfg::A_KMAJOR ? g.lda : 1);
   const int64_t a_kstride = Cfg::A_KMAJOR ? 1 : g.lda;
   const int64_t a_part = (int64_t)Cfg::PM * (Cfg::A_KMAJOR ? g.lda : 1);
@@ -141,15 +143,16 @@ __device__ __forceinline__ void dds_tile_of(const DdsArgs& g, DdsWalk<LINES> w, 
   }
   const WaveCoords wc = wave_coords<Cfg>();
   const int wm0 = wave_m0<Cfg>(wc), wn0 = wave_n0<Cfg>(wc);
-  epilogue<Cfg, STK_STREAM_STORES>(acc, g.out + (int64_t)(m0 + wm0) * g.ldc + (int64_t)bj * BLK + wn0, g.ldc, m_valid - wm0, lines * BLK - wn0, smem);
+  epilogue<Cfg, STK_STREAM_STORES>(acc, g.out + (int64_t)(m0 + wm0) * g.ldc + (int64_t)bj * BLK + wn0, g.ldc, m_valid - wm0, lines * BLK - wn0, smem, 64,
+                                   kNoActivation, nullptr, 0, 0, nullptr, nullptr, 0, nullptr, row_tile * Cfg::TM - m0 - wm0, 0);
 }
 
-// LINES block columns starting at `bj` (identical patterns when LINES > 1), output
-// rows [m0, m0 + Cfg::TM).  Only the first `lines` of the LINES columns exist; the others are
+// LINES block columns starting at `bj` (identical patterns when LINES > 1), the row_tile-th tile of Cfg::TM
+// output rows.  Only the first `lines` of the LINES columns exist; the others are
 // computed on the last one's blocks and dropped.
 template <class Cfg, int BLK, bool TRANS_B, bool FULL, int LINES>
-__device__ __forceinline__ void dds_tile(const DdsArgs& g, int bj, int m0, char* smem, int lines = LINES) {
-  dds_tile_of<Cfg, BLK, TRANS_B, FULL, LINES>(g, dds_walk<LINES, TRANS_B>(g, bj, lines), m0, smem, lines, [] {});
+__device__ __forceinline__ void dds_tile(const DdsArgs& g, int bj, int row_tile, char* smem, int lines = LINES) {
+  dds_tile_of<Cfg, BLK, TRANS_B, FULL, LINES>(g, dds_walk<LINES, TRANS_B>(g, bj, lines), row_tile, smem, lines, [] {});
 }
 
 }  // namespace stk

@@ -15,7 +15,7 @@ __global__ __launch_bounds__(Cfg::kThreads, 2) void dsd_kernel(DsdArgs g) {
   extern __shared__ __align__(16) char smem[];
   const int ntn = (g.n + Cfg::TN - 1) / Cfg::TN;
   const int item = xcd_grouped(blockIdx.x, g.block_rows * ntn);  // no plan, no hint about the lines: small groups
-  dsd_tile<Cfg, BLK, TRANS_A, FULL, 1>(g, item / ntn, (item % ntn) * Cfg::TN, smem);
+  dsd_tile<Cfg, BLK, TRANS_A, FULL, 1>(g, item / ntn, item % ntn, smem);
 }
 
 // Every block row on its own (four wavefronts), in the order of the plan's lists: the rows of the pairs, of the
@@ -35,7 +35,7 @@ __global__ __launch_bounds__(Cfg::kThreads, 2) void dsd_lines_kernel(DsdArgs g, 
   if (l < 2 * pairs) line = const_ints(plan.list(kTallPairs))[l >> 1] + (l & 1);
   else if ((l -= 2 * pairs) < 3 * triples) line = const_ints(plan.list(kTallTriples))[l / 3] + l % 3;
   else line = const_ints(plan.list(kTallSingles))[l - 3 * triples];
-  dsd_tile<Cfg, BLK, TRANS_A, true, 1>(g, line, (item % ntn) * Cfg::TN, smem);
+  dsd_tile<Cfg, BLK, TRANS_A, true, 1>(g, line, item % ntn, smem);
 }
 
 // The lone block rows of a plan's list, one per workgroup (four wavefronts): what dsd_fused64_kernel leaves.
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(Cfg::kThreads, 2) void dsd_singles_kernel(DsdArgs g
   const int tiles = const_ints(plan.counts)[kTallSingles] * ntn;
   if ((int)blockIdx.x >= tiles) return;
   const int item = xcd_grouped(blockIdx.x, tiles);
-  dsd_tile<Cfg, BLK, TRANS_A, FULL, 1>(g, const_ints(plan.list(kTallSingles))[item / ntn], (item % ntn) * Cfg::TN, smem);
+  dsd_tile<Cfg, BLK, TRANS_A, FULL, 1>(g, const_ints(plan.list(kTallSingles))[item / ntn], item % ntn, smem);
 }
 
 // 64-blocks with a plan built for them, eight wavefronts: groups of four identical block rows as 256x256
@@ -57,26 +57,26 @@ template <class Quad, class Pair, class Three, bool TRANS_A>
 __global__ __launch_bounds__(512, 2) void dsd_fused64_kernel(DsdArgs g, PlanLists plan) {
   extern __shared__ __align__(16) char smem[];
   static_assert(Quad::TN == Pair::TN && Quad::TN == Three::TN, "same column tiling");
-  const int ntn = g.n / Quad::TN;
+  const int ntn = (g.n + Quad::TN - 1) / Quad::TN;
   const int quad_tiles = const_ints(plan.counts)[kPairs] * ntn, triple_tiles = const_ints(plan.counts)[kTallTriples] * ntn;
   const int pair_tiles = const_ints(plan.counts)[kTallPairs] * ntn;
   int bid = blockIdx.x;
   // pairs first: they hold the lines that were too long for groups of four, the longest tiles of the launch
   if (bid < pair_tiles) {
     const int item = xcd_item(bid, pair_tiles, ntn, plan.group(kTallPairs));
-    dsd_tile<Pair, 64, TRANS_A, true, 2>(g, const_ints(plan.list(kTallPairs))[item / ntn], (item % ntn) * Pair::TN, smem, 2);
+    dsd_tile<Pair, 64, TRANS_A, true, 2>(g, const_ints(plan.list(kTallPairs))[item / ntn], item % ntn, smem, 2);
     return;
   }
   bid -= pair_tiles;
   if (bid < quad_tiles) {
     const int item = xcd_item(bid, quad_tiles, ntn, plan.group(kPairs));
-    dsd_tile<Quad, 64, TRANS_A, true, 4>(g, const_ints(plan.list(kPairs))[item / ntn], (item % ntn) * Quad::TN, smem, 4);
+    dsd_tile<Quad, 64, TRANS_A, true, 4>(g, const_ints(plan.list(kPairs))[item / ntn], item % ntn, smem, 4);
     return;
   }
   bid -= quad_tiles;
   if (bid < triple_tiles) {
     const int item = xcd_item(bid, triple_tiles, ntn, plan.group(kTallTriples));
-    dsd_tile<Three, 64, TRANS_A, true, 3>(g, const_ints(plan.list(kTallTriples))[item / ntn], (item % ntn) * Three::TN, smem);
+    dsd_tile<Three, 64, TRANS_A, true, 3>(g, const_ints(plan.list(kTallTriples))[item / ntn], item % ntn, smem);
   }
 }
 
@@ -89,9 +89,9 @@ __global__ __launch_bounds__(512, 2) void dsd_fused_kernel(DsdArgs g, PlanLists 
   extern __shared__ __align__(16) char smem[];
   int bid = blockIdx.x;
   if (!plan.counts) {
-    const int ntn = g.n / Fused::TN;
+    const int ntn = (g.n + Fused::TN - 1) / Fused::TN;
     const int item = xcd_grouped(bid, g.block_rows * ntn);
-    dsd_tile<Single, 128, TRANS_A, true, 1, SCATTER>(g, item / ntn, (item % ntn) * Single::TN, smem);
+    dsd_tile<Single, 128, TRANS_A, true, 1, SCATTER>(g, item / ntn, item % ntn, smem);
     return;
   }
   dsd_plan_tile<Fused, Triple, Single, TRANS_A, SCATTER>(g, plan, bid, smem);
@@ -144,12 +144,13 @@ __device__ __forceinline__ void add_slices_in_order(f32x16_t (&acc)[Cfg::IM][Cfg
   }
 }
 
-// Slice `slice` of `slices` of the tile (LINES block rows from bi, columns from n0), the `ordinal`-th tile of the last
+// Slice `slice` of `slices` of the tile (LINES block rows from bi, the column_tile-th tile of columns), the `ordinal`-th tile of the last
 // round; the tile owns the slots [ordinal * slices, (ordinal + 1) * slices) of the workspace.
 template <class Cfg, bool TRANS_A, int LINES, bool SCATTER = false>
-__device__ __forceinline__ void dsd_slice(const DsdArgs& g, const TailArgs& t, int bi, int n0, int slice, int slices, int ordinal, char* smem, int* flag) {
+__device__ __forceinline__ void dsd_slice(const DsdArgs& g, const TailArgs& t, int bi, int column_tile, int slice, int slices, int ordinal, char* smem, int* flag) {
   constexpr int kAcc = Cfg::IM * Cfg::JN;
   static_assert(kAcc * 16 * 512 <= kSlotFloats, "slot too small");
+  const int n0 = edge_start(column_tile, Cfg::TN, g.n), from = column_tile * Cfg::TN - n0;
   const int nseg = g.walk_offsets[bi + 1] - g.walk_offsets[bi];
   const int64_t first_slot = (int64_t)ordinal * slices;
   if (slices > nseg) slices = nseg > 1 ? nseg : 1;
@@ -159,7 +160,7 @@ __device__ __forceinline__ void dsd_slice(const DsdArgs& g, const TailArgs& t, i
   f32x16_t acc[Cfg::IM][Cfg::JN] = {};
   dsd_accumulate<Cfg, 128, TRANS_A, true, LINES>(acc, g, bi, n0, e0, e1, smem);
   if (slices == 1) {
-    dsd_store<Cfg, 128, SCATTER>(acc, g, bi, n0, smem);
+    dsd_store<Cfg, 128, SCATTER>(acc, g, bi, n0, smem, Cfg::TM, from);
     return;
   }
   // Partial tiles and the counter are read and written with device-scope atomic accesses only: these
@@ -219,7 +220,7 @@ __device__ __forceinline__ void dsd_slice(const DsdArgs& g, const TailArgs& t, i
       default: add_slices_in_order<Cfg, 4, 3>(acc, first); break;
     }
   }
-  dsd_store<Cfg, 128, SCATTER>(acc, g, bi, n0, smem);
+  dsd_store<Cfg, 128, SCATTER>(acc, g, bi, n0, smem, Cfg::TM, from);
   if (tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -228,9 +229,9 @@ __global__ __launch_bounds__(512, 2) void dsd_sliced_kernel(DsdArgs g, PlanLists
   extern __shared__ __align__(16) char smem[];
   __shared__ int flag;
   static_assert(Fused::TN == Single::TN && Fused::TN == 2 * Triple::TN, "same column tiling");
-  const int ntn = g.n / Fused::TN;
+  const int ntn = (g.n + Fused::TN - 1) / Fused::TN, narrow = (g.n + Triple::TN - 1) / Triple::TN;
   const int pair_tiles = const_ints(plan.counts)[kTallPairs] * ntn;
-  const int triple_tiles = const_ints(plan.counts)[kTallTriples] * 2 * ntn;
+  const int triple_tiles = const_ints(plan.counts)[kTallTriples] * narrow;
   const int single_tiles = const_ints(plan.counts)[kTallSingles] * ntn;
   const int tiles = pair_tiles + triple_tiles + single_tiles;
   int slices = uniform(plan.hints[(ntn < kTailSliceColumns ? ntn : kTailSliceColumns) - 1]);
@@ -257,13 +258,13 @@ __global__ __launch_bounds__(512, 2) void dsd_sliced_kernel(DsdArgs g, PlanLists
   const int ordinal = item - whole;  // among the tiles of the last round: 0 .. workgroups - 1
   if (item < pair_tiles) {
     const int i = xcd_share(item, pair_tiles, spread);
-    dsd_slice<Fused, TRANS_A, 2, SCATTER>(g, t, const_ints(plan.list(kTallPairs))[i / ntn], (i % ntn) * Fused::TN, slice, slices, ordinal, smem, &flag);
+    dsd_slice<Fused, TRANS_A, 2, SCATTER>(g, t, const_ints(plan.list(kTallPairs))[i / ntn], i % ntn, slice, slices, ordinal, smem, &flag);
     return;
   }
   item -= pair_tiles;
   if (item < triple_tiles) {
     const int i = xcd_share(item, triple_tiles, spread);
-    dsd_slice<Triple, TRANS_A, 3, SCATTER>(g, t, const_ints(plan.list(kTallTriples))[i / (2 * ntn)], (i % (2 * ntn)) * Triple::TN, slice, slices, ordinal, smem, &flag);
+    dsd_slice<Triple, TRANS_A, 3, SCATTER>(g, t, const_ints(plan.list(kTallTriples))[i / narrow], i % narrow, slice, slices, ordinal, smem, &flag);
     return;
   }
   item -= triple_tiles;
@@ -279,7 +280,7 @@ __global__ __launch_bounds__(512, 2) void dsd_sliced_kernel(DsdArgs g, PlanLists
   } else {
     i = xcd_grouped(item, single_tiles);
   }
-  dsd_slice<Single, TRANS_A, 1, SCATTER>(g, t, const_ints(plan.list(kTallSingles))[i / ntn], (i % ntn) * Single::TN, slice, slices, ordinal, smem, &flag);
+  dsd_slice<Single, TRANS_A, 1, SCATTER>(g, t, const_ints(plan.list(kTallSingles))[i / ntn], i % ntn, slice, slices, ordinal, smem, &flag);
 }
 
 template <class Cfg, int BLK, bool TRANS_A, bool FULL>
@@ -306,7 +307,7 @@ static void launch_dsd(const DsdArgs& g, const PlanLists& plan, const TailArgs* 
     // eight wavefronts: 4x2 of 64x128 over two block rows, or 2x4 of 64x64 over one
     using Fused = TileCfg<4, 2, 2, 4, 1, 2, 2, !TRANS_A, BK, BF16, KT, S, false, STREAM>;
     using Single = TileCfg<2, 4, 2, 2, 1, 1, 2, !TRANS_A, BK, BF16, KT, S, false, STREAM>;
-    // four wavefronts, 128x128, for column counts that are not a multiple of 256
+    // four wavefronts, 128x128, for launches with little work and for 128 columns
     // (a K-major operand - sparse blocks that are not transposed, or a .t() view as rhs - in 64-deep K-tiles, whose rows are
     // whole 128-byte lines: on these small tiles that outweighs the deeper ring, config 2 dsd 42.5 -> 38.5 us)
     constexpr int NKT = (!TRANS_A || BK) ? 64 : KT, NS = (!TRANS_A || BK) ? 2 : S;
@@ -314,20 +315,21 @@ static void launch_dsd(const DsdArgs& g, const PlanLists& plan, const TailArgs* 
     using Reg = TileCfg<2, 2, 2, 2, 1, 1, 1, !TRANS_A, BK, BF16, 64, 2>;
     // 4x2 wavefronts of 96x64 over three block rows and 128 columns
     using Triple = TileCfg<4, 2, 3, 2, 1, 3, 1, !TRANS_A, BK, BF16, KT, S, false, STREAM>;
-    if (g.n % Fused::TN == 0 && !g.small) {
+    if (edge_tiles(g.n, Fused::TN) && !g.small) {
+      const int ntn = (g.n + Fused::TN - 1) / Fused::TN;
       constexpr int lds0 = Fused::kSmemBytes > Single::kSmemBytes ? Fused::kSmemBytes : Single::kSmemBytes;
       constexpr int lds = lds0 > Triple::kSmemBytes ? lds0 : Triple::kSmemBytes;
       if (tail) {
         static const int once = (set_lds_limit(&dsd_sliced_kernel<Fused, Triple, Single, TRANS_A>, lds), 0);
         (void)once;
         // upper bound: every line a tile of its own, plus the slices of a full last round (rounded up to whole blocks)
-        const int grid = g.block_rows * (g.n / Fused::TN) + kMaxTailSlices * (tail->workgroups + kTailBlock);
+        const int grid = g.block_rows * ntn + kMaxTailSlices * (tail->workgroups + kTailBlock);
         hipLaunchKernelGGL((dsd_sliced_kernel<Fused, Triple, Single, TRANS_A>), dim3(grid), dim3(512), lds, stream, g, plan, *tail);
         return;
       }
       static const int once = (set_lds_limit(&dsd_fused_kernel<Fused, Triple, Single, TRANS_A>, lds), 0);
       (void)once;
-      hipLaunchKernelGGL((dsd_fused_kernel<Fused, Triple, Single, TRANS_A>), dim3(g.block_rows * (g.n / Fused::TN)), dim3(512), lds, stream, g, plan);
+      hipLaunchKernelGGL((dsd_fused_kernel<Fused, Triple, Single, TRANS_A>), dim3(g.block_rows * ntn), dim3(512), lds, stream, g, plan);
     } else if (g.n % Narrow::TN == 0 && plan.counts) {
       static const int once = (set_lds_limit(&dsd_lines_kernel<Narrow, BLK, TRANS_A>, Narrow::kSmemBytes), 0);
       (void)once;
@@ -341,7 +343,7 @@ static void launch_dsd(const DsdArgs& g, const PlanLists& plan, const TailArgs* 
   } else {
     // 64-blocks: 1x4 wavefronts of 64x64 (tile 64x256)
     using Dma = TileCfg<1, 4, 2, 2, 1, 1, 1, !TRANS_A, BK, BF16, 64, 2, false, STREAM>;
-    if (plan.counts && g.n % 256 == 0 && !g.small) {
+    if (plan.counts && edge_tiles(g.n, 256) && !g.small) {
       // groups of identical block rows on eight wavefronts (4x2 of 64x128 over four block rows, 2x4 of 64x64 over
       // two), then the lone rows one per four-wave workgroup; both grids are upper bounds
       using Quad = TileCfg<4, 2, 2, 4, 1, 4, 2, !TRANS_A, BK, BF16, 64, 2, false, STREAM>;
@@ -352,12 +354,15 @@ static void launch_dsd(const DsdArgs& g, const PlanLists& plan, const TailArgs* 
       static_assert(Three::kSmemBytes <= lds, "the tile of three block rows fits where the tile of four does");
       static const int once = (set_lds_limit(&dsd_fused64_kernel<Quad, Pair, Three, TRANS_A>, lds), set_lds_limit(&dsd_singles_kernel<Dma, 64, TRANS_A, true>, Dma::kSmemBytes), 0);
       (void)once;
-      const int ntn = g.n / 256;
+      const int ntn = (g.n + 255) / 256;
       hipLaunchKernelGGL((dsd_fused64_kernel<Quad, Pair, Three, TRANS_A>), dim3((g.block_rows + 1) / 2 * ntn), dim3(512), lds, stream, g, plan);
       hipLaunchKernelGGL((dsd_singles_kernel<Dma, 64, TRANS_A, true>), dim3(g.block_rows * ntn), dim3(Dma::kThreads), Dma::kSmemBytes, stream, g, plan);
       return;
     }
-    if (g.n % Dma::TN == 0) launch_one<Dma, BLK, TRANS_A, true>(g, stream);
+    // fewer than 256 columns: 64x64 tiles, the four wavefronts split each K-tile
+    using Few = TileCfg<1, 1, 2, 2, 4, 1, 1, !TRANS_A, BK, BF16, 64, 4, false, STREAM>;
+    if (edge_tiles(g.n, Dma::TN)) launch_one<Dma, BLK, TRANS_A, true>(g, stream);
+    else if (edge_tiles(g.n, Few::TN)) launch_one<Few, BLK, TRANS_A, true>(g, stream);
     else launch_one<Dma, BLK, TRANS_A, false>(g, stream);
   }
 }
@@ -375,13 +380,13 @@ static void launch_dsd_scatter(const DsdArgs& g, const PlanLists& plan, const Ta
   if (tail) {
     static const int once = (set_lds_limit(&dsd_sliced_kernel<Fused, Triple, Single, false, true>, lds), 0);
     (void)once;
-    const int grid = g.block_rows * (g.n / Fused::TN) + kMaxTailSlices * (tail->workgroups + kTailBlock);
+    const int grid = g.block_rows * ((g.n + Fused::TN - 1) / Fused::TN) + kMaxTailSlices * (tail->workgroups + kTailBlock);
     hipLaunchKernelGGL((dsd_sliced_kernel<Fused, Triple, Single, false, true>), dim3(grid), dim3(512), lds, stream, g, plan, *tail);
     return;
   }
   static const int once = (set_lds_limit(&dsd_fused_kernel<Fused, Triple, Single, false, true>, lds), 0);
   (void)once;
-  hipLaunchKernelGGL((dsd_fused_kernel<Fused, Triple, Single, false, true>), dim3(g.block_rows * (g.n / Fused::TN)), dim3(512), lds, stream, g, plan);
+  hipLaunchKernelGGL((dsd_fused_kernel<Fused, Triple, Single, false, true>), dim3(g.block_rows * ((g.n + Fused::TN - 1) / Fused::TN)), dim3(512), lds, stream, g, plan);
 }
 
 // The sliced last round of a dsd launch, if this one gets one: for launches of a few rounds of tiles (with many
@@ -390,7 +395,7 @@ static void launch_dsd_scatter(const DsdArgs& g, const PlanLists& plan, const Ta
 static int tail_of(const char* who, const DsdArgs& g, int64_t n, int64_t nnz, int blocking, const uint8_t* plan, void* workspace,
                    int64_t workspace_bytes, TailArgs* tail, bool* sliced) {
   *sliced = false;
-  if (!(workspace && plan && blocking == 128 && n % 256 == 0 && nnz > 0 && !g.small)) return STK_OK;
+  if (!(workspace && plan && blocking == 128 && edge_tiles(n, 256) && nnz > 0 && !g.small)) return STK_OK;
   const int workgroups = compute_units();
   if (workgroups <= 0 || (int64_t)g.block_rows * (n / 128) / 3 >= 8 * (int64_t)workgroups) return STK_OK;
   if (reinterpret_cast<uintptr_t>(workspace) & 255u) return fail(STK_ERR_WORKSPACE, "%s: the workspace must be 256-byte aligned", who);
@@ -523,8 +528,8 @@ extern "C" int stk_dsd_scatter(int64_t m, int64_t k, int64_t n, const void* data
                              out_stride_m, nnz, blocking, dtype, index_dtype, plan, &problem);
   if (rc != STK_OK || problem.empty || num_tokens == 0) return rc;
   if (!row_slots) return fail(STK_ERR_DIMS, "%s: missing row_slots", who);
-  if (n % 256 || problem.g.small)
-    return fail(STK_ERR_UNSUPPORTED, "%s: needs a multiple of 256 columns and at least %lld blocks x 128 columns per compute unit", who,
+  if (!edge_tiles(n, 256) || problem.g.small)
+    return fail(STK_ERR_UNSUPPORTED, "%s: needs 256 columns or more, a multiple of 64, and at least %lld blocks x 128 columns per compute unit", who,
                 (long long)kSmallWorkPerUnit);
   DsdArgs g = problem.g;
   g.row_map = row_slots;
@@ -559,7 +564,7 @@ extern "C" int64_t stk_dsd_workspace_slot_bytes(void) { return (int64_t)(sizeof(
 
 extern "C" int64_t stk_dsd_workspace_bytes(int64_t m, int64_t n, int blocking) {
   using namespace stk;
-  if (blocking != 128 || m <= 0 || n <= 0 || m % 128 || n % 256) return 0;
+  if (blocking != 128 || m <= 0 || n <= 0 || m % 128 || !edge_tiles(n, 256)) return 0;
   const int workgroups = compute_units();
   if (workgroups <= 0 || (m / 128) * (n / 128) / 3 >= 8 * (int64_t)workgroups) return 0;
   return (int64_t)tail_workspace_bytes(workgroups);

@@ -82,26 +82,29 @@ __device__ __forceinline__ void dsd_accumulate(f32x16_t (&acc)[Cfg::IM][Cfg::JN]
   }
 }
 
-// Writes the finished tile: the first `rows` rows from block row `bi` onwards, columns from n0.
+// Writes the finished tile: the first `rows` rows from block row `bi` onwards, columns from n0 + from.
 template <class Cfg, int BLK, bool SCATTER = false>
-__device__ __forceinline__ void dsd_store(f32x16_t (&acc)[Cfg::IM][Cfg::JN], const DsdArgs& g, int bi, int n0, char* smem, int rows = Cfg::TM) {
+__device__ __forceinline__ void dsd_store(f32x16_t (&acc)[Cfg::IM][Cfg::JN], const DsdArgs& g, int bi, int n0, char* smem, int rows = Cfg::TM,
+                                          int from = 0) {
   const int n_valid = (g.n - n0 < Cfg::TN) ? g.n - n0 : Cfg::TN;
   const WaveCoords w = wave_coords<Cfg>();
   const int wm0 = wave_m0<Cfg>(w), wn0 = wave_n0<Cfg>(w);
   if constexpr (SCATTER)
     epilogue<Cfg, STK_STREAM_STORES, true>(acc, g.out + n0 + wn0, g.ldc, rows - wm0, n_valid - wn0, smem, 64, kNoActivation, nullptr, 0, 0,
-                                           g.row_map + (int64_t)bi * BLK + wm0, g.row_scale, g.out_rows);
+                                           g.row_map + (int64_t)bi * BLK + wm0, g.row_scale, g.out_rows, nullptr, 0, from - wn0);
   else
-    epilogue<Cfg, STK_STREAM_STORES>(acc, g.out + ((int64_t)bi * BLK + wm0) * g.ldc + n0 + wn0, g.ldc, rows - wm0, n_valid - wn0, smem);
+    epilogue<Cfg, STK_STREAM_STORES>(acc, g.out + ((int64_t)bi * BLK + wm0) * g.ldc + n0 + wn0, g.ldc, rows - wm0, n_valid - wn0, smem, 64, kNoActivation,
+                                     nullptr, 0, 0, nullptr, nullptr, 0, nullptr, 0, from - wn0);
 }
 
-// The whole tile of LINES block rows starting at `bi` (the first `lines` of them exist), output columns
-// [n0, n0 + Cfg::TN).
+// The whole tile of LINES block rows starting at `bi` (the first `lines` of them exist), the column_tile-th tile of
+// Cfg::TN output columns.  FULL: the columns are whole tiles, or the last one is moved back (edge_start()).
 template <class Cfg, int BLK, bool TRANS_A, bool FULL, int LINES, bool SCATTER = false>
-__device__ __forceinline__ void dsd_tile(const DsdArgs& g, int bi, int n0, char* smem, int lines = LINES) {
+__device__ __forceinline__ void dsd_tile(const DsdArgs& g, int bi, int column_tile, char* smem, int lines = LINES) {
+  const int n0 = FULL ? edge_start(column_tile, Cfg::TN, g.n) : column_tile * Cfg::TN;
   f32x16_t acc[Cfg::IM][Cfg::JN] = {};
   dsd_accumulate<Cfg, BLK, TRANS_A, FULL, LINES>(acc, g, bi, n0, 0, g.walk_offsets[bi + 1] - g.walk_offsets[bi], smem, lines);
-  dsd_store<Cfg, BLK, SCATTER>(acc, g, bi, n0, smem, lines * BLK);
+  dsd_store<Cfg, BLK, SCATTER>(acc, g, bi, n0, smem, lines * BLK, column_tile * Cfg::TN - n0);
 }
 
 // The tile of a launch over the plan's lists of lines (128-blocks, eight wavefronts) that workgroup `bid` takes,
@@ -114,26 +117,26 @@ __device__ __forceinline__ void dsd_tile(const DsdArgs& g, int bi, int n0, char*
 template <class Fused, class Triple, class Single, bool TRANS_A, bool SCATTER = false>
 __device__ __forceinline__ bool dsd_plan_tile(const DsdArgs& g, const PlanLists& plan, int& bid, char* smem) {
   static_assert(Fused::TN == Single::TN && Fused::TN == 2 * Triple::TN, "same column tiling");
-  const int ntn = g.n / Fused::TN;
+  const int ntn = (g.n + Fused::TN - 1) / Fused::TN, narrow = (g.n + Triple::TN - 1) / Triple::TN;
   const int pair_tiles = const_ints(plan.counts)[kTallPairs] * ntn;
-  const int triple_tiles = const_ints(plan.counts)[kTallTriples] * 2 * ntn;
+  const int triple_tiles = const_ints(plan.counts)[kTallTriples] * narrow;
   const int single_tiles = const_ints(plan.counts)[kTallSingles] * ntn;
   if (bid < pair_tiles) {
     const int item = xcd_item(bid, pair_tiles, ntn, plan.group(kTallPairs));
-    dsd_tile<Fused, 128, TRANS_A, true, 2, SCATTER>(g, const_ints(plan.list(kTallPairs))[item / ntn], (item % ntn) * Fused::TN, smem);
+    dsd_tile<Fused, 128, TRANS_A, true, 2, SCATTER>(g, const_ints(plan.list(kTallPairs))[item / ntn], item % ntn, smem);
     return true;
   }
   bid -= pair_tiles;
   if (bid < triple_tiles) {
-    const int item = xcd_item(bid, triple_tiles, 2 * ntn, plan.group(kTallTriples));
-    dsd_tile<Triple, 128, TRANS_A, true, 3, SCATTER>(g, const_ints(plan.list(kTallTriples))[item / (2 * ntn)], (item % (2 * ntn)) * Triple::TN, smem);
+    const int item = xcd_item(bid, triple_tiles, narrow, plan.group(kTallTriples));
+    dsd_tile<Triple, 128, TRANS_A, true, 3, SCATTER>(g, const_ints(plan.list(kTallTriples))[item / narrow], item % narrow, smem);
     return true;
   }
   bid -= triple_tiles;
   if (bid < single_tiles) {
     // (in order of length: no contiguous shares; by stripes of the dense operand when the plan says so, in its 256-wide tiles)
     const int item = xcd_lines(bid, single_tiles, ntn, (plan.stripe_from(true) + 1) >> 1);
-    dsd_tile<Single, 128, TRANS_A, true, 1, SCATTER>(g, const_ints(plan.list(kTallSingles))[item / ntn], (item % ntn) * Single::TN, smem);
+    dsd_tile<Single, 128, TRANS_A, true, 1, SCATTER>(g, const_ints(plan.list(kTallSingles))[item / ntn], item % ntn, smem);
     return true;
   }
   bid -= single_tiles;

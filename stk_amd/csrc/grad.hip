@@ -26,22 +26,25 @@ template <class DsdFused, class DsdTriple, class DsdSingle, class DdsFused, clas
 __global__ __launch_bounds__(512, 2) void dsd_dds_kernel(DsdArgs d, PlanLists rows, DdsArgs s, PlanLists cols) {
   extern __shared__ __align__(16) char smem[];
   static_assert(DdsFused::TM == DdsSingle::TM, "same row tiling");
-  const int ntm = s.m / DdsFused::TM;
+  const int ntm = (s.m + DdsFused::TM - 1) / DdsFused::TM;
   int bid = blockIdx.x;
   if (dsd_plan_tile<DsdFused, DsdTriple, DsdSingle, false>(d, rows, bid, smem)) return;
   const int pair_tiles = const_ints(cols.counts)[kPairs] * ntm, single_tiles = const_ints(cols.counts)[kSingles] * ntm;
   if (bid < pair_tiles) {
     const int item = xcd_item(bid, pair_tiles, ntm, cols.group(kPairs));
-    dds_tile<DdsFused, 128, false, true, 2>(s, const_ints(cols.list(kPairs))[item / ntm], (item % ntm) * DdsFused::TM, smem);
+    dds_tile<DdsFused, 128, false, true, 2>(s, const_ints(cols.list(kPairs))[item / ntm], item % ntm, smem);
     return;
   }
   bid -= pair_tiles;
   if (bid < single_tiles) {
     // (in order of length: no contiguous shares; by stripes of the dense operand when the plan says so, in its 256-wide tiles)
     const int item = xcd_lines(bid, single_tiles, ntm, (cols.stripe_from(false) + 1) >> 1);
-    dds_tile<DdsSingle, 128, false, true, 1>(s, const_ints(cols.list(kSingles))[item / ntm], (item % ntm) * DdsSingle::TM, smem);
+    dds_tile<DdsSingle, 128, false, true, 1>(s, const_ints(cols.list(kSingles))[item / ntm], item % ntm, smem);
   }
 }
+
+// Tiles of 256 rows or columns of a dense extent.
+constexpr int64_t column_tiles(int64_t extent) { return (extent + 255) / 256; }
 
 constexpr int largest(std::initializer_list<int> values) {
   int most = 0;
@@ -64,7 +67,7 @@ static void launch_dsd_dds(const DsdArgs& d, const PlanLists& rows, const DdsArg
   static const int once = (set_lds_limit(kernel, lds), 0);
   (void)once;
   // upper bound: every line a tile of its own in both products
-  const int grid = d.block_rows * (d.n / DsdFused::TN) + s.block_cols * (s.m / DdsFused::TM);
+  const int grid = d.block_rows * column_tiles(d.n) + s.block_cols * column_tiles(s.m);
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds, stream, d, rows, s, cols);
 }
 
@@ -94,7 +97,7 @@ static void launch_dsd_dsd(const DsdArgs& d, const PlanLists& rows, const DsdArg
   static const int once = (set_lds_limit(kernel, lds), 0);
   (void)once;
   // upper bound: every line a tile of its own in both products
-  const int grid = d.block_rows * (d.n / Fused::TN) + t.block_rows * (t.n / FusedT::TN);
+  const int grid = d.block_rows * column_tiles(d.n) + t.block_rows * column_tiles(t.n);
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds, stream, d, rows, t, cols);
 }
 
@@ -133,7 +136,7 @@ static void launch_sdd_dsd(const SddArgs& a, const DsdArgs& d, const PlanLists& 
   // the walkers of the sdd (as many as it would have workgroups on its own), then every line of the dsd a tile of its own
   const int most = (int)sdd_max_tiles(a.block_rows, a.nnz), units = STK_SDD_PERSISTENT ? compute_units() : 0;
   const int walkers = units > 0 && units < most ? units : most;
-  const int grid = walkers + d.block_rows * (d.n / DsdFused::TN);
+  const int grid = walkers + d.block_rows * column_tiles(d.n);
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds, stream, a, d, lines, walkers);
 }
 
@@ -163,9 +166,9 @@ extern "C" int stk_dsd_dds(int64_t m, int64_t k,
                    block_offsets_t, 0, out_dds, out_dds_stride, nnz, blocking, dtype, index_dtype, plan, &dds);
   if (rc != STK_OK) return rc;
   // (the grid of the one launch - an upper bound on the tiles of both products - must be a 32-bit count)
-  const bool together = plan && blocking == 128 && nnz > 0 && !dsd.empty && !dds.empty && dsd.bk && !dds.ak && n_dsd % 256 == 0 &&
-                        m_dds % 256 == 0 && !dsd.g.small && !dds.g.small &&
-                        (int64_t)dsd.g.block_rows * (n_dsd / 256) + (int64_t)dds.g.block_cols * (m_dds / 256) <= INT32_MAX;
+  const bool together = plan && blocking == 128 && nnz > 0 && !dsd.empty && !dds.empty && dsd.bk && !dds.ak && edge_tiles(n_dsd, 256) &&
+                        edge_tiles(m_dds, 256) && !dsd.g.small && !dds.g.small &&
+                        (int64_t)dsd.g.block_rows * column_tiles(n_dsd) + (int64_t)dds.g.block_cols * column_tiles(m_dds) <= INT32_MAX;
   if (!together) {
     // shapes or layouts the joint launch has no tiles for: the two products one after the other
     rc = stk_dsd(m, k, n_dsd, data, offsets, column_indices, offsets_t, column_indices_t, block_offsets_t, 0, rhs, rhs_stride_k, rhs_stride_n,
@@ -207,9 +210,9 @@ extern "C" int stk_dsd_dsd(int64_t m, int64_t k,
                    rhs_t_stride_n, out_t, out_t_stride, nnz, blocking, dtype, index_dtype, plan, &transposed);
   if (rc != STK_OK) return rc;
   // (the grid of the one launch - an upper bound on the tiles of both products - must be a 32-bit count)
-  const bool together = plan && blocking == 128 && nnz > 0 && !plain.empty && !transposed.empty && !plain.bk && !transposed.bk && n % 256 == 0 &&
-                        n_t % 256 == 0 && !plain.g.small && !transposed.g.small &&
-                        (int64_t)plain.g.block_rows * (n / 256) + (int64_t)transposed.g.block_rows * (n_t / 256) <= INT32_MAX;
+  const bool together = plan && blocking == 128 && nnz > 0 && !plain.empty && !transposed.empty && !plain.bk && !transposed.bk && edge_tiles(n, 256) &&
+                        edge_tiles(n_t, 256) && !plain.g.small && !transposed.g.small &&
+                        (int64_t)plain.g.block_rows * column_tiles(n) + (int64_t)transposed.g.block_rows * column_tiles(n_t) <= INT32_MAX;
   if (!together) {
     // shapes or layouts the joint launch has no tiles for: the two products one after the other
     rc = stk_dsd(m, k, n, data, offsets, column_indices, offsets_t, column_indices_t, block_offsets_t, 0, rhs, rhs_stride_k, rhs_stride_n, out,
@@ -257,8 +260,8 @@ extern "C" int stk_sdd_dsd(int64_t m, int64_t n,
                    rhs_dsd, rhs_dsd_stride_k, rhs_dsd_stride_n, out_dsd, out_dsd_stride, nnz, blocking, dtype, index_dtype, plan, &dsd);
   if (rc != STK_OK) return rc;
   const bool together = plan && blocking == 128 && !sdd.empty && !dsd.empty && sdd.g.tiles && nnz > compute_units() && sdd.ak && sdd.bk &&
-                        k_sdd % 64 == 0 && !dsd.bk && n_dsd % 256 == 0 && !dsd.g.small &&
-                        sdd_max_tiles(sdd.g.block_rows, nnz) + (int64_t)dsd.g.block_rows * (n_dsd / 256) <= INT32_MAX;
+                        k_sdd % 64 == 0 && !dsd.bk && edge_tiles(n_dsd, 256) && !dsd.g.small &&
+                        sdd_max_tiles(sdd.g.block_rows, nnz) + (int64_t)dsd.g.block_rows * column_tiles(n_dsd) <= INT32_MAX;
   if (!together) {
     // shapes or layouts the joint launch has no tiles for: the two products one after the other
     rc = stk_sdd(lhs, lhs_stride_m, lhs_stride_k, rhs_sdd, rhs_sdd_stride_k, rhs_sdd_stride_n, m, k_sdd, n, out_sdd, offsets, row_indices,

@@ -112,7 +112,7 @@ def dsd_scatter(a, rhs, route, weights=None):
     """padded_scatter(stk.ops.dsd(a, rhs), route, weights) in one launch for top_k = 1: the product's store writes
     every row to its token's place (times its weight), and the padded result is never made.  The result is
     bit-identical to the two steps.  Used when nothing needs a gradient, the routing is top-1 and the library has the
-    kernel (128-blocks, a multiple of 256 columns, enough work for the eight-wavefront tiles); otherwise the two steps
+    kernel (128-blocks, at least 256 columns, enough work for the eight-wavefront tiles); otherwise the two steps
     run."""
     from stk_amd.ops import linear_ops
     assert isinstance(a, Matrix)
