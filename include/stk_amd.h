@@ -217,6 +217,9 @@ int stk_activation_product(const void* sums, const void* factor, void* out, int6
  * when it is misaligned.
  */
 int64_t stk_dsd_workspace_bytes(int64_t m, int64_t n, int blocking);
+/* 1 when a stk_dsd of nnz blocks with n columns has too little work per compute unit for the tiles whose last round is cut:
+ * it then makes no use of a workspace. */
+int stk_dsd_is_small(int64_t nnz, int64_t n);
 int64_t stk_dsd_workspace_counter_bytes(void);
 int64_t stk_dsd_workspace_slot_bytes(void);
 /*
@@ -452,8 +455,18 @@ int stk_route(const int32_t* top_experts, int64_t slots, int64_t num_experts, in
               void* workspace, size_t workspace_bytes, stk_stream_t stream);
 
 /*
+ * stk_route that also stores padded_bins[num_experts - 1], the rows the padded layout needs, in *total (or NULL) as soon as it
+ * is known, in front of the sorted outputs.  total may be pinned host memory: set to -1 before the call it can be
+ * polled, so that the host learns the number without a copy and without waiting for the stream.
+ */
+int stk_route_total(const int32_t* top_experts, int64_t slots, int64_t num_experts, int blocking, int64_t padded_rows,
+                    int32_t* indices, int32_t* bin_ids, int32_t* bins, int32_t* padded_bins,
+                    int32_t* slot_rows, int32_t* row_slots,
+                    void* workspace, size_t workspace_bytes, int32_t* total, stk_stream_t stream);
+
+/*
  * stk_route for callers that cannot allocate device memory or hand over a workspace (code under HIP graph
- * capture, tight serving loops, harnesses that forbid hipMalloc): the same three launches with the same
+ * capture, tight serving loops, harnesses that forbid hipMalloc): the same launches with the same
  * outputs, bit for bit, but the per-tile table lives in a device array that belongs to the library
  * (STK_ROUTE_STATIC_MAX_ENTRIES int32 entries = 4 MiB on every GPU the library runs on, held until the process
  * ends).  No counterpart in the reference.  The call allocates nothing and frees nothing; the first call on a

@@ -10,6 +10,7 @@ import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), "libstk_amd.so")
+NATIVE_PATH = os.path.join(os.path.dirname(_HERE), "_native.so")
 
 ABI_VERSION = 17
 STK_OK, STK_ERR_DIMS, STK_ERR_UNSUPPORTED, STK_ERR_HIP, STK_ERR_WORKSPACE = 0, 1, 2, 3, 4
@@ -32,6 +33,7 @@ SIGNATURES = {
     "stk_dsd_workspace_bytes": (_i64, [_i64, _i64, _int]),
     "stk_dsd_workspace_counter_bytes": (_i64, []),
     "stk_dsd_workspace_slot_bytes": (_i64, []),
+    "stk_dsd_is_small": (_int, [_i64, _i64]),
     "stk_dsd_tail_slices": (_int, [_i64, _i64, _i64, ctypes.c_double, _int]),
     "stk_dsd": (_int, [_i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _int, _p, _i64, _i64, _p, _i64, _i64, _int, _int, _int, _p, _p, _i64, _p]),
     "stk_dds": (_int, [_i64, _i64, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _p, _int, _p, _i64, _i64, _int, _int, _int, _p, _p]),
@@ -54,6 +56,7 @@ SIGNATURES = {
     "stk_dmoe_topology_plan": (_int, [_p, _i64, _int, _i64, _i64, _int, _p, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "stk_route_workspace_bytes": (_sz, [_i64, _i64]),
     "stk_route": (_int, [_p, _i64, _i64, _int, _i64, _p, _p, _p, _p, _p, _p, _p, _sz, _p]),
+    "stk_route_total": (_int, [_p, _i64, _i64, _int, _i64, _p, _p, _p, _p, _p, _p, _p, _sz, _p, _p]),
     "stk_route_static": (_int, [_p, _i64, _i64, _int, _i64, _p, _p, _p, _p, _p, _p, _p]),
     "stk_padded_gather": (_int, [_p, _i64, _i64, _i64, _p, _p, _int, _i64, _p, _i64, _int, _p]),
     "stk_padded_scatter": (_int, [_p, _i64, _i64, _i64, _p, _p, _int, _i64, _p, _i64, _int, _p]),
@@ -86,6 +89,23 @@ def load():
                 raise RuntimeError("stk_amd: libstk_amd.so has an unexpected ABI version; rebuild it")
             _lib = lib
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The native boundary (csrc/native.cc), built next to the library: the functions that take torch tensors."""
+    global _native
+    if _native is None:
+        load()
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(f"stk_amd: {NATIVE_PATH} is missing. Build it with `make -C stk_amd/csrc`; there is no fallback implementation.")
+        from stk_amd import _native as module
+        if module.abi_version() != ABI_VERSION:
+            raise RuntimeError("stk_amd: _native.so has an unexpected ABI version; rebuild it")
+        _native = module
+    return _native
 
 
 def check(status):

@@ -12,6 +12,8 @@ is produced in the layout of the underlying storage and returned as .t(), so
 that it accumulates into the base tensor without a copy.  Sparse operands carry
 a transpose flag instead of a view; the kernels then walk the CSC metadata.
 """
+import functools
+
 import torch
 
 from stk_amd.backend import hip_kernels as backend
@@ -41,25 +43,25 @@ class _Sparse:
         return (self.shape[1], self.shape[0]) if transposed else self.shape
 
 
-def _run_dsd(sp, data, transposed, rhs):
+def _run_dsd(sp, data, transposed, rhs, stream=-1):
     shape = sp.logical_shape(transposed)
     out = torch.empty((shape[0], rhs.size(1)), dtype=rhs.dtype, device=rhs.device)
-    backend.dsd(shape, data, *sp.meta, transposed, rhs, out)
+    backend.dsd(shape, data, *sp.meta, transposed, rhs, out, stream)
     return out
 
 
-def _run_dds(lhs, sp, data, transposed):
+def _run_dds(lhs, sp, data, transposed, stream=-1):
     shape = sp.logical_shape(transposed)
     out = torch.empty((lhs.size(0), shape[1]), dtype=lhs.dtype, device=lhs.device)
-    backend.dds(lhs, shape, data, *sp.meta, transposed, out)
+    backend.dds(lhs, shape, data, *sp.meta, transposed, out, stream)
     return out
 
 
-def _run_sdd(lhs, rhs, sp):
+def _run_sdd(lhs, rhs, sp, stream=-1):
     out = torch.empty(sp.data.shape, dtype=lhs.dtype, device=lhs.device)
     offsets, row_indices, column_indices, _, _, block_offsets_t = sp.meta
     # visiting blocks column by column keeps the rhs panel of a block column in cache
-    backend.sdd(lhs, rhs, sp.shape, out, offsets, row_indices, column_indices, block_order=block_offsets_t)
+    backend.sdd(lhs, rhs, sp.shape, out, offsets, row_indices, column_indices, block_order=block_offsets_t, stream=stream)
     return out
 
 
@@ -67,6 +69,10 @@ def _run_sdd(lhs, rhs, sp):
 # switch on, the second one runs on a side stream (default priority) next to the first: the workgroups of one
 # fill the compute units that the other leaves idle in its last round.
 OVERLAP_GRADIENTS = True
+# ... for products of at least this many FLOP each.  Two events to record and to wait for cost about 30 us; both gradients
+# of a dsd took, one after the other / side by side, 38 / 70 us at 4 GFLOP, 61 / 67 us at 17, 103 / 98 us at 34 and
+# 188 / 166 us at 69 (those of a dds 99 / 103 us at 34 and 182 / 187 us at 69).
+OVERLAP_FROM = 4e10
 _side_streams = {}
 # Both gradients of sdd (stk_dsd_dds, stk_dsd_dsd) in one launch where the operands' layouts allow it, instead of two
 # launches side by side; the same results.
@@ -82,24 +88,35 @@ def _side_stream(device):
     stream = _side_streams.get(device.index)
     if stream is None:
         stream = _side_streams[device.index] = torch.cuda.Stream(device=device)
-        backend.CONCURRENT_STREAMS.add(stream.cuda_stream)   # its dsd launches get a workspace of their own
+        backend.CONCURRENT_STREAMS[stream.cuda_stream] = stream   # its dsd launches get a workspace of their own
     return stream
 
 
-def _both(first, second, device):
-    """first() and second() -> their results (None for a callable that is None), launched side by side when
-    both are wanted.  Each callable launches one product and returns its freshly allocated output."""
-    if first is None or second is None or not OVERLAP_GRADIENTS or device.type != "cuda":
-        return (first() if first is not None else None), (second() if second is not None else None)
-    main = torch.cuda.current_stream(device)
-    side = _side_stream(device)
-    side.wait_stream(main)          # the operands are ready on the main stream
-    with torch.cuda.stream(side):
-        b = second()
-    a = first()
-    main.wait_stream(side)          # whatever follows on the main stream sees both results
-    b.record_stream(main)           # allocated under the side stream, used and freed under the main one
+def _both(first, second, sp, width):
+    """first(stream) and second(stream) -> their results (None for a callable that is None), launched side by side when
+    both are wanted.  Each callable launches one product, of sp's values with `width` columns or rows, on the stream with the
+    given handle (-1: the current one) and returns its freshly allocated output."""
+    if first is None or second is None:
+        return (first(-1) if first is not None else None), (second(-1) if second is not None else None)
+    data = sp.data
+    if not OVERLAP_GRADIENTS or not data.is_cuda or 2.0 * data.numel() * width < OVERLAP_FROM:
+        return first(-1), second(-1)
+    offsets, _, column_indices, offsets_t, column_indices_t, _ = sp.meta
+    backend.prepare_plan(data, offsets, column_indices, offsets_t, column_indices_t)   # built, if at all, in front of both
+    follow = backend.follow_stream
+    main, side = backend._stream(data.device), _side_stream(data.device).cuda_stream
+    follow(side, main)              # the operands are ready on the main stream
+    try:
+        # (both outputs come from the main stream's memory; the side stream's use of it lies between the two waits)
+        b = second(side)
+        a = first(-1)
+    finally:
+        follow(main, side)          # whatever follows on the main stream sees both results
     return a, b
+
+
+def _wants_grad(*tensors):
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
 class DSD(torch.autograd.Function):
@@ -108,10 +125,11 @@ class DSD(torch.autograd.Function):
     @custom_fwd
     def forward(ctx, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
                 block_offsets_t, transpose_a, rhs):
-        ctx.save_for_backward(data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
-                              block_offsets_t, rhs)
-        ctx.storage_shape = (shape[1], shape[0]) if transpose_a else tuple(shape)
-        ctx.transpose_a = transpose_a
+        if ctx is not None:     # (None: nothing needs a gradient)
+            ctx.save_for_backward(data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
+                                  block_offsets_t, rhs)
+            ctx.storage_shape = (shape[1], shape[0]) if transpose_a else tuple(shape)
+            ctx.transpose_a = transpose_a
         out = torch.empty((shape[0], rhs.size(1)), dtype=rhs.dtype, device=rhs.device)
         backend.dsd(shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
                     block_offsets_t, transpose_a, rhs, out)
@@ -138,13 +156,13 @@ class DSD(torch.autograd.Function):
             return None, ddata, None, None, None, None, None, None, None, drhs
         if ctx.needs_input_grad[1]:
             # d op(S) = dy rhs^T on the pattern; for a transposed S the stored blocks hold (rhs dy^T)
-            want_data = (lambda: _run_sdd(rhs, dy.t(), sp)) if ta else (lambda: _run_sdd(dy, rhs.t(), sp))
+            want_data = (lambda stream: _run_sdd(rhs, dy.t(), sp, stream)) if ta else (lambda stream: _run_sdd(dy, rhs.t(), sp, stream))
         if ctx.needs_input_grad[9]:
             if rhs_is_view:
-                want_rhs = lambda: _run_dds(dy.t(), sp, data, ta)       # dy^T op(S), returned transposed
+                want_rhs = lambda stream: _run_dds(dy.t(), sp, data, ta, stream)       # dy^T op(S), returned transposed
             else:
-                want_rhs = lambda: _run_dsd(sp, data, not ta, dy)       # op(S)^T dy
-        ddata, drhs = _both(want_data, want_rhs, dy.device)
+                want_rhs = lambda stream: _run_dsd(sp, data, not ta, dy, stream)       # op(S)^T dy
+        ddata, drhs = _both(want_data, want_rhs, sp, dy.size(1))
         if drhs is not None and rhs_is_view:
             drhs = drhs.t()
         return None, ddata, None, None, None, None, None, None, None, drhs
@@ -156,10 +174,11 @@ class DDS(torch.autograd.Function):
     @custom_fwd
     def forward(ctx, lhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
                 block_offsets_t, transpose_b):
-        ctx.save_for_backward(lhs, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
-                              block_offsets_t)
-        ctx.storage_shape = (shape[1], shape[0]) if transpose_b else tuple(shape)
-        ctx.transpose_b = transpose_b
+        if ctx is not None:
+            ctx.save_for_backward(lhs, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
+                                  block_offsets_t)
+            ctx.storage_shape = (shape[1], shape[0]) if transpose_b else tuple(shape)
+            ctx.transpose_b = transpose_b
         out = torch.empty((lhs.size(0), shape[1]), dtype=lhs.dtype, device=lhs.device)
         backend.dds(lhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
                     block_offsets_t, transpose_b, out)
@@ -176,13 +195,13 @@ class DDS(torch.autograd.Function):
         lhs_is_view = _is_transposed_view(lhs)
         if ctx.needs_input_grad[0]:
             if lhs_is_view:
-                want_lhs = lambda: _run_dsd(sp, data, tb, dy.t())       # op(S) dy^T, returned transposed
+                want_lhs = lambda stream: _run_dsd(sp, data, tb, dy.t(), stream)       # op(S) dy^T, returned transposed
             else:
-                want_lhs = lambda: _run_dds(dy, sp, data, not tb)       # dy op(S)^T
+                want_lhs = lambda stream: _run_dds(dy, sp, data, not tb, stream)       # dy op(S)^T
         if ctx.needs_input_grad[2]:
             # d op(S) = lhs^T dy on the pattern; for a transposed S the stored blocks hold (dy^T lhs)
-            want_data = (lambda: _run_sdd(dy.t(), lhs, sp)) if tb else (lambda: _run_sdd(lhs.t(), dy, sp))
-        dlhs, ddata = _both(want_lhs, want_data, dy.device)
+            want_data = (lambda stream: _run_sdd(dy.t(), lhs, sp, stream)) if tb else (lambda stream: _run_sdd(lhs.t(), dy, sp, stream))
+        dlhs, ddata = _both(want_lhs, want_data, sp, dy.size(0))
         if dlhs is not None and lhs_is_view:
             dlhs = dlhs.t()
         return dlhs, None, ddata, None, None, None, None, None, None, None
@@ -207,15 +226,15 @@ def _sdd_operand_gradients(ctx, lhs, rhs, sp, ds):
         return dlhs, dbase.t()
     if ctx.needs_input_grad[0]:
         if lhs_is_view:
-            want_lhs = lambda: _run_dds(rhs, sp, ds, True)              # rhs dS^T, returned transposed
+            want_lhs = lambda stream: _run_dds(rhs, sp, ds, True, stream)              # rhs dS^T, returned transposed
         else:
-            want_lhs = lambda: _run_dsd(sp, ds, False, rhs.t())         # dS rhs^T
+            want_lhs = lambda stream: _run_dsd(sp, ds, False, rhs.t(), stream)         # dS rhs^T
     if ctx.needs_input_grad[1]:
         if rhs_is_view:
-            want_rhs = lambda: _run_dsd(sp, ds, True, lhs)              # dS^T lhs, returned transposed
+            want_rhs = lambda stream: _run_dsd(sp, ds, True, lhs, stream)              # dS^T lhs, returned transposed
         else:
-            want_rhs = lambda: _run_dds(lhs.t(), sp, ds, False)         # lhs^T dS
-    dlhs, drhs = _both(want_lhs, want_rhs, ds.device)
+            want_rhs = lambda stream: _run_dds(lhs.t(), sp, ds, False, stream)         # lhs^T dS
+    dlhs, drhs = _both(want_lhs, want_rhs, sp, lhs.size(1))
     if dlhs is not None and lhs_is_view:
         dlhs = dlhs.t()
     if drhs is not None and rhs_is_view:
@@ -229,9 +248,10 @@ class SDD(torch.autograd.Function):
     @custom_fwd
     def forward(ctx, lhs, rhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
                 block_offsets_t):
-        ctx.save_for_backward(lhs, rhs, offsets, row_indices, column_indices, offsets_t, column_indices_t,
-                              block_offsets_t)
-        ctx.shape = tuple(shape)
+        if ctx is not None:
+            ctx.save_for_backward(lhs, rhs, offsets, row_indices, column_indices, offsets_t, column_indices_t,
+                                  block_offsets_t)
+            ctx.shape = tuple(shape)
         out = torch.empty(data.shape, dtype=lhs.dtype, device=lhs.device)
         backend.prepare_plan(data, offsets, column_indices, offsets_t, column_indices_t)
         backend.sdd(lhs, rhs, shape, out, offsets, row_indices, column_indices, block_order=block_offsets_t)
@@ -267,11 +287,13 @@ class SDDFused(torch.autograd.Function):
             raise ValueError(f"unknown activation {activation!r}")
         out = torch.empty(data.shape, dtype=lhs.dtype, device=lhs.device)
         values = None if multiplier is None else multiplier.detach().contiguous()
-        keep = bool(save_sums) and activation not in (None, "none") and lhs.is_cuda and any(ctx.needs_input_grad)
+        keep = bool(save_sums) and activation not in (None, "none") and lhs.is_cuda and ctx is not None
         sums = torch.empty_like(out) if keep else None
         backend.prepare_plan(data, offsets, column_indices, offsets_t, column_indices_t)
         backend.sdd_fused(lhs, rhs, shape, out, offsets, row_indices, column_indices, activation, values,
                           block_order=block_offsets_t, sums=sums)
+        if ctx is None:
+            return out
         ctx.save_for_backward(lhs, rhs, offsets, row_indices, column_indices, offsets_t, column_indices_t,
                               block_offsets_t, *(() if values is None else (values,)), *(() if sums is None else (sums,)))
         ctx.shape = tuple(shape)
@@ -320,8 +342,28 @@ class RowIndices(torch.autograd.Function):
         return out
 
 
-dsd = DSD.apply
-dds = DDS.apply
-sdd = SDD.apply
-sdd_fused = SDDFused.apply
+# The functions that stk.ops calls.  When nothing needs a gradient the forward pass runs by itself: the bookkeeping of
+# an autograd function costs as much host time as the launch.
+def dsd(shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_a, rhs):
+    run = DSD.apply if _wants_grad(data, rhs) else functools.partial(DSD.forward, None)
+    return run(shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_a, rhs)
+
+
+def dds(lhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_b):
+    run = DDS.apply if _wants_grad(data, lhs) else functools.partial(DDS.forward, None)
+    return run(lhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_b)
+
+
+def sdd(lhs, rhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t):
+    run = SDD.apply if _wants_grad(lhs, rhs) else functools.partial(SDD.forward, None)
+    return run(lhs, rhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t)
+
+
+def sdd_fused(lhs, rhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, activation, multiplier,
+              save_sums=False):
+    run = SDDFused.apply if _wants_grad(lhs, rhs, multiplier) else functools.partial(SDDFused.forward, None)
+    return run(lhs, rhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, activation, multiplier,
+               save_sums)
+
+
 row_indices = RowIndices.apply

@@ -97,6 +97,16 @@ def _host_only(*tensors):
             raise RuntimeError("stk_amd: operands of one product must all live in host memory or all on one GPU")
 
 
+def matmul_dims(inner, m, k, n, blocking):
+    """The reference's shape checks, for the calls of its four functions that end up here."""
+    # stk/backend/triton_kernels.py:243, 299, 351 and :15-19 with BLOCK_M = BLOCK_N = blocking, BLOCK_K = 32
+    assert inner == k, "incompatible dimensions"
+    msg = "incompatible dimensions: tensor has dim with length: {}, which must be divisible by {}"
+    assert m % blocking == 0, msg.format(m, blocking)
+    assert k % 32 == 0, msg.format(k, 32)
+    assert n % blocking == 0, msg.format(n, blocking)
+
+
 def sdd(lhs, rhs, shape, out, offsets, row_indices, column_indices):
     _host_only(lhs, rhs, out, row_indices, column_indices)
     m, k = lhs.shape

@@ -461,7 +461,7 @@ int stk::dsd_problem(const char* who, int64_t m, int64_t k, int64_t n,
   p->stream_rhs = !bk && nnz <= 4 * (k / blocking);
   p->ta = ta;
   p->bk = bk;
-  g.small = nnz * (n / 128) < kSmallWorkPerUnit * compute_units();
+  g.small = stk_dsd_is_small(nnz, n);
   if (!g.walk_offsets || (nnz > 0 && (!g.walk_columns || (ta && !g.walk_blocks) || !data))) return fail(STK_ERR_DIMS, "%s: missing metadata pointer", who);
   // lists of the walked lines: block rows of the stored matrix [m, k], or block columns of the stored [k, m]
   p->lists = PlanLists{nullptr, nullptr, 0};
@@ -569,3 +569,5 @@ extern "C" int64_t stk_dsd_workspace_bytes(int64_t m, int64_t n, int blocking) {
   if (workgroups <= 0 || (m / 128) * (n / 128) / 3 >= 8 * (int64_t)workgroups) return 0;
   return (int64_t)tail_workspace_bytes(workgroups);
 }
+
+extern "C" int stk_dsd_is_small(int64_t nnz, int64_t n) { return nnz * (n / 128) < stk::kSmallWorkPerUnit * stk::compute_units(); }

@@ -24,17 +24,10 @@ def route(top_experts, num_experts, blocking, padded_rows=None):
     slot_rows            row of slot token * top_k + choice in the padded layout
     row_slots            slot held by each row of the padded layout, -1 for padding
 
-    padded_rows: rows of the padded layout.  None reads padded_bins[-1] back (one device
-    synchronisation, exact size); an int that is at least padded_bins[-1] avoids that -
+    padded_rows: rows of the padded layout.  None waits for padded_bins[-1] on the host (exact size); an int that is at least padded_bins[-1] avoids that -
     `route_capacity` gives one that is always enough."""
     top_k = top_experts.size(1) if top_experts.dim() == 2 else 1
-    slots = top_experts.numel()
-    exact = padded_rows is None
-    capacity = route_capacity(slots, num_experts, blocking) if exact else padded_rows
-    r = hip_kernels.route(top_experts, num_experts, blocking, capacity)
-    indices, bin_ids, bins, padded_bins, slot_rows, row_slots = r
-    if exact:
-        row_slots = row_slots[:int(padded_bins[-1].item())]
+    indices, bin_ids, bins, padded_bins, slot_rows, row_slots = hip_kernels.route(top_experts, num_experts, blocking, padded_rows)
     return Route(indices, bin_ids, bins, padded_bins, slot_rows, row_slots, top_k, blocking)
 
 
@@ -77,12 +70,16 @@ class _PaddedScatter(torch.autograd.Function):
 def padded_gather(x, route):
     """x [tokens, hidden] -> [padded_rows, hidden]: every slot's token row at its place in the padded
     layout, zeros in the padding rows."""
+    if not _wants_grad(x):
+        return hip_kernels.padded_gather(x, route.row_slots, route.top_k)
     return _PaddedGather.apply(x, route)
 
 
 def padded_scatter(x, route, weights=None):
     """x [padded_rows, hidden] -> [tokens, hidden]: each token's top_k rows, multiplied by
     weights [tokens, top_k] (or [tokens * top_k]) when given, added up in fp32 in the order of the choices."""
+    if not _wants_grad(x, weights):
+        return hip_kernels.padded_scatter(x, route.slot_rows, route.top_k, weights)
     return _PaddedScatter.apply(x, route, weights)
 
 
