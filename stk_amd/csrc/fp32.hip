@@ -384,15 +384,52 @@ __global__ __launch_bounds__(kThreads, 2) void sdd_fast_kernel(SddArgs g, int nn
   t.store(g.out + at, BLK, g.activation, g.multiplier ? g.multiplier + at : nullptr, smem);
 }
 
+// Which tile workgroup `block` computes: line, stretch of the line, tile of the dense operand.  A line takes as long as it
+// has blocks, and a launch with one tile per compute unit as long as its longest line, so the lines are spread evenly over
+// the dies - every die takes all lines for its eighth of the dense operand - and a die's workgroups come longest line first,
+// every second round of its compute units in reverse, so that the units, which hold several small tiles at once, get about
+// equal sums.  More than 64 lines are left in their order: there are enough tiles for the dispatch to even them out.
+struct WalkItem {
+  int line, stretch, tile;
+};
+template <int SIDE>
+__device__ __forceinline__ WalkItem walk_item(const int32_t* offsets, int lines, int tiles, int items) {
+  constexpr int kDies = 8, kUnitsPerDie = 32;
+  const int lane = threadIdx.x & 63, block = uniform((int)blockIdx.x);
+  if (lines > 64) {
+    const int item = xcd_chunked(block, items);
+    return {item / (SIDE * tiles), item % SIDE, item / SIDE % tiles};
+  }
+  const int die = block % kDies, on_die = (items - die + kDies - 1) / kDies;
+  int at = block / kDies;
+  if ((at / kUnitsPerDie) % 2 == 1 && (at / kUnitsPerDie + 1) * kUnitsPerDie <= on_die)
+    at = at / kUnitsPerDie * kUnitsPerDie + kUnitsPerDie - 1 - at % kUnitsPerDie;
+  int rank, rest;   // rank of the line by length; stretch and tile
+  if (tiles % kDies == 0) {
+    const int per_line = SIDE * (tiles / kDies);
+    rank = at / per_line, rest = at % per_line + die * per_line;
+  } else {
+    const int item = at * kDies + die;
+    rank = item / (SIDE * tiles), rest = item % (SIDE * tiles);
+  }
+  // lane i: the length of line i and how many lines come before it
+  const int mine = lane < lines ? offsets[lane + 1] - offsets[lane] : -1;
+  int before = 0;
+  for (int i = 0; i < lines; i++) {
+    const int other = __builtin_amdgcn_readlane(mine, i);
+    before += other > mine || (other == mine && i < lane);
+  }
+  const int line = (int)__ffsll((unsigned long long)__ballot(lane < lines && before == rank)) - 1;
+  return {line, rest % SIDE, rest / SIDE};
+}
+
 // One T-wide stretch of a line of op(S) against a T-wide tile of the dense operand.
 template <int BLK, int T, bool SPARSE_LHS, bool AK, bool BK>
-__global__ __launch_bounds__(kThreads, 2) void walk_fast_kernel(WalkArgs g, int items) {
+__global__ __launch_bounds__(kThreads, 2) void walk_fast_kernel(WalkArgs g, int lines, int items) {
   __shared__ __align__(16) char smem[Fast<T, AK, BK>::kLds];
   constexpr int kSide = BLK / T, kPer = BLK / kFastKT;
-  const int tiles = g.free_extent / T;
-  const int item = xcd_chunked(blockIdx.x, items);
-  // (the stretches of a line next to each other: they share the tile of the dense operand)
-  const int stretch = item % kSide, line = item / (kSide * tiles), f0 = item / kSide % tiles * T, l0 = stretch * T;
+  const WalkItem item = walk_item<kSide>(g.walk_offsets, lines, g.free_extent / T, items);
+  const int line = uniform(item.line), f0 = uniform(item.tile) * T, l0 = uniform(item.stretch) * T;
   const int lane = threadIdx.x & 63;
   const int begin = uniform(g.walk_offsets[line]), end = uniform(g.walk_offsets[line + 1]);
   const float* dense0 = g.dense + (int64_t)f0 * g.ds_outer;
@@ -419,19 +456,24 @@ __global__ __launch_bounds__(kThreads, 2) void walk_fast_kernel(WalkArgs g, int 
 }
 
 // Side of the output tiles for a problem of `area` tiles of 32 x 32 whose extents are multiples of `most`.  The matrix pipe
-// is the bound, so a tile that leaves compute units without work, or with a second tile while others have none, costs in
+// is the bound, so a tile that leaves compute units without work, or with a longer line than others have, costs in
 // proportion, while a smaller tile than needed moves more operand bytes per FLOP.  Kernel times in us with tiles of 128 /
 // 64 / 32:
-//   sdd, 32 blocks of 128, k = 1024 (32 / 128 / 512 tiles)            66 / 23 / 15
-//   dsd, 1024 x 1024 half full x 1024 (64 / 256 / 1024 tiles)         69 / 26 / 27
-//   dds, 3072 x 3072 half full, 2048 rows (384 / 1536 / 6144 tiles)  254 / 175 / 213
-//   dsd, 4096 x 4096 half full x 4096 (1024 / 4096 / 16384 tiles)    546 / 587 / 728
-// so 64 as soon as every unit gets a tile, 128 from four of them for every unit on.  (Before these kernels, with a 128 x 128
-// tile per block in all of these cases: sdd 69, dsd 68, and 990 for the dsd of 4096 x 4096.)
+//   sdd, 32 blocks of 128, k = 1024 (32 / 128 / 512 tiles)            66 / 24 / 15
+//   sdd, 64 blocks of 128, k = 2048 (64 / 256 / 1024 tiles)            - / 49 / 45
+//   dsd, 1024 x 1024 half full x 1024 (64 / 256 / 1024 tiles)         69 / 27 / 17
+//   dsd, 1536 x 640, 30 % full, x 896 (84 / 336 / 1344 tiles)          - / 14 / 12
+//   sdd, 128 blocks of 128, k = 2048 (128 / 512 / 2048 tiles)          - / 77 / 85
+//   dsd, 2048 x 2048, a quarter full, x 2048 (256 / 1024 / 4096 tiles) - / 52 / 58
+//   dds, 3072 x 3072 half full, 2048 rows (384 / 1536 / 6144 tiles)  254 / 165 / 207
+//   dsd, 4096 x 4096 half full x 4096 (1024 / 4096 / 16384 tiles)    521 / 566 / 719
+// so 64 as soon as every unit gets two tiles, 128 from four of them for every unit on.  (Before these kernels, with a
+// 128 x 128 tile per block in all of these cases: sdd 69, dsd 68, and 990 for the dsd of 4096 x 4096; with the lines in their
+// order, a line on one die, the dsd of 1024 x 1024 took 26 us with tiles of 64 and 27 with tiles of 32.)
 inline int fast_tile(int64_t area, int most) {
   const int64_t units = compute_units() > 0 ? compute_units() : 256;
   if (most >= 128 && area / 16 >= 4 * units) return 128;
-  return most >= 64 && area / 4 >= units ? 64 : 32;
+  return most >= 64 && area / 4 >= 2 * units ? 64 : 32;
 }
 
 // A float32 array that the transfers can read: unit stride in one dimension, the other one and the base multiples of 16
@@ -504,7 +546,7 @@ int walk_f32(bool sparse_lhs, const char* who, int64_t lines, int64_t free_exten
       const bool sk = line_major, dk = dense_stride_k == 1;
 #define STK_F32_WALK(BLK, T, SL, SK, DK)                                                                                               \
   if (blocking == BLK && t == T && sparse_lhs == SL && sk == SK && dk == DK)                                                           \
-    hipLaunchKernelGGL((f32::walk_fast_kernel<BLK, T, SL, SL ? SK : DK, SL ? DK : SK>), dim3((unsigned)items), dim3(f32::kThreads), 0, stream, g, (int)items);
+    hipLaunchKernelGGL((f32::walk_fast_kernel<BLK, T, SL, SL ? SK : DK, SL ? DK : SK>), dim3((unsigned)items), dim3(f32::kThreads), 0, stream, g, (int)lines, (int)items);
 #define STK_F32_WALK_LAYOUTS(BLK, T, SL) STK_F32_WALK(BLK, T, SL, true, true) STK_F32_WALK(BLK, T, SL, true, false) STK_F32_WALK(BLK, T, SL, false, true) STK_F32_WALK(BLK, T, SL, false, false)
 #define STK_F32_WALKS(BLK, T) STK_F32_WALK_LAYOUTS(BLK, T, true) STK_F32_WALK_LAYOUTS(BLK, T, false)
       STK_F32_WALKS(128, 128) STK_F32_WALKS(128, 64) STK_F32_WALKS(128, 32) STK_F32_WALKS(64, 64) STK_F32_WALKS(64, 32)

@@ -51,6 +51,21 @@ def test_products_of_every_tile_size_and_layout(rows, cols, inner, density, b, v
     _check(stk.ops.dds(w, s.t()), w, dense.t())
 
 
+# lines of very unequal lengths, empty ones among them: the number of lines (64 are ordered by length, 66 are not), and of
+# tiles of the dense operand that is a multiple of the eight dies (1024), or not, with whole and partial rounds of a
+# die's units
+@pytest.mark.parametrize("lines,inner", [(3, 64), (9, 448), (64, 192), (64, 1024), (66, 192)])
+def test_lines_of_unequal_lengths(lines, inner):
+    gen, b = torch.Generator(device=DEV).manual_seed(lines * inner), 64
+    keep = (torch.rand(lines, 8, generator=gen, device=DEV) < torch.linspace(0, 1.2, lines, device=DEV)[torch.randperm(lines, generator=gen, device=DEV)][:, None])
+    keep = keep.float().repeat_interleave(b, 0).repeat_interleave(b, 1)
+    dense = torch.randn(lines * b, 8 * b, generator=gen, device=DEV) * keep
+    s = stk.ops.to_sparse(dense, b)
+    v, a = torch.randn(8 * b, inner, generator=gen, device=DEV), torch.randn(inner, 8 * b, generator=gen, device=DEV)
+    _check(stk.ops.dsd(s, v), dense, v)
+    _check(stk.ops.dds(a, s.t()), a, dense.t())
+
+
 @pytest.mark.parametrize("inner", [32, 96, 160])
 def test_an_inner_size_of_odd_multiples_of_32(inner):
     gen = torch.Generator(device=DEV).manual_seed(inner)
