@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define STK_AMD_ABI_VERSION 17
+#define STK_AMD_ABI_VERSION 18
 
 /* status codes */
 #define STK_OK 0
@@ -346,6 +346,15 @@ int stk_to_dense(const void* data, const void* row_indices, const void* column_i
                  int elem_bytes, int index_dtype, void* out, stk_stream_t stream);
 
 /*
+ * The same, for a caller that has the matrix's offsets[Rb + 1] too (row r's blocks are the
+ * entries offsets[r] .. offsets[r + 1] - 1): where blocks are made of 16-byte pieces the
+ * result is written in one pass, otherwise as by stk_to_dense.
+ */
+int stk_to_dense_rows(const void* data, const int32_t* offsets, const void* row_indices, const void* column_indices,
+                      int64_t nnz, int blocking, int64_t rows, int64_t cols,
+                      int elem_bytes, int index_dtype, void* out, stk_stream_t stream);
+
+/*
  * Dense -> blocked, in two phases because nnz depends on the values
  * (stk/ops/matrix_ops.py:64-85; the reference synchronises in torch.nonzero too).
  *   count: mask[Rb*Cb] (uint8, row-major) = block holds an element that is not
@@ -387,6 +396,21 @@ int stk_to_sparse_gather(const void* x, int64_t rows, int64_t cols, int64_t x_st
                          int blocking, int elem_bytes,
                          const void* row_indices, const void* column_indices, int64_t nnz,
                          int index_dtype, void* data, stk_stream_t stream);
+
+/*
+ * stk_to_sparse_count_nnz, stk_to_sparse_coordinates and, for the transpose metadata,
+ * stk_transpose_meta in two launches, for matrices of at most STK_TO_SPARSE_INDEX_BLOCKS
+ * blocks and 1024 block rows and block columns (larger: STK_ERR_UNSUPPORTED).  The
+ * index arrays have room for Rb*Cb entries, of which the first nnz are written.  nnz is
+ * stored at nnz_out as soon as it is known: the arrays are complete only when the
+ * launch is, that is for whatever follows on the stream.  Values: stk_to_sparse_gather.
+ */
+#define STK_TO_SPARSE_INDEX_BLOCKS 16384
+int stk_to_sparse_index(const void* x, int64_t rows, int64_t cols, int64_t x_stride,
+                        int blocking, int elem_bytes, uint8_t* mask, int32_t* offsets,
+                        void* row_indices, void* column_indices,
+                        int32_t* offsets_t, void* column_indices_t, int32_t* block_offsets_t,
+                        int index_dtype, int32_t* nnz_out, stk_stream_t stream);
 
 /*
  * Topology of a dropless mixture-of-experts layer, built in one launch from the

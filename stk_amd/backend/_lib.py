@@ -12,7 +12,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), "libstk_amd.so")
 NATIVE_PATH = os.path.join(os.path.dirname(_HERE), "_native.so")
 
-ABI_VERSION = 17
+ABI_VERSION = 18
 STK_OK, STK_ERR_DIMS, STK_ERR_UNSUPPORTED, STK_ERR_HIP, STK_ERR_WORKSPACE = 0, 1, 2, 3, 4
 STK_F16, STK_BF16, STK_F32 = 0, 1, 2
 STK_I16, STK_I32 = 0, 1
@@ -47,6 +47,8 @@ SIGNATURES = {
     "stk_transpose_meta_workspace_bytes": (_sz, [_i64]),
     "stk_transpose_meta": (_int, [_p, _p, _i64, _i64, _int, _p, _p, _p, _p, _sz, _p]),
     "stk_to_dense": (_int, [_p, _p, _p, _i64, _int, _i64, _i64, _int, _int, _p, _p]),
+    "stk_to_dense_rows": (_int, [_p, _p, _p, _p, _i64, _int, _i64, _i64, _int, _int, _p, _p]),
+    "stk_to_sparse_index": (_int, [_p, _i64, _i64, _i64, _int, _int, _p, _p, _p, _p, _p, _p, _p, _int, _p, _p]),
     "stk_to_sparse_count": (_int, [_p, _i64, _i64, _i64, _int, _int, _p, _p, _p]),
     "stk_to_sparse_count_nnz": (_int, [_p, _i64, _i64, _i64, _int, _int, _p, _p, _p, _p]),
     "stk_to_sparse_fill": (_int, [_p, _i64, _i64, _i64, _int, _int, _p, _p, _i64, _p, _p, _p, _int, _p]),

@@ -358,12 +358,19 @@ def dmoe_topology(padded_bins, blocking, block_rows, blocks_per_row, index_dtype
     return tuple(meta)
 
 
-def to_dense(data, row_indices, column_indices, rows, cols):
-    return _lib.native().to_dense(data, row_indices, column_indices, rows, cols)
+def to_dense(data, row_indices, column_indices, rows, cols, offsets=None):
+    """offsets: where given, those of the block rows (row r's blocks are the entries offsets[r] .. offsets[r + 1] - 1)."""
+    return _lib.native().to_dense(data, row_indices, column_indices, rows, cols, offsets)
 
 
 def to_sparse(x, blocking, index_dtype=torch.int16):
     """(data, row_indices, column_indices, offsets) of the nonzero blocks of x."""
+    return to_sparse_meta(x, blocking, index_dtype)[:4]
+
+
+def to_sparse_meta(x, blocking, index_dtype=torch.int16):
+    """The results of to_sparse, then column_indices_t, offsets_t and block_offsets_t, or None for each of these three: they
+    come with the others where the matrix has few blocks."""
     return _lib.native().to_sparse(x, blocking, _INDEX_DTYPES[index_dtype] == _lib.STK_I32)
 
 

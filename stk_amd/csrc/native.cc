@@ -357,54 +357,70 @@ int elem_bytes(const Tensor& t) {
   return (int)t.element_size();
 }
 
-Tensor to_dense(const Tensor& data_, const Tensor& row_indices, const Tensor& column_indices, int64_t rows, int64_t cols) {
+Tensor to_dense(const Tensor& data_, const Tensor& row_indices, const Tensor& column_indices, int64_t rows, int64_t cols, const OptTensor& offsets) {
   need_gpu(data_);
   const c10::DeviceGuard guard(data_.device());
   const Tensor data = data_.detach().contiguous(), ri = index(row_indices), ci = index(column_indices);
   Tensor out = at::empty({rows, cols}, data.options());
-  check(stk_to_dense(ptr<void>(data), ptr<void>(ri), ptr<void>(ci), data.size(0), (int)data.size(-1), rows, cols, elem_bytes(data),
-                     index_dtype(ci.scalar_type()), ptr<void>(out), stream_of(data)));
+  const int64_t blocking = data.size(-1);
+  const bool by_rows = offsets && offsets->scalar_type() == at::kInt && offsets->is_contiguous() && offsets->device() == data.device() && blocking > 0 &&
+                       ci.numel() == data.size(0) && rows % blocking == 0 && offsets->numel() == rows / blocking + 1;
+  check(stk_to_dense_rows(ptr<void>(data), by_rows ? ptr<int32_t>(*offsets) : nullptr, ptr<void>(ri), ptr<void>(ci), data.size(0), (int)blocking, rows, cols,
+                          elem_bytes(data), index_dtype(ci.scalar_type()), ptr<void>(out), stream_of(data)));
   return out;
 }
 
 // Scratch allocations of this size or more are not left alive behind the small views returned.
 constexpr int64_t kKeepBytes = 1 << 16;
 
-// data, row_indices, column_indices and offsets of the nonzero blocks of x
-std::tuple<Tensor, Tensor, Tensor, Tensor> to_sparse(const Tensor& x_, int64_t blocking, bool int32_indices) {
+// data, row_indices, column_indices and offsets of the nonzero blocks of x, and for matrices of few blocks, where they come
+// with the rest, column_indices_t, offsets_t and block_offsets_t
+std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor, OptTensor, OptTensor> to_sparse(const Tensor& x_, int64_t blocking, bool int32_indices) {
   need_gpu(x_);
   require(x_.dim() == 2, "to_sparse takes a matrix");
   const int64_t rows = x_.size(0), cols = x_.size(1);
   require(blocking > 0 && rows % blocking == 0 && cols % blocking == 0, "the matrix must be made of whole blocks");
   const c10::DeviceGuard guard(x_.device());
   const Tensor x = (x_.stride(1) != 1 && cols > 1 ? x_.contiguous() : x_).detach();
-  const int64_t br = rows / blocking, bc = cols / blocking;
+  const int64_t br = rows / blocking, bc = cols / blocking, blocks = br * bc;
   const hipStream_t stream = stream_of(x);
   if (capture_id(reinterpret_cast<int64_t>(stream)))
     raise(PyExc_RuntimeError, "to_sparse sizes its result by the number of nonzero blocks, which the host reads back: it cannot be captured into a graph");
   const int bytes = elem_bytes(x), idx = int32_indices ? STK_I32 : STK_I16;
+  const bool small = blocks > 0 && blocks <= STK_TO_SPARSE_INDEX_BLOCKS && br <= 1024 && bc <= 1024;
   // one allocation for offsets (int32) and the block mask (bytes) behind it
-  Tensor scratch = at::empty({4 * (br + 1) + std::max<int64_t>(br * bc, 1)}, x.options().dtype(at::kByte));
+  Tensor scratch = at::empty({4 * (br + 1) + std::max<int64_t>(blocks, 1)}, x.options().dtype(at::kByte));
   Tensor offsets = scratch.narrow(0, 0, 4 * (br + 1)).view(at::kInt);
   uint8_t* mask = ptr<uint8_t>(scratch) + 4 * (br + 1);
+  // the index arrays need no nnz: launched before the host knows it, into room for every block (the first nnz entries are
+  // written; the index tensors returned are views of that room, at multiples of 256 bytes like allocations of their own)
+  const int64_t half = std::max<int64_t>((blocks + 127) / 128 * 128, 128), columns = (bc + 1 + 63) / 64 * 64;
+  Tensor room = at::empty({(small ? 3 : 2) * half}, x.options().dtype(int32_indices ? at::kInt : at::kShort)), room_t;
+  const auto third = [&](int i) { return ptr<char>(room) + i * half * room.element_size(); };
   const Mailbox box(x.device());
-  check(stk_to_sparse_count_nnz(ptr<void>(x), rows, cols, x.stride(0), (int)blocking, bytes, mask, ptr<int32_t>(offsets), const_cast<int32_t*>(box.word), stream));
-  // the coordinates need no nnz: launched behind the count, into room for every block (the first nnz entries are
-  // written; the index tensors returned are views of that room, both at multiples of 256 bytes like allocations of their own)
-  const int64_t half = std::max<int64_t>((br * bc + 127) / 128 * 128, 128);
-  Tensor room = at::empty({2 * half}, x.options().dtype(int32_indices ? at::kInt : at::kShort));
-  char* second = ptr<char>(room) + half * room.element_size();
-  check(stk_to_sparse_coordinates(rows, cols, (int)blocking, mask, ptr<int32_t>(offsets), ptr<void>(room), second, idx, stream));
+  if (small) {
+    room_t = at::empty({columns + half}, x.options().dtype(at::kInt));
+    check(stk_to_sparse_index(ptr<void>(x), rows, cols, x.stride(0), (int)blocking, bytes, mask, ptr<int32_t>(offsets), third(0), third(1),
+                              ptr<int32_t>(room_t), third(2), ptr<int32_t>(room_t) + columns, idx, const_cast<int32_t*>(box.word), stream));
+  } else {
+    check(stk_to_sparse_count_nnz(ptr<void>(x), rows, cols, x.stride(0), (int)blocking, bytes, mask, ptr<int32_t>(offsets), const_cast<int32_t*>(box.word), stream));
+    check(stk_to_sparse_coordinates(rows, cols, (int)blocking, mask, ptr<int32_t>(offsets), third(0), third(1), idx, stream));
+  }
   const int64_t nnz = box.receive(stream);
   Tensor data = at::empty({nnz, blocking, blocking}, x.options());
-  check(stk_to_sparse_gather(ptr<void>(x), rows, cols, x.stride(0), (int)blocking, bytes, ptr<void>(room), second, nnz, idx, ptr<void>(data), stream));
+  check(stk_to_sparse_gather(ptr<void>(x), rows, cols, x.stride(0), (int)blocking, bytes, third(0), third(1), nnz, idx, ptr<void>(data), stream));
   Tensor ri = room.narrow(0, 0, nnz), ci = room.narrow(0, half, nnz);
+  OptTensor ci_t, offsets_t, bo_t;
+  if (small) ci_t = room.narrow(0, 2 * half, nnz), offsets_t = room_t.narrow(0, 0, bc + 1), bo_t = room_t.narrow(0, columns, nnz);
   // A Matrix keeps these tensors for as long as it lives.  Where the room for every block is much more than the
   // nonzero blocks need (a large, very sparse matrix), they are copied out of it, and the offsets out of the
   // allocation they share with the block mask, so that the O(rows x columns / blocking^2) buffers can go.
-  if (room.numel() * room.element_size() >= kKeepBytes && 4 * nnz <= br * bc) ri = ri.clone(), ci = ci.clone();
+  if (room.numel() * room.element_size() >= kKeepBytes && 4 * nnz <= blocks) {
+    ri = ri.clone(), ci = ci.clone();
+    if (small) ci_t = ci_t->clone(), offsets_t = offsets_t->clone(), bo_t = bo_t->clone();
+  }
   if (scratch.numel() >= kKeepBytes && 16 * (br + 1) <= scratch.numel()) offsets = offsets.clone();
-  return {data, ri, ci, offsets};
+  return {data, ri, ci, offsets, ci_t, offsets_t, bo_t};
 }
 
 // ------------------------------------------------------------------------------------------------ values and routing

@@ -296,6 +296,48 @@ __global__ void block_copy_kernel(VEC_T* __restrict__ data, VEC_T* __restrict__ 
   }
 }
 
+// The whole dense matrix in one pass over it, for matrices whose rows of blocks are known by their offsets: a workgroup
+// writes kDenseRows rows of 256 pieces of one block row, having looked up which block each piece lies in (the entries of the
+// block row in LDS; out of range ones are left out).  Clearing the matrix and copying the blocks over it writes every
+// nonzero block twice and takes two launches: 8192 x 8192 in 16 bits, a quarter of the 128-blocks, 18.8 + 10.7 us against
+// 24.5 (6.8 TB/s of stores and loads).  Memory bounds it.
+constexpr int kDenseRows = 16;
+template <typename VEC_T, typename IDX>
+__global__ __launch_bounds__(256) void dense_rows_kernel(const VEC_T* __restrict__ data, VEC_T* __restrict__ dense,
+                                                         const int32_t* __restrict__ offsets, const IDX* __restrict__ column_indices, int nnz,
+                                                         int b, int b_vec, int ld_vec) {
+  __shared__ int block_of[256 + 1];
+  const int tid = threadIdx.x;
+  const int across = (ld_vec + 255) / 256, down = (b + kDenseRows - 1) / kDenseRows;
+  const int j0 = (int)(blockIdx.x % across) * 256, rest = (int)(blockIdx.x / across);
+  const int i0 = rest % down * kDenseRows, r = rest / down;
+  const int last = j0 + 255 < ld_vec ? j0 + 255 : ld_vec - 1;
+  const int c0 = j0 / b_vec, columns = last / b_vec - c0 + 1;
+  for (int c = tid; c < columns; c += 256) block_of[c] = -1;
+  const int begin = offsets[r] > 0 ? offsets[r] : 0, end = offsets[r + 1] < nnz ? offsets[r + 1] : nnz;
+  __syncthreads();
+  for (int e = begin + tid; e < end; e += 256) {
+    const int c = (int)column_indices[e] - c0;
+    if (c >= 0 && c < columns) block_of[c] = e;
+  }
+  __syncthreads();
+  const int j = j0 + tid;
+  if (j > last) return;
+  const int c = j / b_vec, p = block_of[c - c0];
+  const int rows = b - i0 < kDenseRows ? b - i0 : kDenseRows;
+  const VEC_T* src = data + ((int64_t)p * b + i0) * b_vec + (j - c * b_vec);
+  VEC_T* dst = dense + ((int64_t)r * b + i0) * ld_vec + j;
+  VEC_T v[kDenseRows];
+#pragma unroll
+  for (int i = 0; i < kDenseRows; i++) {
+    v[i] = VEC_T{};
+    if (p >= 0 && i < rows) v[i] = src[(int64_t)i * b_vec];
+  }
+#pragma unroll
+  for (int i = 0; i < kDenseRows; i++)
+    if (i < rows) dst[(int64_t)i * ld_vec] = v[i];
+}
+
 template <bool TO_DENSE>
 static int block_copy(void* data, void* dense, const void* rows, const void* cols, int64_t nnz, int b, int64_t ld,
                       int elem_bytes, int idx32, hipStream_t s) {
@@ -380,6 +422,120 @@ __global__ __launch_bounds__(256) void block_mask_vec_kernel(const char* __restr
       for (int i0 = 4 * rows_per_load; i0 < b; i0 += 8 * rows_per_load) read(i0, 8);
     const uint64_t bal = __ballot(any != 0);
     if (lane == 0) mask[blk] = bal != 0;
+  }
+}
+
+// The same for blocks of at least sixteen such loads (b a multiple of four times the rows of a load): a workgroup per
+// block, its wavefronts every fourth load each.  Every one goes by its own first load - a quarter of the first rows is enough to
+// tell for almost every nonzero block - and has the rest of its part in flight at once; a single wavefront per block
+// waits for memory five times in a row.  8192 x 8192 in 16 bits, a quarter of the 128-blocks nonzero: 27.2 -> 18.4 us.
+template <int ELEM_BYTES>
+__global__ __launch_bounds__(256) void block_mask_wide_kernel(const char* __restrict__ x, int64_t ld_bytes, int b, int log2_pieces,
+                                                              int block_cols, int64_t blocks, uint8_t* __restrict__ mask) {
+  __shared__ int found[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr uint32_t kAbs = ELEM_BYTES == 2 ? 0x7fff7fffu : 0x7fffffffu;   // everything but the sign bits
+  const int rows_per_load = 64 >> log2_pieces;
+  const int64_t first = (int64_t)(wave * rows_per_load + (lane >> log2_pieces)) * ld_bytes + (int64_t)(lane & ((1 << log2_pieces) - 1)) * 16;
+  const int64_t step = (int64_t)4 * rows_per_load * ld_bytes;
+  const int loads = b / rows_per_load / 4;   // of a wavefront
+  for (int64_t blk = blockIdx.x; blk < blocks; blk += gridDim.x) {
+    const int64_t r = blk / block_cols, c = blk - r * block_cols;
+    const char* base = x + r * b * ld_bytes + c * (int64_t)b * ELEM_BYTES + first;
+    auto bits = [&](const uint4& v) { return (v.x | v.y | v.z | v.w) & kAbs; };
+    uint32_t any = bits(*reinterpret_cast<const uint4*>(base));
+    if (__ballot(any != 0) == 0)
+      for (int u0 = 1; u0 < loads; u0 += 8) {
+        uint4 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          v[u] = make_uint4(0u, 0u, 0u, 0u);
+          if (u0 + u < loads) v[u] = *reinterpret_cast<const uint4*>(base + (u0 + u) * step);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) any |= bits(v[u]);
+      }
+    const uint64_t bal = __ballot(any != 0);
+    if (lane == 0) found[wave] = bal != 0;
+    __syncthreads();
+    if (threadIdx.x == 0) mask[blk] = (found[0] | found[1] | found[2] | found[3]) != 0;
+    __syncthreads();
+  }
+}
+
+// Everything that follows from the mask of a small matrix, in one launch of one workgroup: offsets and their total, the
+// coordinates of the nonzero blocks and the transpose metadata (block columns ascending, ascending block id inside one).
+// The mask is kept as bits, by rows and by columns, so that a block's place in either order is an offset plus a count of bits.
+// The host waits for the total, which is delivered first, and the rest runs while it prepares the next launch; as three
+// launches (offsets, coordinates, and the sort of the pairs once their number was known) these took 4.6 + 4.0 + 5.2 us, the
+// last of them behind the copy of the values; this kernel takes 7.2 us, hidden behind the host's.  Latency bounds it.
+constexpr int kIndexLines = 1024;                       // block rows and block columns, a thread each
+constexpr int kIndexBlocks = STK_TO_SPARSE_INDEX_BLOCKS;
+constexpr int kIndexWords = kIndexBlocks / 64 + kIndexLines;   // lines x words of a line, rounded up line by line
+template <typename IDX>
+__global__ __launch_bounds__(1024) void mask_index_kernel(const uint8_t* __restrict__ mask, int block_rows, int block_cols,
+                                                          int32_t* __restrict__ offsets, IDX* __restrict__ row_indices,
+                                                          IDX* __restrict__ column_indices, int32_t* __restrict__ offsets_t,
+                                                          IDX* __restrict__ column_indices_t, int32_t* __restrict__ block_offsets_t,
+                                                          int32_t* total_out) {
+  __shared__ uint64_t row_bits[kIndexWords], col_bits[kIndexWords];   // [row][words of a row], [column][words of a column]
+  __shared__ int first[kIndexLines], first_t[kIndexLines];
+  __shared__ int part[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wr = (block_cols + 63) / 64, wc = (block_rows + 63) / 64, words = block_rows * wr;
+  for (int q0 = wave; q0 < words; q0 += 64) {   // four words, 16 apart, in flight
+    bool nz[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int q = q0 + 16 * u, c = q % wr * 64 + lane;
+      nz[u] = q < words && c < block_cols && mask[q / wr * block_cols + c];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const uint64_t bal = __ballot(nz[u]);
+      if (lane == 0 && q0 + 16 * u < words) row_bits[q0 + 16 * u] = bal;
+    }
+  }
+  __syncthreads();
+  int count = 0, total;
+  if (tid < block_rows)
+    for (int j = 0; j < wr; j++) count += __popcll(row_bits[tid * wr + j]);
+  const int before = block_exclusive_scan(count, part, &total);
+  // (may be pinned host memory that the host polls: a system-scope store, made visible at once)
+  if (total_out && tid == 0) __hip_atomic_store(total_out, total, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (tid == 0) offsets[0] = 0, offsets_t[0] = 0;
+  if (tid < block_rows) offsets[tid + 1] = before + count, first[tid] = before;
+  // 64 x 64 bits at a time: lane i holds the word of row i, then the word of column i
+  for (int q = wave; q < wr * wc; q += 16) {
+    const int j = q % wr, i = q / wr, r = 64 * i + lane;
+    const uint64_t word = r < block_rows ? row_bits[r * wr + j] : 0;
+    uint64_t column = 0;
+    for (int c = 0; c < 64; c++) {
+      const uint64_t bal = __ballot((word >> c) & 1);
+      if (lane == c) column = bal;
+    }
+    if (64 * j + lane < block_cols) col_bits[(64 * j + lane) * wc + i] = column;
+  }
+  __syncthreads();
+  count = 0;
+  if (tid < block_cols)
+    for (int i = 0; i < wc; i++) count += __popcll(col_bits[tid * wc + i]);
+  const int before_t = block_exclusive_scan(count, part, &total);
+  if (tid < block_cols) offsets_t[tid + 1] = before_t + count, first_t[tid] = before_t;
+  __syncthreads();
+  for (int q = wave; q < words; q += 16) {
+    const int r = q / wr, j = q % wr, c = 64 * j + lane;
+    const uint64_t word = row_bits[q];
+    if (!((word >> lane) & 1)) continue;
+    int p = first[r] + __popcll(word & lanes_below(lane));
+    for (int i = 0; i < j; i++) p += __popcll(row_bits[r * wr + i]);
+    const uint64_t* column = col_bits + c * wc;
+    int t = first_t[c] + __popcll(column[r / 64] & lanes_below(r % 64));
+    for (int i = 0; i < r / 64; i++) t += __popcll(column[i]);
+    row_indices[p] = static_cast<IDX>(r);
+    column_indices[p] = static_cast<IDX>(c);
+    column_indices_t[t] = static_cast<IDX>(r);
+    block_offsets_t[t] = p;
   }
 }
 
@@ -514,19 +670,41 @@ extern "C" int stk_to_dense(const void* data, const void* row_indices, const voi
                           index_dtype == STK_I32, s);
 }
 
+extern "C" int stk_to_dense_rows(const void* data, const int32_t* offsets, const void* row_indices, const void* column_indices, int64_t nnz,
+                                 int blocking, int64_t rows, int64_t cols, int elem_bytes, int index_dtype, void* out, stk_stream_t stream) {
+  const int b = blocking;
+  const int64_t bytes = rows * cols * elem_bytes, ld_vec = cols * elem_bytes / 16;
+  // 16-byte pieces that lie in one block each; everything else, and what is refused, as without the offsets
+  if (b > 0 && bytes > 0 && rows % b == 0 && cols % b == 0 && nnz >= 0 && nnz <= INT32_MAX && (elem_bytes == 2 || elem_bytes == 4) &&
+      (index_dtype == STK_I16 || index_dtype == STK_I32) && (b * elem_bytes) % 16 == 0 && offsets && out && aligned16(out) && aligned16(data) &&
+      (nnz == 0 || (data && column_indices)) && ld_vec <= INT32_MAX) {
+    const int64_t groups = (rows / b) * ((b + kDenseRows - 1) / kDenseRows) * ((ld_vec + 255) / 256);
+    if (groups <= INT32_MAX) {
+      hipStream_t s = static_cast<hipStream_t>(stream);
+      if (index_dtype == STK_I32)
+        hipLaunchKernelGGL((dense_rows_kernel<uint4, int32_t>), dim3((unsigned)groups), dim3(256), 0, s, static_cast<const uint4*>(data),
+                           static_cast<uint4*>(out), offsets, static_cast<const int32_t*>(column_indices), (int)nnz, b, b * elem_bytes / 16, (int)ld_vec);
+      else
+        hipLaunchKernelGGL((dense_rows_kernel<uint4, int16_t>), dim3((unsigned)groups), dim3(256), 0, s, static_cast<const uint4*>(data),
+                           static_cast<uint4*>(out), offsets, static_cast<const int16_t*>(column_indices), (int)nnz, b, b * elem_bytes / 16, (int)ld_vec);
+      return check_launch("stk_to_dense");
+    }
+  }
+  return stk_to_dense(data, row_indices, column_indices, nnz, blocking, rows, cols, elem_bytes, index_dtype, out, stream);
+}
+
 extern "C" int stk_to_sparse_count(const void* x, int64_t rows, int64_t cols, int64_t x_stride, int blocking, int elem_bytes,
                                    uint8_t* mask, int32_t* offsets, stk_stream_t stream) {
   return stk_to_sparse_count_nnz(x, rows, cols, x_stride, blocking, elem_bytes, mask, offsets, nullptr, stream);
 }
 
-extern "C" int stk_to_sparse_count_nnz(const void* x, int64_t rows, int64_t cols, int64_t x_stride, int blocking, int elem_bytes,
-                                       uint8_t* mask, int32_t* offsets, int32_t* nnz_out, stk_stream_t stream) {
+// The mask of the nonzero blocks.
+static int launch_mask(const void* x, int64_t rows, int64_t cols, int64_t x_stride, int blocking, int elem_bytes, uint8_t* mask, hipStream_t s) {
   if (elem_bytes != 2 && elem_bytes != 4) return fail(STK_ERR_UNSUPPORTED, "stk_to_sparse_count: element size %d", elem_bytes);
   if (blocking <= 0 || rows < 0 || cols < 0 || rows % blocking || cols % blocking)
     return fail(STK_ERR_DIMS, "stk_to_sparse_count: [%lld, %lld] is not divisible by blocking %d", (long long)rows, (long long)cols, blocking);
   const int64_t br = rows / blocking, bc = cols / blocking;
   if (br > INT32_MAX || bc > INT32_MAX || (int64_t)blocking * blocking > INT32_MAX) return fail(STK_ERR_UNSUPPORTED, "stk_to_sparse_count: size exceeds 32-bit range");
-  hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t blocks = br * bc;
   // 16-byte loads when a block row is a power-of-two number (up to 64) of aligned 16-byte pieces
   const int64_t row_bytes = (int64_t)blocking * elem_bytes;
@@ -534,7 +712,15 @@ extern "C" int stk_to_sparse_count_nnz(const void* x, int64_t rows, int64_t cols
   if (row_bytes % 16 == 0 && (x_stride * elem_bytes) % 16 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0)
     for (int l = 0; l <= 6; l++)
       if (row_bytes == (16 << l)) log2_pieces = l;
-  if (blocks > 0 && log2_pieces >= 0) {
+  if (blocks > 0 && log2_pieces >= 0 && blocking % (4 * (64 >> log2_pieces)) == 0 && blocking / (64 >> log2_pieces) >= 16) {
+    const int grid = (int)(blocks < 262144 ? blocks : 262144);
+    if (elem_bytes == 2)
+      hipLaunchKernelGGL((block_mask_wide_kernel<2>), dim3(grid), dim3(256), 0, s, static_cast<const char*>(x), x_stride * elem_bytes, blocking,
+                         log2_pieces, (int)bc, blocks, mask);
+    else
+      hipLaunchKernelGGL((block_mask_wide_kernel<4>), dim3(grid), dim3(256), 0, s, static_cast<const char*>(x), x_stride * elem_bytes, blocking,
+                         log2_pieces, (int)bc, blocks, mask);
+  } else if (blocks > 0 && log2_pieces >= 0) {
     const int grid = (int)((blocks + 3) / 4 < 262144 ? (blocks + 3) / 4 : 262144);
     if (elem_bytes == 2)
       hipLaunchKernelGGL((block_mask_vec_kernel<2>), dim3(grid), dim3(256), 0, s, static_cast<const char*>(x), x_stride * elem_bytes, blocking,
@@ -549,8 +735,39 @@ extern "C" int stk_to_sparse_count_nnz(const void* x, int64_t rows, int64_t cols
     else
       hipLaunchKernelGGL((block_mask_kernel<uint32_t>), dim3(grid), dim3(256), 0, s, static_cast<const uint32_t*>(x), x_stride, blocking, (int)bc, blocks, mask);
   }
-  hipLaunchKernelGGL(row_offsets_kernel, dim3(1), dim3(1024), 0, s, mask, (int)br, (int)bc, offsets, nnz_out);
   return check_launch("stk_to_sparse_count");
+}
+
+extern "C" int stk_to_sparse_count_nnz(const void* x, int64_t rows, int64_t cols, int64_t x_stride, int blocking, int elem_bytes,
+                                       uint8_t* mask, int32_t* offsets, int32_t* nnz_out, stk_stream_t stream) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rc = launch_mask(x, rows, cols, x_stride, blocking, elem_bytes, mask, s);
+  if (rc != STK_OK) return rc;
+  hipLaunchKernelGGL(row_offsets_kernel, dim3(1), dim3(1024), 0, s, mask, (int)(rows / blocking), (int)(cols / blocking), offsets, nnz_out);
+  return check_launch("stk_to_sparse_count");
+}
+
+extern "C" int stk_to_sparse_index(const void* x, int64_t rows, int64_t cols, int64_t x_stride, int blocking, int elem_bytes, uint8_t* mask,
+                                   int32_t* offsets, void* row_indices, void* column_indices, int32_t* offsets_t, void* column_indices_t,
+                                   int32_t* block_offsets_t, int index_dtype, int32_t* nnz_out, stk_stream_t stream) {
+  const char* who = "stk_to_sparse_index";
+  if (index_dtype != STK_I16 && index_dtype != STK_I32) return fail(STK_ERR_UNSUPPORTED, "%s: index dtype %d", who, index_dtype);
+  if (blocking > 0 && (rows / blocking > kIndexLines || cols / blocking > kIndexLines || (rows / blocking) * (cols / blocking) > kIndexBlocks))
+    return fail(STK_ERR_UNSUPPORTED, "%s: %lld x %lld blocks (at most %d in all and %d in a line)", who, (long long)(rows / blocking),
+                (long long)(cols / blocking), kIndexBlocks, kIndexLines);
+  if (!offsets || !offsets_t || (rows > 0 && cols > 0 && (!x || !mask || !row_indices || !column_indices || !column_indices_t || !block_offsets_t)))
+    return fail(STK_ERR_DIMS, "%s: missing pointer", who);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rc = launch_mask(x, rows, cols, x_stride, blocking, elem_bytes, mask, s);
+  if (rc != STK_OK) return rc;
+  const int br = (int)(rows / blocking), bc = (int)(cols / blocking);
+  if (index_dtype == STK_I32)
+    hipLaunchKernelGGL((mask_index_kernel<int32_t>), dim3(1), dim3(1024), 0, s, mask, br, bc, offsets, static_cast<int32_t*>(row_indices),
+                       static_cast<int32_t*>(column_indices), offsets_t, static_cast<int32_t*>(column_indices_t), block_offsets_t, nnz_out);
+  else
+    hipLaunchKernelGGL((mask_index_kernel<int16_t>), dim3(1), dim3(1024), 0, s, mask, br, bc, offsets, static_cast<int16_t*>(row_indices),
+                       static_cast<int16_t*>(column_indices), offsets_t, static_cast<int16_t*>(column_indices_t), block_offsets_t, nnz_out);
+  return check_launch(who);
 }
 
 extern "C" int stk_to_sparse_coordinates(int64_t rows, int64_t cols, int blocking, const uint8_t* mask, const int32_t* offsets,

@@ -20,8 +20,11 @@ def row_indices(shape, data, offsets, column_indices):
 def to_dense(x):
     assert isinstance(x, Matrix)
     rows, cols = int(np.prod(x.shape[:-1])), x.shape[-1]
-    impl = hip_kernels if x.is_cuda else host_format
-    return impl.to_dense(x.data, x.row_indices, x.column_indices, rows, cols).reshape(x.size())
+    if x.is_cuda:
+        dense = hip_kernels.to_dense(x.data, x.row_indices, x.column_indices, rows, cols, x.offsets if x.is_contiguous() else None)
+    else:
+        dense = host_format.to_dense(x.data, x.row_indices, x.column_indices, rows, cols)
+    return dense.reshape(x.size())
 
 
 @torch.no_grad()
@@ -29,9 +32,9 @@ def to_sparse(x, blocking=1):
     assert x.dim() == 2
     assert x.size()[0] % blocking == 0
     assert x.size()[1] % blocking == 0
-    impl = hip_kernels if x.is_cuda else host_format
-    data, rows, cols, offsets = impl.to_sparse(x, blocking)
-    return Matrix(x.size(), data, rows, cols, offsets)
+    if x.is_cuda:
+        return Matrix(x.size(), *hip_kernels.to_sparse_meta(x, blocking))
+    return Matrix(x.size(), *host_format.to_sparse(x, blocking))
 
 
 @torch.no_grad()

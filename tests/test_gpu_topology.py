@@ -458,3 +458,43 @@ def test_to_sparse_of_a_large_sparse_matrix_keeps_only_what_it_uses():
     data, topo = O.to_sparse(x.cpu().numpy(), 8)
     U.assert_topology_equal(m, topo, "large sparse")
     assert torch.equal(stk.ops.to_dense(m), x)
+
+
+# rows, columns in blocks, blocking, dtype, share of nonzero blocks, int32 indices: one block; lines of 64 blocks and one more or
+# less (a word of the bit sets); 1024 blocks a line in either direction and as many blocks as the one-launch path takes; one
+# block more than that, one line more; no nonzero block and all of them; rows of a block that are 16-byte pieces or not; the
+# wide mask kernel (128-blocks), and blocks below it
+_CONVERSIONS = [(1, 1, 128, torch.float16, 1.0, False), (64, 64, 32, torch.bfloat16, 0.25, False), (65, 63, 16, torch.float32, 0.5, False),
+                (16, 1024, 8, torch.float16, 0.3, False), (1024, 16, 8, torch.float16, 0.3, True), (128, 128, 8, torch.float16, 0.1, False),
+                (3, 5000, 2, torch.float16, 0.5, False), (1025, 3, 4, torch.float32, 0.5, False), (145, 113, 4, torch.float16, 0.5, False),
+                (7, 9, 128, torch.float32, 0.4, True), (12, 10, 128, torch.bfloat16, 0.0, False), (5, 6, 64, torch.float32, 1.0, False),
+                (9, 11, 24, torch.float16, 0.6, False), (4, 3, 256, torch.float16, 0.5, False)]
+
+
+@pytest.mark.parametrize("br,bc,b,dtype,share,int32", _CONVERSIONS)
+def test_conversions_by_every_path(br, bc, b, dtype, share, int32):
+    gen = torch.Generator().manual_seed(br * bc + b)
+    keep = torch.rand(br, bc, generator=gen) < share
+    x = torch.zeros(br, b, bc, b)
+    # one element of every kept block, anywhere in it
+    r, c = keep.nonzero(as_tuple=True)
+    at = torch.randint(0, b, (2, r.numel()), generator=gen)
+    x[r, at[0], c, at[1]] = 1.5
+    x = x.reshape(br * b, bc * b).to(dtype).to(DEV)
+    index_dtype = torch.int32 if int32 else torch.int16
+    data, ri, ci, offsets, cit, ot, bot = hip_kernels.to_sparse_meta(x, b, index_dtype)
+    with_transpose = br * bc <= 16384 and br <= 1024 and bc <= 1024
+    assert (cit is not None) == (ot is not None) == (bot is not None) == with_transpose
+    m = stk.Matrix(x.size(), data, ri, ci, offsets, cit, ot, bot)
+    assert ri.dtype == ci.dtype == m.column_indices_t.dtype == index_dtype
+    assert torch.equal(ri.cpu().long(), r) and torch.equal(ci.cpu().long(), c)
+    assert offsets.tolist() == [0] + keep.sum(1).cumsum(0).tolist()
+    rt, ct = keep.t().nonzero(as_tuple=True)[1], torch.arange(r.numel())[torch.sort(c, stable=True).indices]
+    assert m.offsets_t.tolist() == [0] + keep.sum(0).cumsum(0).tolist()
+    assert torch.equal(m.column_indices_t.cpu().long(), rt) and torch.equal(m.block_offsets_t.cpu().long(), ct)
+    # back: with the offsets, without them, and with the entries of every row in another order
+    assert torch.equal(stk.ops.to_dense(m), x)
+    assert torch.equal(hip_kernels.to_dense(data, ri, ci, *x.shape), x)
+    if r.numel():
+        back = torch.cat([torch.arange(a, e).flip(0) for a, e in zip(offsets.tolist()[:-1], offsets.tolist()[1:])]).to(DEV)
+        assert torch.equal(stk.ops.to_dense(stk.Matrix(x.size(), data[back], ri[back], ci[back], offsets)), x)
