@@ -15,6 +15,7 @@ a transpose flag instead of a view; the kernels then walk the CSC metadata.
 import functools
 
 import torch
+from torch.autograd import forward_ad
 
 from stk_amd.backend import hip_kernels as backend
 from stk_amd.backend.autocast import custom_bwd, custom_fwd
@@ -117,6 +118,12 @@ def _both(first, second, sp, width):
 
 def _wants_grad(*tensors):
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
+def applies(*tensors):
+    """Whether a function of this kind has to be applied, and not just its forward pass run.  Forward-mode differentiation
+    and functorch's transforms see, and refuse, an applied function only."""
+    return _wants_grad(*tensors) or forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
 
 
 class DSD(torch.autograd.Function):
@@ -345,23 +352,23 @@ class RowIndices(torch.autograd.Function):
 # The functions that stk.ops calls.  When nothing needs a gradient the forward pass runs by itself: the bookkeeping of
 # an autograd function costs as much host time as the launch.
 def dsd(shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_a, rhs):
-    run = DSD.apply if _wants_grad(data, rhs) else functools.partial(DSD.forward, None)
+    run = DSD.apply if applies(data, rhs) else functools.partial(DSD.forward, None)
     return run(shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_a, rhs)
 
 
 def dds(lhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_b):
-    run = DDS.apply if _wants_grad(data, lhs) else functools.partial(DDS.forward, None)
+    run = DDS.apply if applies(data, lhs) else functools.partial(DDS.forward, None)
     return run(lhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_b)
 
 
 def sdd(lhs, rhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t):
-    run = SDD.apply if _wants_grad(lhs, rhs) else functools.partial(SDD.forward, None)
+    run = SDD.apply if applies(lhs, rhs) else functools.partial(SDD.forward, None)
     return run(lhs, rhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t)
 
 
 def sdd_fused(lhs, rhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, activation, multiplier,
               save_sums=False):
-    run = SDDFused.apply if _wants_grad(lhs, rhs, multiplier) else functools.partial(SDDFused.forward, None)
+    run = SDDFused.apply if applies(lhs, rhs, multiplier) else functools.partial(SDDFused.forward, None)
     return run(lhs, rhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, activation, multiplier,
                save_sums)
 

@@ -9,6 +9,7 @@ from collections import namedtuple
 import torch
 
 from stk_amd.backend import hip_kernels
+from stk_amd.backend.autograd import applies
 from stk_amd.matrix import Matrix
 
 Route = namedtuple("Route", "indices bin_ids bins padded_bins slot_rows row_slots top_k blocking")
@@ -70,7 +71,7 @@ class _PaddedScatter(torch.autograd.Function):
 def padded_gather(x, route):
     """x [tokens, hidden] -> [padded_rows, hidden]: every slot's token row at its place in the padded
     layout, zeros in the padding rows."""
-    if not _wants_grad(x):
+    if not applies(x):
         return hip_kernels.padded_gather(x, route.row_slots, route.top_k)
     return _PaddedGather.apply(x, route)
 
@@ -78,7 +79,7 @@ def padded_gather(x, route):
 def padded_scatter(x, route, weights=None):
     """x [padded_rows, hidden] -> [tokens, hidden]: each token's top_k rows, multiplied by
     weights [tokens, top_k] (or [tokens * top_k]) when given, added up in fp32 in the order of the choices."""
-    if not _wants_grad(x, weights):
+    if not applies(x, weights):
         return hip_kernels.padded_scatter(x, route.slot_rows, route.top_k, weights)
     return _PaddedScatter.apply(x, route, weights)
 

@@ -259,6 +259,31 @@ def test_host_products_keep_the_error_contract():
     assert rc == 1 and b"outside the matrix" in lib.stk_cpu_last_error()
 
 
+@pytest.mark.parametrize("dual", ["dense", "values"])
+def test_products_refuse_forward_mode_differentiation(dual):
+    """None of the products has a jvp: with a tangent on an operand, and no gradient wanted, they raise and do not drop it."""
+    from torch.autograd import forward_ad
+    s = stk.ops.to_sparse(torch.ones(64, 64), 32)
+    x = torch.ones(64, 64)
+    with torch.no_grad(), forward_ad.dual_level():
+        if dual == "dense":
+            x = forward_ad.make_dual(x, torch.ones_like(x))
+            calls = [lambda: stk.ops.dsd(s, x), lambda: stk.ops.dds(x, s), lambda: stk.ops.sdd(x, x, s)]
+        else:
+            s = stk.Matrix(s.size(), forward_ad.make_dual(s.data, torch.ones_like(s.data)), s.row_indices, s.column_indices, s.offsets)
+            calls = [lambda: stk.ops.dsd(s, x), lambda: stk.ops.dds(x, s)]
+        for call in calls:
+            with pytest.raises(NotImplementedError, match="jvp"):
+                call()
+
+
+def test_products_refuse_functorch_transforms():
+    s, x = stk.ops.to_sparse(torch.ones(64, 64), 32), torch.ones(2, 64, 64)
+    for call in (lambda d: stk.ops.dsd(s, d), lambda d: stk.ops.dds(d, s), lambda d: stk.ops.sdd(d, d, s).data):
+        with pytest.raises(RuntimeError, match="functorch"):
+            torch.vmap(call)(x)
+
+
 def test_products_never_mix_host_and_device_tensors():
     # the dispatch is by where the output lives; a device tensor among host operands is an error, not a copy
     class Fake:
