@@ -122,8 +122,10 @@ def _wants_grad(*tensors):
 
 def applies(*tensors):
     """Whether a function of this kind has to be applied, and not just its forward pass run.  Forward-mode differentiation
-    and functorch's transforms see, and refuse, an applied function only."""
-    return _wants_grad(*tensors) or forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
+    and functorch's transforms see, and refuse, an applied function only; torch.jit.trace records one as one step, where
+    the forward pass by itself leaves it the allocation of the result and nothing that fills it."""
+    return (_wants_grad(*tensors) or forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
+            or torch._C._is_tracing())
 
 
 class DSD(torch.autograd.Function):

@@ -284,6 +284,17 @@ def test_products_refuse_functorch_transforms():
             torch.vmap(call)(x)
 
 
+@pytest.mark.parametrize("product", ["dsd", "dds", "sdd"])
+def test_a_traced_product_computes_its_result(product):
+    """torch.jit.trace, with no gradient wanted: the graph holds the product, for other inputs than the traced ones too."""
+    g = torch.Generator().manual_seed(7)
+    s = stk.ops.to_sparse(torch.randn(128, 128, generator=g), 32)
+    call = {"dsd": lambda x: stk.ops.dsd(s, x), "dds": lambda x: stk.ops.dds(x.t(), s), "sdd": lambda x: stk.ops.sdd(x, x.t(), s).data}[product]
+    x, y = torch.randn(128, 64, generator=g), torch.randn(128, 64, generator=g)
+    traced = torch.jit.trace(call, (x,), check_trace=False)
+    assert torch.equal(traced(x), call(x)) and torch.equal(traced(y), call(y))
+
+
 def test_products_never_mix_host_and_device_tensors():
     # the dispatch is by where the output lives; a device tensor among host operands is an error, not a copy
     class Fake:
