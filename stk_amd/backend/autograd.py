@@ -44,25 +44,35 @@ class _Sparse:
         return (self.shape[1], self.shape[0]) if transposed else self.shape
 
 
-def _run_dsd(sp, data, transposed, rhs, stream=-1):
+def _launch(side, product, *args, **kwargs):
+    """product(*args) with the stream `side` (None: as it is) as torch's current one: whatever the call does - copies of
+    operands, its plan and workspace, the launch - then happens on that stream."""
+    if side is None:
+        product(*args, **kwargs)
+    else:
+        with torch.cuda.stream(side):
+            product(*args, **kwargs)
+
+
+def _run_dsd(sp, data, transposed, rhs, side=None):
     shape = sp.logical_shape(transposed)
     out = torch.empty((shape[0], rhs.size(1)), dtype=rhs.dtype, device=rhs.device)
-    backend.dsd(shape, data, *sp.meta, transposed, rhs, out, stream)
+    _launch(side, backend.dsd, shape, data, *sp.meta, transposed, rhs, out)
     return out
 
 
-def _run_dds(lhs, sp, data, transposed, stream=-1):
+def _run_dds(lhs, sp, data, transposed, side=None):
     shape = sp.logical_shape(transposed)
     out = torch.empty((lhs.size(0), shape[1]), dtype=lhs.dtype, device=lhs.device)
-    backend.dds(lhs, shape, data, *sp.meta, transposed, out, stream)
+    _launch(side, backend.dds, lhs, shape, data, *sp.meta, transposed, out)
     return out
 
 
-def _run_sdd(lhs, rhs, sp, stream=-1):
+def _run_sdd(lhs, rhs, sp, side=None):
     out = torch.empty(sp.data.shape, dtype=lhs.dtype, device=lhs.device)
     offsets, row_indices, column_indices, _, _, block_offsets_t = sp.meta
     # visiting blocks column by column keeps the rhs panel of a block column in cache
-    backend.sdd(lhs, rhs, sp.shape, out, offsets, row_indices, column_indices, block_order=block_offsets_t, stream=stream)
+    _launch(side, backend.sdd, lhs, rhs, sp.shape, out, offsets, row_indices, column_indices, block_order=block_offsets_t)
     return out
 
 
@@ -89,30 +99,30 @@ def _side_stream(device):
     stream = _side_streams.get(device.index)
     if stream is None:
         stream = _side_streams[device.index] = torch.cuda.Stream(device=device)
-        backend.CONCURRENT_STREAMS[stream.cuda_stream] = stream   # its dsd launches get a workspace of their own
+        backend.CONCURRENT_STREAMS.add(stream.cuda_stream)   # its dsd launches get a workspace of their own
     return stream
 
 
 def _both(first, second, sp, width):
-    """first(stream) and second(stream) -> their results (None for a callable that is None), launched side by side when
-    both are wanted.  Each callable launches one product, of sp's values with `width` columns or rows, on the stream with the
-    given handle (-1: the current one) and returns its freshly allocated output."""
+    """first(side) and second(side) -> their results (None for a callable that is None), launched side by side when
+    both are wanted.  Each callable launches one product, of sp's values with `width` columns or rows, on the given stream
+    (None: the current one) and returns its output, which it allocates on the current one."""
     if first is None or second is None:
-        return (first(-1) if first is not None else None), (second(-1) if second is not None else None)
+        return (first(None) if first is not None else None), (second(None) if second is not None else None)
     data = sp.data
     if not OVERLAP_GRADIENTS or not data.is_cuda or 2.0 * data.numel() * width < OVERLAP_FROM:
-        return first(-1), second(-1)
+        return first(None), second(None)
     offsets, _, column_indices, offsets_t, column_indices_t, _ = sp.meta
     backend.prepare_plan(data, offsets, column_indices, offsets_t, column_indices_t)   # built, if at all, in front of both
     follow = backend.follow_stream
-    main, side = backend._stream(data.device), _side_stream(data.device).cuda_stream
-    follow(side, main)              # the operands are ready on the main stream
+    main, side = backend._stream(data.device), _side_stream(data.device)
+    follow(side.cuda_stream, main)              # the operands are ready on the main stream
     try:
         # (both outputs come from the main stream's memory; the side stream's use of it lies between the two waits)
         b = second(side)
-        a = first(-1)
+        a = first(None)
     finally:
-        follow(main, side)          # whatever follows on the main stream sees both results
+        follow(main, side.cuda_stream)          # whatever follows on the main stream sees both results
     return a, b
 
 
@@ -165,12 +175,12 @@ class DSD(torch.autograd.Function):
             return None, ddata, None, None, None, None, None, None, None, drhs
         if ctx.needs_input_grad[1]:
             # d op(S) = dy rhs^T on the pattern; for a transposed S the stored blocks hold (rhs dy^T)
-            want_data = (lambda stream: _run_sdd(rhs, dy.t(), sp, stream)) if ta else (lambda stream: _run_sdd(dy, rhs.t(), sp, stream))
+            want_data = (lambda side: _run_sdd(rhs, dy.t(), sp, side)) if ta else (lambda side: _run_sdd(dy, rhs.t(), sp, side))
         if ctx.needs_input_grad[9]:
             if rhs_is_view:
-                want_rhs = lambda stream: _run_dds(dy.t(), sp, data, ta, stream)       # dy^T op(S), returned transposed
+                want_rhs = lambda side: _run_dds(dy.t(), sp, data, ta, side)       # dy^T op(S), returned transposed
             else:
-                want_rhs = lambda stream: _run_dsd(sp, data, not ta, dy, stream)       # op(S)^T dy
+                want_rhs = lambda side: _run_dsd(sp, data, not ta, dy, side)       # op(S)^T dy
         ddata, drhs = _both(want_data, want_rhs, sp, dy.size(1))
         if drhs is not None and rhs_is_view:
             drhs = drhs.t()
@@ -204,12 +214,12 @@ class DDS(torch.autograd.Function):
         lhs_is_view = _is_transposed_view(lhs)
         if ctx.needs_input_grad[0]:
             if lhs_is_view:
-                want_lhs = lambda stream: _run_dsd(sp, data, tb, dy.t(), stream)       # op(S) dy^T, returned transposed
+                want_lhs = lambda side: _run_dsd(sp, data, tb, dy.t(), side)       # op(S) dy^T, returned transposed
             else:
-                want_lhs = lambda stream: _run_dds(dy, sp, data, not tb, stream)       # dy op(S)^T
+                want_lhs = lambda side: _run_dds(dy, sp, data, not tb, side)       # dy op(S)^T
         if ctx.needs_input_grad[2]:
             # d op(S) = lhs^T dy on the pattern; for a transposed S the stored blocks hold (dy^T lhs)
-            want_data = (lambda stream: _run_sdd(dy.t(), lhs, sp, stream)) if tb else (lambda stream: _run_sdd(lhs.t(), dy, sp, stream))
+            want_data = (lambda side: _run_sdd(dy.t(), lhs, sp, side)) if tb else (lambda side: _run_sdd(lhs.t(), dy, sp, side))
         dlhs, ddata = _both(want_lhs, want_data, sp, dy.size(0))
         if dlhs is not None and lhs_is_view:
             dlhs = dlhs.t()
@@ -235,14 +245,14 @@ def _sdd_operand_gradients(ctx, lhs, rhs, sp, ds):
         return dlhs, dbase.t()
     if ctx.needs_input_grad[0]:
         if lhs_is_view:
-            want_lhs = lambda stream: _run_dds(rhs, sp, ds, True, stream)              # rhs dS^T, returned transposed
+            want_lhs = lambda side: _run_dds(rhs, sp, ds, True, side)              # rhs dS^T, returned transposed
         else:
-            want_lhs = lambda stream: _run_dsd(sp, ds, False, rhs.t(), stream)         # dS rhs^T
+            want_lhs = lambda side: _run_dsd(sp, ds, False, rhs.t(), side)         # dS rhs^T
     if ctx.needs_input_grad[1]:
         if rhs_is_view:
-            want_rhs = lambda stream: _run_dsd(sp, ds, True, lhs, stream)              # dS^T lhs, returned transposed
+            want_rhs = lambda side: _run_dsd(sp, ds, True, lhs, side)              # dS^T lhs, returned transposed
         else:
-            want_rhs = lambda stream: _run_dds(lhs.t(), sp, ds, False, stream)         # lhs^T dS
+            want_rhs = lambda side: _run_dds(lhs.t(), sp, ds, False, side)         # lhs^T dS
     dlhs, drhs = _both(want_lhs, want_rhs, sp, lhs.size(1))
     if dlhs is not None and lhs_is_view:
         dlhs = dlhs.t()

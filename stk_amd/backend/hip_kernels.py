@@ -154,18 +154,17 @@ ACTIVATIONS = {None: 0, "none": 0, "relu": 1, "gelu_tanh": 2, "gelu": 3, "silu":
                "relu_grad": 5, "gelu_tanh_grad": 6, "gelu_grad": 7, "silu_grad": 8}
 
 
-def sdd(lhs, rhs, shape, out, offsets, row_indices, column_indices, block_order=None, stream=-1):
+def sdd(lhs, rhs, shape, out, offsets, row_indices, column_indices, block_order=None):
     """out[p] = lhs[block row p] @ rhs[block column p]; out is [nnz, b, b].
 
     block_order (optional, not in the reference signature) is a permutation of
     the blocks that sets the visiting order of workgroups for 64x64 blocks.
-    stream (here and below): handle of the stream to launch on, -1 for torch's current one.
     """
-    sdd_fused(lhs, rhs, shape, out, offsets, row_indices, column_indices, None, None, block_order, None, stream)
+    sdd_fused(lhs, rhs, shape, out, offsets, row_indices, column_indices, None, None, block_order)
 
 
 def sdd_fused(lhs, rhs, shape, out, offsets, row_indices, column_indices, activation=None, multiplier=None,
-              block_order=None, sums=None, stream=-1):
+              block_order=None, sums=None):
     """sdd whose store applies `activation` (a key of ACTIVATIONS) to the fp32 sums and, after the
     rounding, multiplies by `multiplier` ([nnz, b, b] values of a matrix with the same topology).
     `sums` (like `out`, or None) also receives the rounded sums themselves (stk_sdd_fused_sums).
@@ -182,7 +181,7 @@ def sdd_fused(lhs, rhs, shape, out, offsets, row_indices, column_indices, activa
     plan = None
     if FUSION and (b == 128 or b == 64) and offsets is not None and out.shape[0] > 0:
         plan = fusion_plan(offsets, column_indices, blocking=b)
-    _lib.native().sdd(lhs, rhs, out, offsets, row_indices, column_indices, plan, ACTIVATIONS[activation], multiplier, block_order, sums, stream)
+    _lib.native().sdd(lhs, rhs, out, offsets, row_indices, column_indices, plan, ACTIVATIONS[activation], multiplier, block_order, sums)
 
 
 def activation_product(sums, factor, activation):
@@ -201,10 +200,10 @@ SLICE_LAST_ROUND = True
 # 128 tiles be cut in two, or one of 64 tiles in four; a launch that would like more is cut less.  The buffer is
 # allocated on the first dsd that can use it and kept; release_workspaces() frees it.
 DSD_WORKSPACE_SLOTS = 256
-# Streams, by handle, whose dsd launches may run beside those of other streams (the autograd layer's side stream): they get
+# Streams (their handles) whose dsd launches may run beside those of other streams (the autograd layer's side stream): they get
 # a workspace of their own.  Everything else shares one per device, and a launch on another stream than the
 # last one first waits for that stream.
-CONCURRENT_STREAMS = {}
+CONCURRENT_STREAMS = set()
 _dsd_workspaces = {}   # (device index, concurrent lane) -> [buffer, stream of the last launch]
 
 
@@ -235,9 +234,9 @@ def _new_workspace(device, nbytes, counters):
     return ws
 
 
-def _dsd_workspace(data, m, n, stream=-1):
-    """Workspace of stk_dsd for a product with these sparse values, or None: [counters | slots], the counters zero between
-    launches."""
+def _dsd_workspace(data, m, n):
+    """Workspace of stk_dsd for a product with these sparse values, launched on the current stream, or None:
+    [counters | slots], the counters zero between launches."""
     blocking = data.shape[-1]
     if not SLICE_LAST_ROUND or blocking != 128:
         return None
@@ -246,7 +245,7 @@ def _dsd_workspace(data, m, n, stream=-1):
     if lib.stk_dsd_workspace_bytes(m, n, blocking) <= 0 or lib.stk_dsd_is_small(data.shape[0], n):
         return None
     device = data.device
-    handle = _stream(device) if stream < 0 else stream
+    handle = _stream(device)
     key = (device.index, handle in CONCURRENT_STREAMS)
     entry = _dsd_workspaces.get(key)
     counters = lib.stk_dsd_workspace_counter_bytes()
@@ -254,27 +253,21 @@ def _dsd_workspace(data, m, n, stream=-1):
     if entry is not None and entry[0].numel() != nbytes:
         entry = None
     choice = _workspace_choice(_capture_id(handle) != 0, None if entry is None else entry[1].cuda_stream, handle)
-    if choice == "shared":
-        return entry[0]
-    # (allocated and cleared on the stream that the launch goes to)
-    current = torch.cuda.current_stream(device)
-    launch = current if handle == current.cuda_stream else CONCURRENT_STREAMS[handle]
-    if choice == "wait":
-        launch.wait_stream(entry[1])   # launches that share a workspace must not overlap
-        entry[1] = launch
-        return entry[0]
-    with torch.cuda.stream(launch):
-        buffer = _new_workspace(device, nbytes, counters)
     if choice == "private":
         # zeroed by a fill kernel that is part of the graph; the memory goes back to the graph's pool when the
         # caller drops it, where only later allocations of the same capture, which run behind this launch, reuse it
-        return buffer
-    _dsd_workspaces[key] = [buffer, launch]
-    return buffer
+        return _new_workspace(device, nbytes, counters)
+    if choice == "create":
+        entry = _dsd_workspaces[key] = [_new_workspace(device, nbytes, counters), torch.cuda.current_stream(device)]
+    elif choice == "wait":
+        stream = torch.cuda.current_stream(device)
+        stream.wait_stream(entry[1])   # launches that share a workspace must not overlap
+        entry[1] = stream
+    return entry[0]
 
 
 def dsd(shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
-        block_offsets_t, transpose_a, rhs, out, stream=-1):
+        block_offsets_t, transpose_a, rhs, out):
     """out = op(sparse) @ rhs; `shape` is the logical shape of the sparse operand."""
     if not out.is_cuda:
         host_kernels.matmul_dims(shape[1], shape[0], rhs.shape[0], rhs.shape[1], data.shape[-1])
@@ -282,9 +275,9 @@ def dsd(shape, data, offsets, row_indices, column_indices, offsets_t, column_ind
                                 transpose_a, rhs, out)
     m, k = shape
     plan = _plan_for(data, offsets, column_indices, offsets_t, column_indices_t)
-    ws = _dsd_workspace(data, m, out.shape[1], stream) if plan is not None else None
+    ws = _dsd_workspace(data, m, out.shape[1]) if plan is not None else None
     try:
-        _lib.native().dsd(m, k, data, offsets, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_a, rhs, out, plan, ws, stream)
+        _lib.native().dsd(m, k, data, offsets, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_a, rhs, out, plan, ws)
     except Exception:
         if ws is not None:
             release_workspaces()   # whatever a failed launch left in the counters is not reused
@@ -292,7 +285,7 @@ def dsd(shape, data, offsets, row_indices, column_indices, offsets_t, column_ind
 
 
 def dds(lhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
-        block_offsets_t, transpose_b, out, stream=-1):
+        block_offsets_t, transpose_b, out):
     """out = lhs @ op(sparse); `shape` is the logical shape of the sparse operand."""
     if not out.is_cuda:
         host_kernels.matmul_dims(lhs.shape[1], lhs.shape[0], shape[0], shape[1], data.shape[-1])
@@ -300,7 +293,7 @@ def dds(lhs, shape, data, offsets, row_indices, column_indices, offsets_t, colum
                                 transpose_b, out)
     k, n = shape
     plan = _plan_for(data, offsets, column_indices, offsets_t, column_indices_t)
-    _lib.native().dds(lhs, k, n, data, offsets, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_b, out, plan, stream)
+    _lib.native().dds(lhs, k, n, data, offsets, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_b, out, plan)
 
 
 def dsd_dds(shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, rhs, out_dsd, lhs, out_dds):

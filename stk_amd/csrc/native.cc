@@ -3,8 +3,8 @@
 // (include/stk_amd.h); what this saves is the host time of a launch.  Through ctypes, with the checks in Python, a call
 // took 10 - 14 us on the host, more than most kernels of a small problem take on the GPU; here it takes 3 - 5 us.
 //
-// Everything launches on torch's current stream of the tensors' device, or on the stream handle `stream` >= 0 where a
-// function takes one.  No state is kept between calls but one pinned word per host thread and device (Mailbox).
+// Everything - copies of operands, allocations, launches - happens on torch's current stream of the tensors' device.  No
+// state is kept between calls but one pinned word per host thread and device (Mailbox).
 #include <torch/extension.h>
 
 #include <c10/hip/HIPStream.h>
@@ -57,21 +57,14 @@ int index_dtype(at::ScalarType t) {
   if (t == at::kInt) return STK_I32;
   raise(PyExc_NotImplementedError, std::string("stk_amd: indices must be int16 or int32, got ") + c10::toString(t));
 }
-// Whether an operand of the call under way has been copied, on the current stream (see stream_of).
-thread_local bool copied = false;
-Tensor packed(const Tensor& t) {
-  if (t.is_contiguous()) return t;
-  copied = true;
-  return t.contiguous();
-}
 // Index tensors may arrive as strided views (stk/ops/matrix_ops.py:73-75).
 Tensor index(const Tensor& t) {
   index_dtype(t.scalar_type());
-  return packed(t);
+  return t.contiguous();
 }
 Tensor offsets32(const Tensor& t) {
   if (t.scalar_type() != at::kInt) raise(PyExc_NotImplementedError, std::string("stk_amd: offsets must be int32, got ") + c10::toString(t.scalar_type()));
-  return packed(t);
+  return t.contiguous();
 }
 bool aligned(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) == 0; }
 // A 2-D operand the kernels can read in place: unit stride in one dimension, the other stride a multiple of 8
@@ -80,7 +73,6 @@ Tensor dense_operand(const Tensor& x) {
   require(x.dim() == 2, "dense operands have two dimensions");
   const int64_t s0 = x.stride(0), s1 = x.stride(1);
   if (((s1 == 1 && s0 % 8 == 0) || (s0 == 1 && s1 % 8 == 0 && x.size(0) > 1)) && aligned(x)) return x;
-  copied = true;
   Tensor c = x.contiguous();
   if (!aligned(c) || c.stride(0) % 8) raise(PyExc_NotImplementedError, "stk_amd: dense operands need a row length divisible by 8");
   return c;
@@ -100,12 +92,8 @@ T* ptr(const Tensor& t) { return static_cast<T*>(const_cast<void*>(t.const_data_
 template <class T>
 T* ptr(const OptTensor& t) { return t ? ptr<T>(*t) : nullptr; }
 
-// The stream a call launches on.  A copy that the call has made of an operand is ordered and freed on the current stream,
-// so the launch stays there too.
-hipStream_t stream_of(const Tensor& t, int64_t stream = -1) {
-  if (stream >= 0 && !copied) return reinterpret_cast<hipStream_t>(stream);
-  return c10::hip::getCurrentHIPStream(t.device().index()).stream();
-}
+// The stream a call launches on.
+hipStream_t stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
 // ------------------------------------------------------------------------------------------------ products
 // The sparse operand's arrays as the launches take them.
@@ -120,8 +108,7 @@ struct Meta {
 #define META_PTRS(m) ptr<int32_t>(m.offsets), ptr<void>(m.ci), ptr<int32_t>(m.offsets_t), ptr<void>(m.cit), ptr<int32_t>(m.bot)
 
 void sdd(const Tensor& lhs_, const Tensor& rhs_, const Tensor& out, const OptTensor& offsets, const Tensor& row_indices, const Tensor& column_indices,
-         const OptTensor& plan, int activation, const OptTensor& multiplier, const OptTensor& block_order, const OptTensor& sums, int64_t stream) {
-  copied = false;
+         const OptTensor& plan, int activation, const OptTensor& multiplier, const OptTensor& block_order, const OptTensor& sums) {
   need_gpu(lhs_), need_gpu(rhs_), need_gpu(out);
   require(lhs_.dim() == 2 && rhs_.dim() == 2 && lhs_.size(1) == rhs_.size(0), "incompatible dimensions");
   const int64_t m = lhs_.size(0), k = lhs_.size(1), n = rhs_.size(1), b = out.size(-1), nnz = row_indices.numel();
@@ -150,12 +137,11 @@ void sdd(const Tensor& lhs_, const Tensor& rhs_, const Tensor& out, const OptTen
   if (plan) offs = offsets32(*offsets);
   check(stk_sdd_fused_sums(ptr<void>(lhs), lhs.stride(0), lhs.stride(1), ptr<void>(rhs), rhs.stride(0), rhs.stride(1), m, k, n, ptr<void>(out),
                            ptr<int32_t>(offs), ptr<void>(ri), ptr<void>(ci), ptr<int32_t>(order), nnz, (int)b, value_dtype(out),
-                           index_dtype(ri.scalar_type()), ptr<uint8_t>(plan), activation, ptr<void>(multiplier), ptr<void>(sums), stream_of(out, stream)));
+                           index_dtype(ri.scalar_type()), ptr<uint8_t>(plan), activation, ptr<void>(multiplier), ptr<void>(sums), stream_of(out)));
 }
 
 void dsd(int64_t m, int64_t k, const Tensor& data, META_ARGS, bool transpose_a, const Tensor& rhs_, const Tensor& out, const OptTensor& plan,
-         const OptTensor& workspace, int64_t stream) {
-  copied = false;
+         const OptTensor& workspace) {
   need_gpu(data), need_gpu(rhs_), need_gpu(out);
   require(rhs_.dim() == 2 && k == rhs_.size(0), "incompatible dimensions");
   const int64_t n = rhs_.size(1), b = data.size(-1);
@@ -167,12 +153,10 @@ void dsd(int64_t m, int64_t k, const Tensor& data, META_ARGS, bool transpose_a, 
   const Meta s(offsets, column_indices, offsets_t, column_indices_t, block_offsets_t);
   check(stk_dsd(m, k, n, ptr<void>(data), META_PTRS(s), transpose_a, ptr<void>(rhs), rhs.stride(0), rhs.stride(1), ptr<void>(out), out.stride(0),
                 data.size(0), (int)b, value_dtype(out), s.idx, ptr<uint8_t>(plan), ptr<void>(workspace), workspace ? workspace->numel() : 0,
-                stream_of(out, stream)));
+                stream_of(out)));
 }
 
-void dds(const Tensor& lhs_, int64_t k, int64_t n, const Tensor& data, META_ARGS, bool transpose_b, const Tensor& out, const OptTensor& plan,
-         int64_t stream) {
-  copied = false;
+void dds(const Tensor& lhs_, int64_t k, int64_t n, const Tensor& data, META_ARGS, bool transpose_b, const Tensor& out, const OptTensor& plan) {
   need_gpu(data), need_gpu(lhs_), need_gpu(out);
   require(lhs_.dim() == 2 && lhs_.size(1) == k, "incompatible dimensions");
   const int64_t m = lhs_.size(0), b = data.size(-1);
@@ -183,7 +167,7 @@ void dds(const Tensor& lhs_, int64_t k, int64_t n, const Tensor& data, META_ARGS
   require(data.scalar_type() == lhs.scalar_type() && data.scalar_type() == out.scalar_type(), "operands and out must have one dtype");
   const Meta s(offsets, column_indices, offsets_t, column_indices_t, block_offsets_t);
   check(stk_dds(m, k, n, ptr<void>(lhs), lhs.stride(0), lhs.stride(1), ptr<void>(data), META_PTRS(s), transpose_b, ptr<void>(out), out.stride(0),
-                data.size(0), (int)b, value_dtype(out), s.idx, ptr<uint8_t>(plan), stream_of(out, stream)));
+                data.size(0), (int)b, value_dtype(out), s.idx, ptr<uint8_t>(plan), stream_of(out)));
 }
 
 void dsd_dds(int64_t m, int64_t k, const Tensor& data, META_ARGS, const Tensor& rhs_, const Tensor& out_dsd, const Tensor& lhs_, const Tensor& out_dds,
