@@ -71,6 +71,7 @@ def test_forward_chain_replays_from_a_graph(blocking, dtype, warm_up_on_capture_
 def test_forward_and_backward_replay_from_a_graph(joint_dsd_gradients, monkeypatch):
     from stk_amd.backend import autograd
     monkeypatch.setattr(autograd, "JOINT_DSD_GRADIENTS", joint_dsd_gradients)
+    monkeypatch.setattr(autograd, "OVERLAP_FROM", 0.0)
     dtype = torch.bfloat16
     topo, tm, x, w1, w2, g = _case(1024, 4096, 128, dtype, 43)
     xs, w1s, w2s = (t.detach().clone().requires_grad_(True) for t in (x, w1, w2))

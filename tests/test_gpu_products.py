@@ -691,18 +691,24 @@ def test_both_gradients_of_dsd_in_one_call(dtype, blocking, hidden, ffn, tokens,
 
 def test_gradients_side_by_side_equal_gradients_one_after_the_other(monkeypatch):
     # backward launches the two gradients of a product on two streams; same kernels, so the same bits
-    from stk_amd.backend import autograd
+    from stk_amd.backend import autograd, hip_kernels
     tokens = np.array([256, 384, 128, 512, 256, 384, 640, 128])
     topo, tm, x, w1, w2 = _dmoe_case(tokens, 256, 512, 128, torch.bfloat16, 21)
+    monkeypatch.setattr(autograd, "OVERLAP_FROM", 0.0)     # (products of 0.7 GFLOP)
+    waits = []
+    follow = hip_kernels.follow_stream
+    monkeypatch.setattr(hip_kernels, "follow_stream", lambda *streams: (waits.append(streams), follow(*streams)))
     grads = {}
     for overlap in (True, False, True):
         monkeypatch.setattr(autograd, "OVERLAP_GRADIENTS", overlap)
+        waits.clear()
         xs, w1s, w2s = (t.detach().clone().requires_grad_(True) for t in (x, w1, w2))
         h = stk.ops.sdd(xs, w1s, tm)
         y = stk.ops.dsd(h, w2s)
         z = stk.ops.dds(y.t()[:256].contiguous(), h)          # a third product on the same sparse values
         (y.float().square().sum() + z.float().sum()).backward()
         torch.cuda.synchronize()
+        assert len(waits) == (4 if overlap else 0)         # there and back for the pairs of dsd and dds
         got = [xs.grad.clone(), w1s.grad.clone(), w2s.grad.clone()]
         if overlap in grads:
             assert all(torch.equal(a, b) for a, b in zip(got, grads[overlap]))     # and repeatable
