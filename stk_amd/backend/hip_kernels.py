@@ -212,6 +212,15 @@ def release_workspaces():
     _dsd_workspaces.clear()
 
 
+def _check_launch(status, ws):
+    """Raises for a launch that was refused or failed.  Whatever a failed launch has left in the counters of the workspace
+    `ws` is not reused; a call that was refused has not touched them."""
+    if status == _lib.STK_ERR_HIP and ws is not None:
+        for key in [key for key, entry in _dsd_workspaces.items() if entry[0] is ws]:
+            del _dsd_workspaces[key]
+    _lib.check(status)
+
+
 def _workspace_choice(capturing, entry_stream, handle):
     """Which workspace a dsd launch on the stream `handle` takes.  `capturing`: a graph capture is under way on that
     stream; `entry_stream`: handle of the stream that last used the device's shared workspace (None: there is none yet).
@@ -262,6 +271,7 @@ def _dsd_workspace(data, m, n):
     elif choice == "wait":
         stream = torch.cuda.current_stream(device)
         stream.wait_stream(entry[1])   # launches that share a workspace must not overlap
+        entry[0].record_stream(stream)   # (dropped, its memory is not handed out again before they have ended)
         entry[1] = stream
     return entry[0]
 
@@ -276,12 +286,7 @@ def dsd(shape, data, offsets, row_indices, column_indices, offsets_t, column_ind
     m, k = shape
     plan = _plan_for(data, offsets, column_indices, offsets_t, column_indices_t)
     ws = _dsd_workspace(data, m, out.shape[1]) if plan is not None else None
-    try:
-        _lib.native().dsd(m, k, data, offsets, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_a, rhs, out, plan, ws)
-    except Exception:
-        if ws is not None:
-            release_workspaces()   # whatever a failed launch left in the counters is not reused
-        raise
+    _check_launch(_lib.native().dsd(m, k, data, offsets, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_a, rhs, out, plan, ws), ws)
 
 
 def dds(lhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
@@ -410,9 +415,8 @@ def dsd_scatter(shape, data, offsets, column_indices, offsets_t, column_indices_
         return False
     plan = fusion_plan(offsets, column_indices, offsets_t, column_indices_t, blocking=128)
     ws = _dsd_workspace(data, m, n)
-    try:
-        return _lib.native().dsd_scatter(m, k, data, offsets, column_indices, rhs, row_slots, weights, out, plan, ws)
-    except Exception:
-        if ws is not None:
-            release_workspaces()
-        raise
+    status = _lib.native().dsd_scatter(m, k, data, offsets, column_indices, rhs, row_slots, weights, out, plan, ws)
+    if status == _lib.STK_ERR_UNSUPPORTED:
+        return False
+    _check_launch(status, ws)
+    return True

@@ -140,8 +140,9 @@ void sdd(const Tensor& lhs_, const Tensor& rhs_, const Tensor& out, const OptTen
                            index_dtype(ri.scalar_type()), ptr<uint8_t>(plan), activation, ptr<void>(multiplier), ptr<void>(sums), stream_of(out)));
 }
 
-void dsd(int64_t m, int64_t k, const Tensor& data, META_ARGS, bool transpose_a, const Tensor& rhs_, const Tensor& out, const OptTensor& plan,
-         const OptTensor& workspace) {
+// The status of the launch: the caller owns the workspace, whose state depends on it.  (Operands that are refused raise.)
+int dsd(int64_t m, int64_t k, const Tensor& data, META_ARGS, bool transpose_a, const Tensor& rhs_, const Tensor& out, const OptTensor& plan,
+        const OptTensor& workspace) {
   need_gpu(data), need_gpu(rhs_), need_gpu(out);
   require(rhs_.dim() == 2 && k == rhs_.size(0), "incompatible dimensions");
   const int64_t n = rhs_.size(1), b = data.size(-1);
@@ -151,9 +152,9 @@ void dsd(int64_t m, int64_t k, const Tensor& data, META_ARGS, bool transpose_a, 
   require(data.is_contiguous() && out.stride(1) == 1, "the sparse values must be contiguous and out row-major");
   require(data.scalar_type() == rhs.scalar_type() && data.scalar_type() == out.scalar_type(), "operands and out must have one dtype");
   const Meta s(offsets, column_indices, offsets_t, column_indices_t, block_offsets_t);
-  check(stk_dsd(m, k, n, ptr<void>(data), META_PTRS(s), transpose_a, ptr<void>(rhs), rhs.stride(0), rhs.stride(1), ptr<void>(out), out.stride(0),
-                data.size(0), (int)b, value_dtype(out), s.idx, ptr<uint8_t>(plan), ptr<void>(workspace), workspace ? workspace->numel() : 0,
-                stream_of(out)));
+  return stk_dsd(m, k, n, ptr<void>(data), META_PTRS(s), transpose_a, ptr<void>(rhs), rhs.stride(0), rhs.stride(1), ptr<void>(out), out.stride(0),
+                 data.size(0), (int)b, value_dtype(out), s.idx, ptr<uint8_t>(plan), ptr<void>(workspace), workspace ? workspace->numel() : 0,
+                 stream_of(out));
 }
 
 void dds(const Tensor& lhs_, int64_t k, int64_t n, const Tensor& data, META_ARGS, bool transpose_b, const Tensor& out, const OptTensor& plan) {
@@ -538,8 +539,9 @@ bool sdd_gather(const Tensor& x_, const Tensor& row_slots, int top_k, const Tens
   return true;
 }
 
-// out = padded_scatter(sparse @ rhs, top_k = 1, weights); false, with nothing launched, when the library has no such kernel
-bool dsd_scatter(int64_t m, int64_t k, const Tensor& data, const Tensor& offsets, const Tensor& column_indices, const Tensor& rhs_, const Tensor& row_slots,
+// out = padded_scatter(sparse @ rhs, top_k = 1, weights); the status, STK_ERR_UNSUPPORTED, with nothing launched, when the
+// library has no such kernel
+int dsd_scatter(int64_t m, int64_t k, const Tensor& data, const Tensor& offsets, const Tensor& column_indices, const Tensor& rhs_, const Tensor& row_slots,
                  const OptTensor& weights, const Tensor& out, const Tensor& plan, const OptTensor& workspace) {
   need_gpu(data), need_gpu(rhs_), need_gpu(row_slots), need_gpu(out);
   require(rhs_.dim() == 2 && k == rhs_.size(0), "incompatible dimensions");
@@ -552,13 +554,10 @@ bool dsd_scatter(int64_t m, int64_t k, const Tensor& data, const Tensor& offsets
   require(row_slots.scalar_type() == at::kInt && row_slots.is_contiguous() && row_slots.numel() >= m, "row_slots must name the rows of the padded layout");
   const OptTensor w = weights32(weights, out.size(0));
   const Tensor ci = index(column_indices), offs = offsets32(offsets);
-  const int status = stk_dsd_scatter(m, k, n, ptr<void>(data), ptr<int32_t>(offs), ptr<void>(ci), ptr<void>(rhs), rhs.stride(0), rhs.stride(1),
-                                     ptr<int32_t>(row_slots), ptr<float>(w), out.size(0), ptr<void>(out), out.stride(0), data.size(0), (int)b, value_dtype(out),
-                                     index_dtype(ci.scalar_type()), ptr<uint8_t>(plan), ptr<void>(workspace), workspace ? workspace->numel() : 0,
-                                     stream_of(out));
-  if (status == STK_ERR_UNSUPPORTED) return false;
-  check(status);
-  return true;
+  return stk_dsd_scatter(m, k, n, ptr<void>(data), ptr<int32_t>(offs), ptr<void>(ci), ptr<void>(rhs), rhs.stride(0), rhs.stride(1),
+                         ptr<int32_t>(row_slots), ptr<float>(w), out.size(0), ptr<void>(out), out.stride(0), data.size(0), (int)b, value_dtype(out),
+                         index_dtype(ci.scalar_type()), ptr<uint8_t>(plan), ptr<void>(workspace), workspace ? workspace->numel() : 0,
+                         stream_of(out));
 }
 
 }  // namespace

@@ -238,6 +238,62 @@ def test_dsd_workspace_choice():
     assert _workspace_choice(False, 7, 5) == "wait"
 
 
+def _dsd_with(monkeypatch, outcome):
+    """hip_kernels.dsd on stand-ins, with a workspace of its lane and one of another lane, its native call ending as `outcome`
+    says: the lanes that are left."""
+    from types import SimpleNamespace as S
+    from stk_amd.backend import hip_kernels as hk
+
+    def native(*args):
+        if isinstance(outcome, Exception):
+            raise outcome
+        return outcome
+
+    mine, others = object(), object()
+    lanes = {(0, False): [mine, None], (0, True): [others, None]}
+    monkeypatch.setattr(hk, "_dsd_workspaces", lanes)
+    monkeypatch.setattr(hk, "_plan_for", lambda *args: object())
+    monkeypatch.setattr(hk, "_dsd_workspace", lambda *args: mine)
+    monkeypatch.setattr(hk._lib, "native", lambda: S(dsd=native))
+    monkeypatch.setattr(hk._lib, "load", lambda: S(stk_last_error=lambda: b"said by the library"))
+    t = S(is_cuda=True, shape=(256, 256))
+    raised = None
+    try:
+        hk.dsd((256, 256), t, None, None, None, None, None, None, False, t, t)
+    except Exception as e:
+        raised = type(e)
+    return raised, set(lanes)
+
+
+def test_a_refused_dsd_keeps_the_workspaces_and_a_failed_one_drops_its_own(monkeypatch):
+    from stk_amd.backend import _lib
+    both = {(0, False), (0, True)}
+    assert _dsd_with(monkeypatch, _lib.STK_OK) == (None, both)
+    for refusal in (AssertionError("incompatible dimensions"), NotImplementedError("dtype"), RuntimeError("not on a GPU")):
+        assert _dsd_with(monkeypatch, refusal) == (type(refusal), both)
+    assert _dsd_with(monkeypatch, _lib.STK_ERR_DIMS) == (AssertionError, both)
+    assert _dsd_with(monkeypatch, _lib.STK_ERR_HIP) == (RuntimeError, {(0, True)})
+
+
+def test_a_workspace_that_changes_streams_is_recorded_on_the_new_one(monkeypatch):
+    # (the caching allocator otherwise hands a dropped workspace out on the stream it was allocated on, at once)
+    from types import SimpleNamespace as S
+    from stk_amd.backend import hip_kernels as hk
+    events = []
+    stream = lambda handle: S(cuda_stream=handle, wait_stream=lambda other: events.append(("wait", handle, other.cuda_stream)))
+    buffer = S(numel=lambda: 8 + hk.DSD_WORKSPACE_SLOTS * 4, record_stream=lambda s: events.append(("record", s.cuda_stream)))
+    lib = S(stk_dsd_workspace_bytes=lambda *a: 1, stk_dsd_is_small=lambda *a: 0, stk_dsd_workspace_counter_bytes=lambda: 8, stk_dsd_workspace_slot_bytes=lambda: 4)
+    monkeypatch.setattr(hk._lib, "load", lambda: lib)
+    monkeypatch.setattr(hk, "_capture_id", lambda handle: 0)
+    monkeypatch.setattr(hk, "_dsd_workspaces", {(0, False): [buffer, stream(5)]})
+    data = S(shape=(64, 128, 128), device=S(index=0))
+    for handle in (5, 7, 7, 5):
+        monkeypatch.setattr(hk, "_stream", lambda device: handle)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: stream(handle))
+        assert hk._dsd_workspace(data, 256, 256) is buffer
+    assert events == [("wait", 7, 5), ("record", 7), ("wait", 5, 7), ("record", 5)]
+
+
 def test_fusion_plan_cache_is_tied_to_the_index_tensors_it_was_built_from():
     # the plan of a topology is cached on its offsets tensor; the entry holds the other index tensors, so that
     # a new tensor at a recycled address, an in-place change or a tensor without a version counter miss
