@@ -16,6 +16,8 @@ the reference's plumbing configuration - products on CPU tensors - runs here.
 The checks, allocations and launches are native code (csrc/native.cc); what is left here is what depends on the
 switches below and on the caches: which fusion plan and which workspace a launch gets.
 """
+import threading
+
 import torch
 
 from stk_amd.backend import _lib, host_kernels
@@ -205,6 +207,9 @@ DSD_WORKSPACE_SLOTS = 256
 # last one first waits for that stream.
 CONCURRENT_STREAMS = set()
 _dsd_workspaces = {}   # (device index, concurrent lane) -> [buffer, stream of the last launch]
+# Held from the choice of a workspace to its launch: a thread that takes it over for another stream waits for what has been
+# launched, which has to include the launch that the entry names.
+_workspace_lock = threading.RLock()
 
 
 def release_workspaces():
@@ -285,8 +290,10 @@ def dsd(shape, data, offsets, row_indices, column_indices, offsets_t, column_ind
                                 transpose_a, rhs, out)
     m, k = shape
     plan = _plan_for(data, offsets, column_indices, offsets_t, column_indices_t)
-    ws = _dsd_workspace(data, m, out.shape[1]) if plan is not None else None
-    _check_launch(_lib.native().dsd(m, k, data, offsets, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_a, rhs, out, plan, ws), ws)
+    with _workspace_lock:
+        ws = _dsd_workspace(data, m, out.shape[1]) if plan is not None else None
+        _check_launch(_lib.native().dsd(m, k, data, offsets, column_indices, offsets_t, column_indices_t, block_offsets_t, transpose_a, rhs, out, plan,
+                                        ws), ws)
 
 
 def dds(lhs, shape, data, offsets, row_indices, column_indices, offsets_t, column_indices_t,
@@ -414,9 +421,10 @@ def dsd_scatter(shape, data, offsets, column_indices, offsets_t, column_indices_
     if data.shape[-1] != 128 or n < 256 or n % 64 or not FUSION or data.shape[0] == 0 or out.shape[0] == 0:
         return False
     plan = fusion_plan(offsets, column_indices, offsets_t, column_indices_t, blocking=128)
-    ws = _dsd_workspace(data, m, n)
-    status = _lib.native().dsd_scatter(m, k, data, offsets, column_indices, rhs, row_slots, weights, out, plan, ws)
-    if status == _lib.STK_ERR_UNSUPPORTED:
-        return False
-    _check_launch(status, ws)
+    with _workspace_lock:
+        ws = _dsd_workspace(data, m, n)
+        status = _lib.native().dsd_scatter(m, k, data, offsets, column_indices, rhs, row_slots, weights, out, plan, ws)
+        if status == _lib.STK_ERR_UNSUPPORTED:
+            return False
+        _check_launch(status, ws)
     return True

@@ -294,6 +294,38 @@ def test_a_workspace_that_changes_streams_is_recorded_on_the_new_one(monkeypatch
     assert events == [("wait", 7, 5), ("record", 7), ("wait", 5, 7), ("record", 5)]
 
 
+def test_a_workspace_is_launched_with_before_another_thread_takes_it_over(monkeypatch):
+    import threading
+    import time
+    from types import SimpleNamespace as S
+    from stk_amd.backend import hip_kernels as hk
+    events = []
+
+    def choose(*args):
+        events.append(("chosen", threading.current_thread().name))
+
+    def launch(*args):
+        time.sleep(0.05)       # (native code runs without the interpreter's lock)
+        events.append(("launched", threading.current_thread().name))
+        return 0
+
+    monkeypatch.setattr(hk, "_plan_for", lambda *args: object())
+    monkeypatch.setattr(hk, "fusion_plan", lambda *args, **kwargs: object())
+    monkeypatch.setattr(hk, "_dsd_workspace", choose)
+    monkeypatch.setattr(hk._lib, "native", lambda: S(dsd=launch, dsd_scatter=launch))
+    t = S(is_cuda=True, shape=(256, 256))
+    data = S(is_cuda=True, shape=(4, 128, 128))
+    calls = [lambda: hk.dsd((256, 256), data, None, None, None, None, None, None, False, t, t),
+             lambda: hk.dsd_scatter((256, 256), data, None, None, None, None, t, None, None, t)]
+    threads = [threading.Thread(target=calls[i % 2], name=str(i)) for i in range(4)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert [kind for kind, _ in events] == ["chosen", "launched"] * 4
+    assert all(events[i][1] == events[i + 1][1] for i in range(0, 8, 2))
+
+
 def test_fusion_plan_cache_is_tied_to_the_index_tensors_it_was_built_from():
     # the plan of a topology is cached on its offsets tensor; the entry holds the other index tensors, so that
     # a new tensor at a recycled address, an in-place change or a tensor without a version counter miss
