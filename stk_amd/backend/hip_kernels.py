@@ -86,8 +86,8 @@ def _plan_cache_get(tensors, blocking):
 
 def _plan_cache_put(tensors, blocking, plan, stream_handle, built, capture):
     """Remembers `plan` on tensors[0]; tensors without a version counter (made under inference mode)
-    cannot be watched for in-place changes and are not cached.  `built`: the torch stream whose handle is
-    stream_handle, on which the plan was built; `capture`: the graph capture it was built in (0: none)."""
+    cannot be watched for in-place changes and are not cached.  `built`: the event behind the build on the stream with the
+    handle stream_handle; `capture`: the graph capture it was built in (0: none)."""
     versions = tuple(_version_of(t) for t in tensors)
     if None in versions:
         return False
@@ -121,7 +121,7 @@ def fusion_plan(offsets, column_indices, offsets_t=None, column_indices_t=None, 
         if built_in in (0, capture):
             if cached[3] != handle and (built_in != 0 or capture == 0):
                 # built on another stream: what this one launches next comes after the build
-                torch.cuda.current_stream(offsets.device).wait_stream(cached[4])
+                torch.cuda.current_stream(offsets.device).wait_event(cached[4])
             return cached[1]
     plan = _lib.native().build_plan(offsets, column_indices, offsets_t if want_cols else None, column_indices_t if want_cols else None, blocking)
     _remember_plan(tensors, blocking, plan)
@@ -131,7 +131,9 @@ def fusion_plan(offsets, column_indices, offsets_t=None, column_indices_t=None, 
 def _remember_plan(tensors, blocking, plan):
     """The plan has just been built on the current stream: into the cache with it."""
     stream = torch.cuda.current_stream(tensors[0].device)
-    _plan_cache_put(tensors, blocking, plan, stream.cuda_stream, stream, _capture_id(stream.cuda_stream))
+    built = torch.cuda.Event()
+    built.record(stream)
+    _plan_cache_put(tensors, blocking, plan, stream.cuda_stream, built, _capture_id(stream.cuda_stream))
 
 
 def _plan_for(data, offsets, column_indices, offsets_t, column_indices_t):

@@ -326,6 +326,43 @@ def test_a_workspace_is_launched_with_before_another_thread_takes_it_over(monkey
     assert all(events[i][1] == events[i + 1][1] for i in range(0, 8, 2))
 
 
+def _plan_streams(monkeypatch):
+    """hip_kernels on stand-ins for streams, events and the plan: a list of what happens on the streams, and use(stream) to have
+    the plan of one topology used on a stream."""
+    from types import SimpleNamespace as S
+    from stk_amd.backend import hip_kernels as hk
+    log = []
+
+    class Event:
+        def record(self, stream):
+            self.after = len([e for e in log if e == ("work", stream.cuda_stream)])
+            log.append(("event", stream.cuda_stream))
+
+    plan = S(record_stream=lambda stream: log.append(("lifetime", stream.cuda_stream)))
+    offsets, ci = torch.arange(0, 20, 4, dtype=torch.int32), torch.zeros(16, dtype=torch.int16)
+    monkeypatch.setattr(hk, "_need_gpu", lambda *tensors: None)
+    monkeypatch.setattr(hk, "_capture_id", lambda handle: 0)
+    monkeypatch.setattr(hk._lib, "native", lambda: S(build_plan=lambda *args: plan))
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+
+    def use(handle):
+        stream = S(cuda_stream=handle, wait_event=lambda event: log.append(("wait", handle, event.after)),
+                   wait_stream=lambda other: log.append(("wait", handle, len([e for e in log if e == ("work", other.cuda_stream)]))))
+        monkeypatch.setattr(hk, "_stream", lambda device: handle)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: stream)
+        assert hk.fusion_plan(offsets, ci, blocking=128) is plan
+        log.append(("work", handle))
+    return log, use
+
+
+def test_a_plan_from_another_stream_is_waited_for_and_nothing_behind_it(monkeypatch):
+    log, use = _plan_streams(monkeypatch)
+    for handle in (5, 5, 5, 7, 5, 7):
+        use(handle)
+    assert [e for e in log if e[0] == "wait"] == [("wait", 7, 0), ("wait", 7, 0)]     # for none of the work on stream 5
+    assert [e for e in log if e[0] == "event"] == [("event", 5)]
+
+
 def test_fusion_plan_cache_is_tied_to_the_index_tensors_it_was_built_from():
     # the plan of a topology is cached on its offsets tensor; the entry holds the other index tensors, so that
     # a new tensor at a recycled address, an in-place change or a tensor without a version counter miss
