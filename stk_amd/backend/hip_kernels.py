@@ -121,7 +121,9 @@ def fusion_plan(offsets, column_indices, offsets_t=None, column_indices_t=None, 
         if built_in in (0, capture):
             if cached[3] != handle and (built_in != 0 or capture == 0):
                 # built on another stream: what this one launches next comes after the build
-                torch.cuda.current_stream(offsets.device).wait_event(cached[4])
+                stream = torch.cuda.current_stream(offsets.device)
+                stream.wait_event(cached[4])
+                cached[1].record_stream(stream)   # (dropped with its topology, its memory outlives what is launched now)
             return cached[1]
     plan = _lib.native().build_plan(offsets, column_indices, offsets_t if want_cols else None, column_indices_t if want_cols else None, blocking)
     _remember_plan(tensors, blocking, plan)

@@ -363,6 +363,13 @@ def test_a_plan_from_another_stream_is_waited_for_and_nothing_behind_it(monkeypa
     assert [e for e in log if e[0] == "event"] == [("event", 5)]
 
 
+def test_a_plan_outlives_its_use_on_another_stream(monkeypatch):
+    log, use = _plan_streams(monkeypatch)
+    for handle in (5, 7, 5):
+        use(handle)
+    assert [e for e in log if e[0] == "lifetime"] == [("lifetime", 7)]
+
+
 def test_fusion_plan_cache_is_tied_to_the_index_tensors_it_was_built_from():
     # the plan of a topology is cached on its offsets tensor; the entry holds the other index tensors, so that
     # a new tensor at a recycled address, an in-place change or a tensor without a version counter miss
