@@ -146,12 +146,19 @@ def _plan_for(data, offsets, column_indices, offsets_t, column_indices_t):
     return None
 
 
+def _can_be_cached(*tensors):
+    """Whether a plan of these index tensors would be found again: tensors made under inference mode keep no version counter."""
+    return not any(t.is_inference() for t in tensors)
+
+
 def prepare_plan(data, offsets, column_indices, offsets_t, column_indices_t):
     """Builds the fusion plan of a topology for both directions if there is none yet.  sdd itself needs the block rows
     only (its signature, the reference's, has no transpose metadata), so a plan built by its first call would be built
     again, with the columns, by the dsd or dds that follows on the same topology; callers that have the whole metadata
-    at hand (the autograd functions) call this first and every product finds the one plan."""
-    if data.dim() == 3 and offsets.is_cuda and column_indices.numel() > 0:
+    at hand (the autograd functions) call this first and every product finds the one plan.  Nothing is built for index tensors
+    whose plan no product would find."""
+    if (data.dim() == 3 and offsets.is_cuda and column_indices.numel() > 0
+            and _can_be_cached(offsets, column_indices, offsets_t, column_indices_t)):
         _plan_for(data, offsets, column_indices, offsets_t, column_indices_t)
 
 
@@ -358,8 +365,10 @@ def dmoe_topology(padded_bins, blocking, block_rows, blocks_per_row, index_dtype
     """(offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t) of the
     block-diagonal dropless-MoE pattern, one launch, no sort.  padded_bins: int32 device tensor,
     inclusive prefix sum of the per-expert row counts (each a multiple of `blocking`).  The launch also
-    builds the fusion plan, which the products on the topology then find on `offsets`."""
-    with_plan = FUSION and blocking in (64, 128) and block_rows * blocks_per_row > 0 and padded_bins.numel() <= DMOE_PLAN_EXPERTS
+    builds the fusion plan, which the products on the topology then find on `offsets` (not under inference mode, where
+    they could not)."""
+    with_plan = (FUSION and blocking in (64, 128) and block_rows * blocks_per_row > 0 and padded_bins.numel() <= DMOE_PLAN_EXPERTS
+                 and not torch.is_inference_mode_enabled())
     *meta, plan = _lib.native().dmoe_topology(padded_bins, blocking, block_rows, blocks_per_row, _INDEX_DTYPES[index_dtype] == _lib.STK_I32, with_plan)
     if plan is not None:
         offsets, _, column_indices, offsets_t, column_indices_t, _ = meta

@@ -370,6 +370,30 @@ def test_a_plan_outlives_its_use_on_another_stream(monkeypatch):
     assert [e for e in log if e[0] == "lifetime"] == [("lifetime", 7)]
 
 
+def test_no_plan_is_built_ahead_where_no_product_would_find_it(monkeypatch):
+    # (tensors made under inference mode keep no version counter, so their plan is not cached: every product builds its own)
+    from types import SimpleNamespace as S
+    from stk_amd.backend import hip_kernels as hk
+    asked = []
+    monkeypatch.setattr(hk, "_plan_for", lambda *args: asked.append("prepared"))
+    monkeypatch.setattr(hk, "_remember_plan", lambda *args: None)
+    monkeypatch.setattr(hk._lib, "native", lambda: S(dmoe_topology=lambda *args: asked.append(args[-1]) or (None,) * 7))
+    bins = torch.tensor([128, 256], dtype=torch.int32)
+
+    def meta(frozen):
+        return [S(is_cuda=True, numel=lambda: 4, is_inference=lambda i=i: frozen == i) for i in range(4)]
+    for frozen, want in ((None, ["prepared"]), (0, []), (1, []), (2, []), (3, [])):
+        hk.prepare_plan(S(dim=lambda: 3), *meta(frozen))
+        assert asked == want, frozen
+        asked.clear()
+    hk.dmoe_topology(bins, 128, 2, 2)
+    with torch.inference_mode():
+        hk.dmoe_topology(bins, 128, 2, 2)
+    with torch.no_grad():
+        hk.dmoe_topology(bins, 128, 2, 2)
+    assert asked == [True, False, True]
+
+
 def test_fusion_plan_cache_is_tied_to_the_index_tensors_it_was_built_from():
     # the plan of a topology is cached on its offsets tensor; the entry holds the other index tensors, so that
     # a new tensor at a recycled address, an in-place change or a tensor without a version counter miss
