@@ -44,12 +44,12 @@ struct DmoeArgs {
 };
 
 // First block row of expert e; the rows past the last bin belong to the last expert, bins that claim more rows than there
-// are stay inside the arrays.
+// are, or less than none, stay inside the arrays.
 __device__ __forceinline__ int first_row_of(const DmoeArgs& g, int e) {
   if (e == 0) return 0;
   if (e == g.experts) return g.block_rows;
   const int r = g.bins[e - 1] / g.blocking;
-  return r < g.block_rows ? r : g.block_rows;
+  return r < 0 ? 0 : r < g.block_rows ? r : g.block_rows;
 }
 
 // Groups of a run of n identical lines, by the plan list that holds their first lines.  FOURS: the plan of 64-blocks.
@@ -349,7 +349,7 @@ __device__ __forceinline__ void dmoe_arrays(const DmoeArgs& g, First&& first, in
       column_indices[p] = (IDX)(e * width + j);
       if (j == 0) g.offsets[i] = i * width;
       const int64_t q = (int64_t)f * width + (int64_t)j * (first(e + 1) - f) + (i - f);
-      if (q >= 0 && q < nnz) {   // (false for bins that do not ascend only)
+      if (q >= 0 && q < nnz) {   // (false for bins that do not ascend, without a plan, only)
         column_indices_t[q] = (IDX)i;
         g.block_offsets_t[q] = (int32_t)p;
       }
@@ -370,8 +370,18 @@ template <typename IDX, bool FOURS>
 __global__ __launch_bounds__(256) void dmoe_plan_kernel(DmoeArgs g) {
   extern __shared__ int lds[];
   const DmoeLds s(lds, g.experts);
-  for (int e = threadIdx.x; e <= g.experts; e += 256) s.first[e] = first_row_of(g, e);
-  __syncthreads();
+  bool descends = false;
+  for (int e = threadIdx.x; e <= g.experts; e += 256) {
+    s.first[e] = first_row_of(g, e);
+    descends |= e < g.experts && first_row_of(g, e + 1) < s.first[e];
+  }
+  // Bins that do not ascend are read as their running maximum: an expert whose bin lies below an earlier one has no rows.
+  // The experts' rows then add up to block_rows, which is what the lengths of the plan's lists rest on.
+  if (__syncthreads_or(descends)) {
+    if (threadIdx.x == 0)
+      for (int e = 1; e <= g.experts; e++) s.first[e] = max(s.first[e], s.first[e - 1]);
+    __syncthreads();
+  }
   const int64_t thread = blockIdx.x * (int64_t)256 + threadIdx.x, threads = (int64_t)gridDim.x * 256;
   dmoe_arrays<IDX>(g, [&](int e) { return s.first[e]; }, thread, threads);
   dmoe_plan<FOURS>(g, s, thread, threads);

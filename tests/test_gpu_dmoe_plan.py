@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import stk_amd as stk
-from stk_amd.backend import hip_kernels
+from stk_amd.backend import _lib, hip_kernels
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -61,3 +61,25 @@ def test_rows_behind_the_last_bin_belong_to_the_last_expert():
     compared = hip_kernels.fusion_plan(m.offsets.clone(), m.column_indices, m.offsets_t, m.column_indices_t, blocking=128)
     assert m.offsets_t.tolist() == [0, 2, 4, 6, 10, 14, 18]
     assert _parts(m.offsets._stk_plan[1], 6, 6, 18) == _parts(compared, 6, 6, 18)
+
+
+# 1024 experts whose bins go up and down: their row counts, each taken on its own, add up to 512 times the rows there are
+@pytest.mark.parametrize("blocking", [128, 64])
+@pytest.mark.parametrize("bins,block_rows", [([5, 2, 9, 9, 4, 12], 12), ([-3, 4, -1, 8], 8), ([0, 40] * 512, 40), ([50, 10, 60], 8)])
+def test_bins_that_do_not_ascend_stay_inside_the_plan(bins, block_rows, blocking):
+    E, width = len(bins), 3
+    nnz, columns = block_rows * width, E * width
+    given = torch.tensor(bins, dtype=torch.int32, device=DEV) * blocking
+    read_as = torch.cummax(given.clamp(0, block_rows * blocking), 0).values
+    lib = _lib.load()
+    size, guard = lib.stk_plan_bytes(block_rows, columns, nnz), 1 << 16
+    ends = {}
+    for name, b in (("given", given), ("read as", read_as)):
+        plan = torch.full((size + guard,), 0xa5, dtype=torch.uint8, device=DEV)
+        ints = [torch.full((n,), -7, dtype=torch.int32, device=DEV) for n in (block_rows + 1, nnz, nnz, columns + 1, nnz, nnz)]
+        _lib.check(lib.stk_dmoe_topology_plan(b.data_ptr(), E, blocking, block_rows, width, _lib.STK_I32, *(t.data_ptr() for t in ints),
+                                              plan.data_ptr(), size, torch.cuda.current_stream().cuda_stream))
+        assert (plan[size:] == 0xa5).all()
+        ends[name] = [t.tolist() for t in ints], _parts(plan[:size], block_rows, columns, nnz)
+    assert ends["given"] == ends["read as"]
+    assert sorted(ends["given"][0][5]) == list(range(nnz))     # every block has its place in the columns' order
