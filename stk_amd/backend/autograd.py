@@ -119,7 +119,8 @@ def _both(first, second, sp, width):
     follow(side.cuda_stream, main)              # the operands are ready on the main stream
     try:
         # (both outputs come from the main stream's memory; the side stream's use of it lies between the two waits)
-        b = second(side)
+        with backend.following(main):
+            b = second(side)
         a = first(None)
     finally:
         follow(main, side.cuda_stream)          # whatever follows on the main stream sees both results
@@ -130,12 +131,14 @@ def _wants_grad(*tensors):
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
+_transforms_active, _is_tracing = torch._C._are_functorch_transforms_active, torch._C._is_tracing
+
+
 def applies(*tensors):
     """Whether a function of this kind has to be applied, and not just its forward pass run.  Forward-mode differentiation
     and functorch's transforms see, and refuse, an applied function only; torch.jit.trace records one as one step, where
     the forward pass by itself leaves it the allocation of the result and nothing that fills it."""
-    return (_wants_grad(*tensors) or forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active()
-            or torch._C._is_tracing())
+    return _wants_grad(*tensors) or forward_ad._current_level >= 0 or _transforms_active() or _is_tracing()
 
 
 class DSD(torch.autograd.Function):

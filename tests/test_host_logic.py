@@ -327,47 +327,79 @@ def test_a_workspace_is_launched_with_before_another_thread_takes_it_over(monkey
 
 
 def _plan_streams(monkeypatch):
-    """hip_kernels on stand-ins for streams, events and the plan: a list of what happens on the streams, and use(stream) to have
-    the plan of one topology used on a stream."""
+    """hip_kernels on stand-ins for streams and plans (a plan is the pair of the stream and the capture it was built on): the
+    plans built, and use(stream, capture) for the plan that the topology has there."""
     from types import SimpleNamespace as S
     from stk_amd.backend import hip_kernels as hk
-    log = []
-
-    class Event:
-        def record(self, stream):
-            self.after = len([e for e in log if e == ("work", stream.cuda_stream)])
-            log.append(("event", stream.cuda_stream))
-
-    plan = S(record_stream=lambda stream: log.append(("lifetime", stream.cuda_stream)))
+    built, at = [], [0, 0]
     offsets, ci = torch.arange(0, 20, 4, dtype=torch.int32), torch.zeros(16, dtype=torch.int16)
     monkeypatch.setattr(hk, "_need_gpu", lambda *tensors: None)
+    monkeypatch.setattr(hk, "_stream", lambda device: at[0])
+    monkeypatch.setattr(hk, "_capture_id", lambda handle: at[1])
+    monkeypatch.setattr(hk._lib, "native", lambda: S(build_plan=lambda *args: built.append(tuple(at)) or tuple(at)))
+
+    def use(handle, capture=0):
+        at[:] = handle, capture
+        return hk.fusion_plan(offsets, ci, blocking=128)
+    return built, use
+
+
+def test_every_stream_has_a_plan_of_its_own(monkeypatch):
+    # (so that no stream waits for another one, and no plan is dropped while a stream other than its own reads it)
+    built, use = _plan_streams(monkeypatch)
+    for handle in (5, 5, 7, 5, 0, 7, 0, 5):
+        assert use(handle) == (handle, 0)
+    assert built == [(5, 0), (7, 0), (0, 0)]
+
+
+def test_the_plans_of_all_streams_are_for_the_same_directions(monkeypatch):
+    from types import SimpleNamespace as S
+    from stk_amd.backend import hip_kernels as hk
+    at, tensors = [5], [torch.arange(0, 20, 4, dtype=torch.int32), torch.zeros(16, dtype=torch.int16)] * 2
+    monkeypatch.setattr(hk, "_need_gpu", lambda *t: None)
+    monkeypatch.setattr(hk, "_stream", lambda device: at[0])
     monkeypatch.setattr(hk, "_capture_id", lambda handle: 0)
-    monkeypatch.setattr(hk._lib, "native", lambda: S(build_plan=lambda *args: plan))
-    monkeypatch.setattr(torch.cuda, "Event", Event)
-
-    def use(handle):
-        stream = S(cuda_stream=handle, wait_event=lambda event: log.append(("wait", handle, event.after)),
-                   wait_stream=lambda other: log.append(("wait", handle, len([e for e in log if e == ("work", other.cuda_stream)]))))
-        monkeypatch.setattr(hk, "_stream", lambda device: handle)
-        monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: stream)
-        assert hk.fusion_plan(offsets, ci, blocking=128) is plan
-        log.append(("work", handle))
-    return log, use
+    monkeypatch.setattr(hk._lib, "native", lambda: S(build_plan=lambda a, b, c, d, blocking: (at[0], c is not None and d is not None)))
+    assert hk.fusion_plan(*tensors) == (5, True)
+    at[0] = 7
+    assert hk.fusion_plan(*tensors[:2]) == hk.fusion_plan(*tensors) == (7, True)    # first asked for without the columns
+    tensors[3][0] = 1                                                               # modified in place: everything is built again
+    assert hk.fusion_plan(*tensors) == (7, True)
+    at[0] = 5
+    assert hk.fusion_plan(*tensors) == (5, True)
 
 
-def test_a_plan_from_another_stream_is_waited_for_and_nothing_behind_it(monkeypatch):
-    log, use = _plan_streams(monkeypatch)
-    for handle in (5, 5, 5, 7, 5, 7):
-        use(handle)
-    assert [e for e in log if e[0] == "wait"] == [("wait", 7, 0), ("wait", 7, 0)]     # for none of the work on stream 5
-    assert [e for e in log if e[0] == "event"] == [("event", 5)]
+def test_the_plans_kept_for_further_streams_are_bounded(monkeypatch):
+    from stk_amd.backend import hip_kernels as hk
+    monkeypatch.setattr(hk, "PLAN_STREAMS", 2)
+    built, use = _plan_streams(monkeypatch)
+    for handle in (1, 2, 3, 4, 4, 3, 1, 2):
+        assert use(handle) == (handle, 0)
+    assert built == [(h, 0) for h in (1, 2, 3, 4, 2)]
 
 
-def test_a_plan_outlives_its_use_on_another_stream(monkeypatch):
-    log, use = _plan_streams(monkeypatch)
-    for handle in (5, 7, 5):
-        use(handle)
-    assert [e for e in log if e[0] == "lifetime"] == [("lifetime", 7)]
+def test_plans_under_a_capture(monkeypatch):
+    built, use = _plan_streams(monkeypatch)
+    assert use(5) == (5, 0)
+    assert use(7, 9) == (5, 0)          # built before the capture: used as it is
+    assert use(7) == (7, 0)
+    built, use = _plan_streams(monkeypatch)
+    assert use(5, 9) == use(5, 9) == (5, 9) and use(7, 9) == use(7, 9) == (7, 9)
+    assert use(5) == use(5) == (5, 0)   # a plan of a capture serves that capture only
+    assert built == [(5, 9), (7, 9), (5, 0)]
+
+
+def test_a_following_stream_takes_the_plan_of_the_stream_it_follows(monkeypatch):
+    from stk_amd.backend import hip_kernels as hk
+    built, use = _plan_streams(monkeypatch)
+    assert use(5) == (5, 0) and use(0) == (0, 0)
+    for main in (0, 5):
+        with hk.following(main):
+            assert use(9) == (main, 0)
+    assert use(9) == (9, 0) and built == [(5, 0), (0, 0), (9, 0)]
+    with hk.following(6):               # nothing prepared there: built for this launch, and not for stream 6
+        assert use(9) == (9, 0)
+    assert use(6) == (6, 0) and built[3:] == [(9, 0), (6, 0)]
 
 
 def test_no_plan_is_built_ahead_where_no_product_would_find_it(monkeypatch):
