@@ -80,18 +80,20 @@ def _run_sdd(lhs, rhs, sp, side=None):
 # switch on, the second one runs on a side stream (default priority) next to the first: the workgroups of one
 # fill the compute units that the other leaves idle in its last round.
 OVERLAP_GRADIENTS = True
-# ... for products of at least this many FLOP each.  Two events to record and to wait for cost about 30 us; both gradients
-# of a dsd took, one after the other / side by side, 38 / 70 us at 4 GFLOP, 61 / 67 us at 17, 103 / 98 us at 34 and
-# 188 / 166 us at 69 (those of a dds 99 / 103 us at 34 and 182 / 187 us at 69).
-OVERLAP_FROM = 4e10
+# ... for products of at least this many FLOP each.  The change of streams and the two events cost about 50 us on the host,
+# which shorter pairs wait for.  Backward pass one after the other / side by side in us, dMoE topologies of 64 experts, evenly
+# and Zipf-distributed (8 experts at 40 and 73 GFLOP):
+#   dsd   17 GFLOP 92 / 132, 34 182 / 193, 40 110 / 135, 69 313 / 318, 73 168 / 173, 83 347 / 337, 168 464 / 456, 335 905 / 877
+#   dds   17 GFLOP 116 / 134, 34 160 / 171, 40 115 / 128, 69 269 / 279, 73 187 / 178, 83 374 / 358, 168 483 / 473, 335 857 / 843
+OVERLAP_FROM = 8e10
 _side_streams = {}
 # Both gradients of sdd (stk_dsd_dds, stk_dsd_dsd) in one launch where the operands' layouts allow it, instead of two
 # launches side by side; the same results.
 JOINT_GRADIENTS = True
-# The same for both gradients of dsd (stk_sdd_dsd).  What a joint launch gains is its tail: the short tiles of the second
-# product fill the compute units that the last round of the first leaves idle.  An sdd that runs as one workgroup per
-# compute unit walking its tile list has no such round left, and the two launches are then the shorter way (benchmark
-# topology, sdd(dy, W2^T) + dsd(h^T, dy) back to back: 462 us as two launches, 473 us as one).
+# The same for both gradients of dsd (stk_sdd_dsd), on request only: the dsd of the joint launch does without the workspace
+# that cuts its last round, so that its sums are associated differently from those of the launch by itself.  It is
+# the shorter way (backward pass, one after the other / side by side / joint: 182 / 193 / 182 us at 34 GFLOP each, 313 / 318 / 305
+# at 69, 464 / 456 / 439 at 168, 882 / 865 / 848 at 335).
 JOINT_DSD_GRADIENTS = False
 
 
