@@ -178,10 +178,10 @@ static void launch_dds(const DdsArgs& g, const PlanLists& plan, hipStream_t stre
     // eight wavefronts: 2x4... see dsd.hip; here 4x2 of 64x128 over two block columns, or 4x2 of 64x64 over one
     using Fused = TileCfg<4, 2, 2, 4, 1, 2, 2, AK, TRANS_B, BF16, KT, S, STREAM>;
     using Single = TileCfg<4, 2, 2, 2, 1, 2, 1, AK, TRANS_B, BF16, KT, S, STREAM>;
-    // four wavefronts, 128x128, for launches with little work and for 128 rows
+    // four wavefronts, 128x128, for launches with little work and where edge_pays() says so
     using Narrow = TileCfg<2, 2, 2, 2, 1, 1, 1, AK, TRANS_B, BF16, KT, S, STREAM>;
     using Reg = TileCfg<2, 2, 2, 2, 1, 1, 1, AK, TRANS_B, BF16, 64, 2>;
-    if (edge_tiles(g.m, Fused::TM) && !g.small) {
+    if (edge_pays(false, g.block_cols, g.m) && !g.small) {
       constexpr int lds = Fused::kSmemBytes > Single::kSmemBytes ? Fused::kSmemBytes : Single::kSmemBytes;
       static const int once = (set_lds_limit(&dds_fused_kernel<Fused, Single, TRANS_B>, lds), 0);
       (void)once;
@@ -201,7 +201,7 @@ static void launch_dds(const DdsArgs& g, const PlanLists& plan, hipStream_t stre
   } else {
     // 64-blocks: 4x1 wavefronts of 64x64 (tile 256x64)
     using Dma = TileCfg<4, 1, 2, 2, 1, 1, 1, AK, TRANS_B, BF16, 64, 2, STREAM>;
-    if (plan.counts && edge_tiles(g.m, 256) && !g.small) {
+    if (plan.counts && edge_groups_pay(g.block_cols, g.m) && !g.small) {
       // groups of identical block columns on eight wavefronts (4x2 of 64x128 over four block columns, 4x2 of 64x64
       // over two), then the lone columns one per four-wave workgroup; both grids are upper bounds
       using Quad = TileCfg<4, 2, 2, 4, 1, 2, 4, AK, TRANS_B, BF16, 64, 2, STREAM>;

@@ -307,7 +307,7 @@ static void launch_dsd(const DsdArgs& g, const PlanLists& plan, const TailArgs* 
     // eight wavefronts: 4x2 of 64x128 over two block rows, or 2x4 of 64x64 over one
     using Fused = TileCfg<4, 2, 2, 4, 1, 2, 2, !TRANS_A, BK, BF16, KT, S, false, STREAM>;
     using Single = TileCfg<2, 4, 2, 2, 1, 1, 2, !TRANS_A, BK, BF16, KT, S, false, STREAM>;
-    // four wavefronts, 128x128, for launches with little work and for 128 columns
+    // four wavefronts, 128x128, for launches with little work and where edge_pays() says so
     // (a K-major operand - sparse blocks that are not transposed, or a .t() view as rhs - in 64-deep K-tiles, whose rows are
     // whole 128-byte lines: on these small tiles that outweighs the deeper ring, config 2 dsd 42.5 -> 38.5 us)
     constexpr int NKT = (!TRANS_A || BK) ? 64 : KT, NS = (!TRANS_A || BK) ? 2 : S;
@@ -315,7 +315,7 @@ static void launch_dsd(const DsdArgs& g, const PlanLists& plan, const TailArgs* 
     using Reg = TileCfg<2, 2, 2, 2, 1, 1, 1, !TRANS_A, BK, BF16, 64, 2>;
     // 4x2 wavefronts of 96x64 over three block rows and 128 columns
     using Triple = TileCfg<4, 2, 3, 2, 1, 3, 1, !TRANS_A, BK, BF16, KT, S, false, STREAM>;
-    if (edge_tiles(g.n, Fused::TN) && !g.small) {
+    if (edge_pays(!TRANS_A, g.block_rows, g.n) && !g.small) {
       const int ntn = (g.n + Fused::TN - 1) / Fused::TN;
       constexpr int lds0 = Fused::kSmemBytes > Single::kSmemBytes ? Fused::kSmemBytes : Single::kSmemBytes;
       constexpr int lds = lds0 > Triple::kSmemBytes ? lds0 : Triple::kSmemBytes;
@@ -343,7 +343,7 @@ static void launch_dsd(const DsdArgs& g, const PlanLists& plan, const TailArgs* 
   } else {
     // 64-blocks: 1x4 wavefronts of 64x64 (tile 64x256)
     using Dma = TileCfg<1, 4, 2, 2, 1, 1, 1, !TRANS_A, BK, BF16, 64, 2, false, STREAM>;
-    if (plan.counts && edge_tiles(g.n, 256) && !g.small) {
+    if (plan.counts && edge_groups_pay(g.block_rows, g.n) && !g.small) {
       // groups of identical block rows on eight wavefronts (4x2 of 64x128 over four block rows, 2x4 of 64x64 over
       // two), then the lone rows one per four-wave workgroup; both grids are upper bounds
       using Quad = TileCfg<4, 2, 2, 4, 1, 4, 2, !TRANS_A, BK, BF16, 64, 2, false, STREAM>;

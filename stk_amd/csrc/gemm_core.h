@@ -924,7 +924,7 @@ __device__ __forceinline__ void epilogue(f32x16_t (&acc)[Cfg::IM][Cfg::JN], elem
 // Where the t-th tile of `tile` columns (or rows) starts when the extent, at least `tile` and a multiple of 64, is not a
 // multiple of it: the last tile is moved back to end with the extent.  The columns it shares with the one before it are
 // computed twice and written once, by the earlier tile (the epilogue's m_from / n_from = t * tile - edge_start).  Without
-// this the whole extent runs on 128 x 128 tiles of four wavefronts (128-blocks; 11264 rows over 16 experts, hidden 1152,
+// this the extent runs on 128 x 128 tiles of four wavefronts (128-blocks; 11264 rows over 16 experts, hidden 1152,
 // ffn 2944: the four dsd of a training step 417 us, of which 90 us for dsd(h, W2), now 88 us, and 210 us for the gradients
 // of the first product, now 168 us in their joint launch) or through registers with predicated loads (64-blocks; the
 // products of 7744 x 5888 with inner size 2496 and all gradients 1744 -> 1596 us).
@@ -933,6 +933,33 @@ __device__ __forceinline__ int edge_start(int t, int tile, int extent) {
   return at + tile > extent ? extent - tile : at;
 }
 inline __host__ __device__ bool edge_tiles(int64_t extent, int tile) { return extent >= tile && extent % 64 == 0; }
+// Whether a product of `lines` block rows or columns of 128 takes the wide tiles where it can; 128 x 128 tiles otherwise.  The
+// columns computed twice are a third more work at 384, a seventh at 896, and with few lines the wide tiles fill the last
+// round of the compute units badly.  Times in us on 128 x 128 / wide tiles, dMoE topologies (tokens / experts), inner size or
+// result 2944 - 4096 wide:
+//   dsd            16k / 64:  640 165 / 115, 1152 267 / 211    32k / 16:  384 88 / 105, 640 131 / 141, 896 199 / 191
+//   dsd of S^T     16k / 64:  384 90 / 108, 640 146 / 149, 1152 259 / 240    32k / 16:  640 132 / 148, 896 177 / 171
+//   dds            32k / 16:  384 92 / 106, 640 130 / 161, 896 180 / 174     16k / 64:  1152 281 / 244
+//   dds of S^T     16k / 64:  384 103 / 127, 640 184 / 203, 896 262 / 256    4k / 64:  640 107 / 120, 1152 196 / 215
+// A dsd whose tiles do not fill the units often gains at 640 already, since its last round is cut along k.
+inline bool edge_pays(bool dsd_rows, int64_t lines, int64_t extent) {
+  if (extent % 256 == 0) return extent > 0;
+  if (!edge_tiles(extent, 256)) return false;
+  const int64_t tiles = lines * (extent / 128), units = compute_units();
+  return dsd_rows ? extent >= (tiles < 4 * units ? 640 : 896) : extent >= 896 && tiles >= 8 * units;
+}
+// The same for lines of 64-blocks: groups of identical lines on wide tiles and the lone ones in a second launch, or every line
+// by itself in one launch of 256-wide tiles.  Where these fill the units a few times at most, two launches one behind the
+// other, of fewer tiles, take up to twice as long.  Times in us line by line / in groups (through registers with predicated
+// loads, as before there were moved-back tiles):
+//   dsd, 4k tokens / 64 experts (about 100 lines):   448 89 / 163 (96)    1088 149 / 183 (137)
+//   dsd, 8k / 8 (132):                               640 35 / 59 (48)     1600 69 / 94 (90)
+//   dsd, 16k / 64 (about 290):                       448 165 / 125 (185)  640 180 / 187 (197)    832 248 / 212 (280)
+//   dsd, 32k / 16 (about 520):                       640 175 / 152 (211)  1600 422 / 334 (483)
+inline bool edge_groups_pay(int64_t lines, int64_t extent) {
+  if (extent % 256 == 0) return extent > 0;
+  return edge_tiles(extent, 256) && lines * ((extent + 255) / 256) >= 4 * (int64_t)compute_units();
+}
 
 // Workgroup id -> work item, so that each of the 8 XCDs (which take workgroup
 // ids round-robin and own a private L2) receives a contiguous range of items.

@@ -23,12 +23,13 @@ def _case(rows_per_expert, width, b, dtype, hidden, seed):
     return s, operand(cols, hidden), operand(rows, hidden), operand(hidden, rows), operand(hidden, cols)
 
 
-# runs of one, two, three and more rows (lone lines, pairs, threes, fours); `many` has the work for the eight-wave tiles
-_FEW, _MANY = [1, 2, 3], [1, 2, 3, 5, 4, 0, 7, 1] * 6
+# runs of one, two, three and more rows (lone lines, pairs, threes, fours); `many` has the work for the eight-wave tiles, and
+# `more` the lines for them where block rows are walked and the extent is no multiple of 256
+_FEW, _MANY, _MORE = [1, 2, 3], [1, 2, 3, 5, 4, 0, 7, 1] * 6, [1, 2, 3, 5, 4, 0, 7, 1, 22] * 6
 
 
 @pytest.mark.parametrize("b,hidden", [(128, 128), (128, 384), (128, 640), (128, 1152), (64, 64), (64, 192), (64, 320), (64, 448), (64, 704), (64, 1216)])
-@pytest.mark.parametrize("rows,width", [(_FEW, 3), (_MANY, 23)])
+@pytest.mark.parametrize("rows,width", [(_FEW, 3), (_MANY, 23), (_MORE, 8)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_products_with_ragged_dense_extents(b, hidden, rows, width, dtype):
     s, v, a, u, w = _case(rows, width, b, dtype, hidden, hidden + width)
