@@ -44,27 +44,27 @@ class _Sparse:
         return (self.shape[1], self.shape[0]) if transposed else self.shape
 
 
-def _launch(side, product, *args, **kwargs):
-    """product(*args) with the stream `side` (None: as it is) as torch's current one: whatever the call does - copies of
-    operands, its plan and workspace, the launch - then happens on that stream."""
-    if side is None:
-        product(*args, **kwargs)
-    else:
-        with torch.cuda.stream(side):
-            product(*args, **kwargs)
-
-
+# `side`: a stream that becomes torch's current one for the call (None: as it is).  Whatever the call does - copies of operands,
+# its plan and workspace, the launch - then happens on that stream; the output is allocated before.
 def _run_dsd(sp, data, transposed, rhs, side=None):
     shape = sp.logical_shape(transposed)
     out = torch.empty((shape[0], rhs.size(1)), dtype=rhs.dtype, device=rhs.device)
-    _launch(side, backend.dsd, shape, data, *sp.meta, transposed, rhs, out)
+    if side is None:
+        backend.dsd(shape, data, *sp.meta, transposed, rhs, out)
+    else:
+        with torch.cuda.stream(side):
+            backend.dsd(shape, data, *sp.meta, transposed, rhs, out)
     return out
 
 
 def _run_dds(lhs, sp, data, transposed, side=None):
     shape = sp.logical_shape(transposed)
     out = torch.empty((lhs.size(0), shape[1]), dtype=lhs.dtype, device=lhs.device)
-    _launch(side, backend.dds, lhs, shape, data, *sp.meta, transposed, out)
+    if side is None:
+        backend.dds(lhs, shape, data, *sp.meta, transposed, out)
+    else:
+        with torch.cuda.stream(side):
+            backend.dds(lhs, shape, data, *sp.meta, transposed, out)
     return out
 
 
@@ -72,7 +72,11 @@ def _run_sdd(lhs, rhs, sp, side=None):
     out = torch.empty(sp.data.shape, dtype=lhs.dtype, device=lhs.device)
     offsets, row_indices, column_indices, _, _, block_offsets_t = sp.meta
     # visiting blocks column by column keeps the rhs panel of a block column in cache
-    _launch(side, backend.sdd, lhs, rhs, sp.shape, out, offsets, row_indices, column_indices, block_order=block_offsets_t)
+    if side is None:
+        backend.sdd(lhs, rhs, sp.shape, out, offsets, row_indices, column_indices, block_offsets_t)
+    else:
+        with torch.cuda.stream(side):
+            backend.sdd(lhs, rhs, sp.shape, out, offsets, row_indices, column_indices, block_offsets_t)
     return out
 
 

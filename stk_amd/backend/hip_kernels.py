@@ -137,15 +137,18 @@ def fusion_plan(offsets, column_indices, offsets_t=None, column_indices_t=None, 
     _need_gpu(offsets, column_indices)
     want_cols = offsets_t is not None and column_indices_t is not None
     tensors = (offsets, column_indices) + ((offsets_t, column_indices_t) if want_cols else ())
-    followed = getattr(_followed, "handle", None)
-    handle = _stream(offsets.device) if followed is None else followed
     cached = _plan_cache_get(tensors, blocking)
-    elsewhere = None
     if cached is not None:
-        built_in = cached[6]
+        handle, built_in = _stream(offsets.device), cached[6]
         if built_in == 0 and cached[3] == handle:
             return cached[1]
-        if built_in == _capture_id(_stream(offsets.device)):
+    followed = getattr(_followed, "handle", None)
+    elsewhere = None
+    if cached is not None:
+        capture = _capture_id(handle)
+        if followed is not None:
+            handle = followed
+        if built_in == capture:
             if cached[3] == handle:
                 return cached[1]
             whole = (offsets,) + cached[0]    # (the plans of all streams are for the same directions)
@@ -181,19 +184,15 @@ def _plan_for(data, offsets, column_indices, offsets_t, column_indices_t):
     return None
 
 
-def _can_be_cached(*tensors):
-    """Whether a plan of these index tensors would be found again: tensors made under inference mode keep no version counter."""
-    return not any(t.is_inference() for t in tensors)
-
-
 def prepare_plan(data, offsets, column_indices, offsets_t, column_indices_t):
     """Builds the fusion plan of a topology for both directions if there is none yet.  sdd itself needs the block rows
     only (its signature, the reference's, has no transpose metadata), so a plan built by its first call would be built
     again, with the columns, by the dsd or dds that follows on the same topology; callers that have the whole metadata
     at hand (the autograd functions) call this first and every product finds the one plan.  Nothing is built for index tensors
     whose plan no product would find."""
+    # (tensors made under inference mode keep no version counter: their plan is not cached)
     if (data.dim() == 3 and offsets.is_cuda and column_indices.numel() > 0
-            and _can_be_cached(offsets, column_indices, offsets_t, column_indices_t)):
+            and not (offsets.is_inference() or column_indices.is_inference() or offsets_t.is_inference() or column_indices_t.is_inference())):
         _plan_for(data, offsets, column_indices, offsets_t, column_indices_t)
 
 
