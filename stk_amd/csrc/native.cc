@@ -383,15 +383,17 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor, OptTensor, OptTensor> to_s
   Tensor room = at::empty({(small ? 3 : 2) * half}, x.options().dtype(int32_indices ? at::kInt : at::kShort)), room_t;
   const auto third = [&](int i) { return ptr<char>(room) + i * half * room.element_size(); };
   const Mailbox box(x.device());
+  int coordinates = STK_OK;
   if (small) {
     room_t = at::empty({columns + half}, x.options().dtype(at::kInt));
     check(stk_to_sparse_index(ptr<void>(x), rows, cols, x.stride(0), (int)blocking, bytes, mask, ptr<int32_t>(offsets), third(0), third(1),
                               ptr<int32_t>(room_t), third(2), ptr<int32_t>(room_t) + columns, idx, const_cast<int32_t*>(box.word), stream));
   } else {
     check(stk_to_sparse_count_nnz(ptr<void>(x), rows, cols, x.stride(0), (int)blocking, bytes, mask, ptr<int32_t>(offsets), const_cast<int32_t*>(box.word), stream));
-    check(stk_to_sparse_coordinates(rows, cols, (int)blocking, mask, ptr<int32_t>(offsets), third(0), third(1), idx, stream));
+    coordinates = stk_to_sparse_coordinates(rows, cols, (int)blocking, mask, ptr<int32_t>(offsets), third(0), third(1), idx, stream);
   }
-  const int64_t nnz = box.receive(stream);
+  const int64_t nnz = box.receive(stream);   // (also where a launch behind the count's failed: the word is free only once it is delivered)
+  check(coordinates);
   Tensor data = at::empty({nnz, blocking, blocking}, x.options());
   check(stk_to_sparse_gather(ptr<void>(x), rows, cols, x.stride(0), (int)blocking, bytes, third(0), third(1), nnz, idx, ptr<void>(data), stream));
   Tensor ri = room.narrow(0, 0, nnz), ci = room.narrow(0, half, nnz);
