@@ -476,3 +476,10 @@ def dsd_scatter(shape, data, offsets, column_indices, offsets_t, column_indices_
             return False
         _check_launch(status, ws)
     return True
+
+
+def dsd_scatter_few(shape, data, offsets, column_indices, rhs, row_slots, slot_rows, top_k, weights):
+    """padded_scatter(sparse @ rhs, top_k, weights) from the rows that hold a slot alone (stk_dsd_scatter_few); None, with
+    nothing launched, when the library has no such kernel for this case (the block rows hold many slots, other than 128-blocks
+    of 16-bit values)."""
+    return _lib.native().dsd_scatter_few(*shape, data, offsets, column_indices, rhs, row_slots, slot_rows, top_k, weights)

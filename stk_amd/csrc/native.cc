@@ -562,6 +562,36 @@ int dsd_scatter(int64_t m, int64_t k, const Tensor& data, const Tensor& offsets,
                          stream_of(out));
 }
 
+// padded_scatter(sparse @ rhs, top_k, weights) where the block rows hold few slots each; nothing, with nothing launched, when the
+// library has no kernel for this case
+OptTensor dsd_scatter_few(int64_t m, int64_t k, const Tensor& data, const Tensor& offsets, const Tensor& column_indices, const Tensor& rhs_,
+                          const Tensor& row_slots, const Tensor& slot_rows, int top_k, const OptTensor& weights) {
+  // (what the two calls refuse is left to them)
+  if (rhs_.dim() != 2 || k != rhs_.size(0) || top_k < 1) return {};
+  const int64_t n = rhs_.size(1), b = data.size(-1), slots = slot_rows.numel(), nnz = data.size(0);
+  for (const Tensor* t : {&rhs_, &row_slots, &slot_rows, &offsets, &column_indices})
+    if (t->device() != data.device()) return {};
+  for (const Tensor* t : {&row_slots, &slot_rows})
+    if (t->scalar_type() != at::kInt || !t->is_contiguous()) return {};
+  if (b != 128 || n % b || slots % top_k || data.scalar_type() != rhs_.scalar_type() || !data.is_contiguous() || !aligned(data) || row_slots.numel() < m ||
+      (data.scalar_type() != at::kHalf && data.scalar_type() != at::kBFloat16))
+    return {};
+  const int64_t bytes = stk_dsd_scatter_few_bytes(m, n, nnz, slots);
+  if (bytes == 0) return {};
+  const c10::DeviceGuard guard(rhs_.device());
+  const Tensor rhs = dense_operand(rhs_);
+  const OptTensor w = weights32(weights, slots);
+  const Tensor ci = index(column_indices), offs = offsets32(offsets);
+  Tensor out = at::empty({slots / top_k, n}, rhs.options());
+  const Tensor sums = at::empty({bytes / 4}, rhs.options().dtype(at::kFloat));
+  const int status = stk_dsd_scatter_few(m, k, n, ptr<void>(data), ptr<int32_t>(offs), ptr<void>(ci), ptr<void>(rhs), rhs.stride(0), rhs.stride(1),
+                                         ptr<int32_t>(row_slots), ptr<int32_t>(slot_rows), ptr<float>(w), top_k, slots / top_k, ptr<void>(out), n, nnz,
+                                         (int)b, value_dtype(rhs), index_dtype(ci.scalar_type()), ptr<void>(sums), bytes, stream_of(rhs));
+  if (status == STK_ERR_UNSUPPORTED) return {};
+  check(status);
+  return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -586,5 +616,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("padded_scatter", &padded_scatter, py::call_guard<py::gil_scoped_release>());
   m.def("padded_scatter_weight_gradient", &padded_scatter_weight_gradient, py::call_guard<py::gil_scoped_release>());
   m.def("sdd_gather", &sdd_gather, py::call_guard<py::gil_scoped_release>());
+  m.def("dsd_scatter_few", &dsd_scatter_few, py::call_guard<py::gil_scoped_release>());
   m.def("dsd_scatter", &dsd_scatter, py::call_guard<py::gil_scoped_release>());
 }

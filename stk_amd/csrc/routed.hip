@@ -3,6 +3,7 @@
 // The transfers of the lhs tiles take every row of the padded layout from the token row it is a copy of (a row
 // offset per lane, computed once per tile); the rows that are padding are computed on the first token row and set to
 // zero before the store, which is what the zero rows of a padded copy give.
+#include "few_rows.h"
 #include "sdd_tile.h"
 
 namespace stk {
@@ -86,6 +87,10 @@ extern "C" int stk_sdd_gather(const void* tokens, int64_t num_tokens, int64_t to
   g.top_k = top_k;
   g.slots = (int)(num_tokens * top_k);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (few_rows(g.slots, m / 128) && k > 0 && k % 64 == 0) {
+    sdd_few(g, problem.bk, dtype == STK_BF16, s);
+    return check_launch(who);
+  }
   if (dtype == STK_BF16) launch_gather<true>(g, problem.bk, problem.stream_rhs, s);
   else launch_gather<false>(g, problem.bk, problem.stream_rhs, s);
   return check_launch(who);

@@ -111,9 +111,14 @@ def dsd_scatter(a, rhs, route, weights=None):
     every row to its token's place (times its weight), and the padded result is never made.  The result is
     bit-identical to the two steps.  Used when nothing needs a gradient, the routing is top-1 and the library has the
     kernel (128-blocks, at least 256 columns, enough work for the eight-wavefront tiles); otherwise the two steps
-    run."""
+    run.  Where the block rows hold few tokens each, only the rows of tokens are computed, for any top_k; the result then
+    differs from the two steps' by the order of the fp32 sums."""
     from stk_amd.ops import linear_ops
     assert isinstance(a, Matrix)
+    if a.is_contiguous() and a.data.is_cuda and a.data.shape[0] > 0 and not applies(a.data, rhs, weights) and not torch.is_autocast_enabled():
+        out = hip_kernels.dsd_scatter_few(a.size(), a.data, a.offsets, a.column_indices, rhs, route.row_slots, route.slot_rows, route.top_k, weights)
+        if out is not None:
+            return out
     if route.top_k == 1 and a.is_contiguous() and a.data.is_cuda and not _wants_grad(a.data, rhs, weights):
         tokens = route.slot_rows.numel()
         out = torch.empty((tokens, rhs.shape[1]), dtype=a.dtype, device=a.data.device)
