@@ -14,7 +14,7 @@
 // the experts in order of descending R_e - and its entries can be written by any thread once the shares have been
 // added up.  Every workgroup adds them up for itself (a few hundred values from LDS); stk_build_plan, which has to find
 // the runs by comparing the lines, takes two launches and a single workgroup per direction for what follows from them.
-// 20096 rows over 64 experts of 32 block columns: 17 us for both, against 4 us for the topology and 31 us for the
+// 20096 rows over 64 experts of 32 block columns: 16.7 us for both, against 4 us for the topology and 31 us for the
 // two launches of stk_build_plan; it is latency, not bandwidth, on either side.
 #include "common.h"
 #include "plan_sim.h"
@@ -187,7 +187,7 @@ struct DmoeLds {
 };
 
 template <bool FOURS>
-__device__ __forceinline__ void dmoe_plan(const DmoeArgs& g, const DmoeLds& s, int64_t thread, int64_t threads) {
+__device__ __forceinline__ void dmoe_plan(const DmoeArgs& g, const DmoeLds& s, int group, int64_t thread, int64_t threads) {
   const int E = g.experts, width = g.width, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const DmoePlan<FOURS> plan{g, s.first};
   for (int w = tid; w < (E + 3) / 4; w += 256) {
@@ -272,7 +272,7 @@ __device__ __forceinline__ void dmoe_plan(const DmoeArgs& g, const DmoeLds& s, i
     const int e = last_not_above([&](int i) { return s.tiles[i]; }, E, (int)t);
     plan.sdd_tile(e, (int)t - s.tiles[e], g.sdd + 2 + 2 * t);
   }
-  if (blockIdx.x == 0 && tid < 10) {
+  if (group == 0 && tid < 10) {
     lists[tid] = s.count[tid];
     // entries that go to one compute die at a time: a quarter of a die's share of the list's blocks (plan.hip)
     int entries = 1;
@@ -281,53 +281,69 @@ __device__ __forceinline__ void dmoe_plan(const DmoeArgs& g, const DmoeLds& s, i
     hints[(tid >= kPlanLists ? kPlanHintBytes : 0) + kGroupHint + tid % kPlanLists] = (uint8_t)entries;
     if (tid == 0) g.sdd[0] = fits ? total_tiles : 0, g.sdd[1] = 0;
   }
-  // workgroup b simulates the launches of one direction and width of the dense operand, a wavefront per number of slices
-  static_assert(kMaxTailSlices == 4, "one wavefront per number of slices");
-  for (int item = blockIdx.x; item < 2 * kTailSliceColumns; item += gridDim.x) {
-    const bool cols = item >= kTailSliceColumns;
-    const int column = item % kTailSliceColumns, ntn = column + 1, lines = cols ? block_cols : g.block_rows;
-    const int* c = s.count + (cols ? kPlanLists : 0);
+  if (group == 0 && wave < 2) {
+    // wavefront 0 the rows, wavefront 1 the columns: do equal eighths of the lines hold about equal numbers of blocks?
+    const bool cols = wave == 1;
+    const int lines = cols ? block_cols : g.block_rows;
     uint8_t* h = hints + (cols ? kPlanHintBytes : 0);
-    const int kinds[3] = {uniform_int(c[kTallPairs] * ntn), uniform_int(c[kTallTriples] * 2 * ntn), uniform_int(c[kTallSingles] * ntn)};
-    float end = 0.f;
-    if (tail_slices_considered(kinds[0] + kinds[1] + kinds[2], g.compute_units)) {
-      WaveSim sim;
-      end = simulate_launch(sim, kinds, (float)nnz / (float)lines, g.compute_units, uniform_int(wave) + 1);
+    bool uneven = false;
+    if (lane < 8) {
+      auto offset_of = [&](int64_t line) -> int64_t {
+        if (!cols) return line * width;
+        const int e = (int)(line / width);
+        return (int64_t)s.first[e] * width + (line % width) * (e < E ? plan.rows_of(e) : 0);
+      };
+      const int64_t share = offset_of((int64_t)(lane + 1) * lines / 8) - offset_of((int64_t)lane * lines / 8);
+      uneven = share * 32 > nnz * 5;
     }
-    if (lane == 0) s.ends[wave] = end;
-    __syncthreads();
-    if (tid == 0) {
-      const float all[kMaxTailSlices] = {s.ends[0], s.ends[1], s.ends[2], s.ends[3]};
-      h[column] = (uint8_t)choose_tail_slices(all);
-    }
-    if (column == 0 && wave == 1) {
-      // do equal eighths of the lines hold about equal numbers of blocks?
-      bool uneven = false;
-      if (lane < 8) {
-        auto offset_of = [&](int64_t line) -> int64_t {
-          if (!cols) return line * width;
-          const int e = (int)(line / width);
-          return (int64_t)s.first[e] * width + (line % width) * (e < E ? plan.rows_of(e) : 0);
-        };
-        const int64_t share = offset_of((int64_t)(lane + 1) * lines / 8) - offset_of((int64_t)lane * lines / 8);
-        uneven = share * 32 > nnz * 5;
+    const uint64_t any = __ballot(uneven);
+    if (lane == 0) h[kSpreadHint] = any != 0;
+    // from which width of the dense operand on stripes beat lines
+    if (lane < 2) {
+      const int* b = s.blocks + (cols ? kPlanLists : 0);
+      const int64_t panels = lane == 0 ? (int64_t)b[kTallPairs] + b[kTallTriples] + b[kTallSingles] : (int64_t)b[kPairs] + b[kSingles];
+      const int64_t saved = panels - (cols ? g.block_rows : block_cols);
+      int from = 0;
+      if (!FOURS && saved > 0) {
+        const int64_t wide = (7 * nnz + saved - 1) / saved;
+        from = wide > 255 ? 0 : (wide < 1 ? 1 : (int)wide);
       }
-      const uint64_t any = __ballot(uneven);
-      if (lane == 0) h[kSpreadHint] = any != 0;
-      // from which width of the dense operand on stripes beat lines
-      if (lane < 2) {
-        const int* b = s.blocks + (cols ? kPlanLists : 0);
-        const int64_t panels = lane == 0 ? (int64_t)b[kTallPairs] + b[kTallTriples] + b[kTallSingles] : (int64_t)b[kPairs] + b[kSingles];
-        const int64_t saved = panels - (cols ? g.block_rows : block_cols);
-        int from = 0;
-        if (!FOURS && saved > 0) {
-          const int64_t wide = (7 * nnz + saved - 1) / saved;
-          from = wide > 255 ? 0 : (wide < 1 ? 1 : (int)wide);
-        }
-        h[kStripeHint + lane] = (uint8_t)from;
-      }
+      h[kStripeHint + lane] = (uint8_t)from;
     }
-    __syncthreads();
+  }
+}
+
+// The launches of one direction and width of the dense operand, a wavefront per number of slices.  All that they need of
+// the plan is how many groups of each height a direction has, which every wavefront adds up for itself without the order
+// of the experts and the shares in front of each.
+constexpr int kSimulations = 2 * kTailSliceColumns;
+static_assert(kMaxTailSlices == 4, "one wavefront per number of slices");
+template <bool FOURS>
+__device__ __forceinline__ void dmoe_simulation(const DmoeArgs& g, const DmoeLds& s, int item) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const DmoePlan<FOURS> plan{g, s.first};
+  const bool cols = item >= kTailSliceColumns;
+  const int column = item % kTailSliceColumns, ntn = column + 1, block_cols = g.experts * g.width, lines = cols ? block_cols : g.block_rows;
+  int pairs = 0, triples = 0, singles = 0;
+  for (int e = lane; e < g.experts; e += 64) {
+    pairs += plan.share(cols, kTallPairs, e);
+    triples += plan.share(cols, kTallTriples, e);
+    singles += plan.share(cols, kTallSingles, e);
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) pairs += __shfl_xor(pairs, d, 64), triples += __shfl_xor(triples, d, 64), singles += __shfl_xor(singles, d, 64);
+  const int kinds[3] = {uniform_int(pairs * ntn), uniform_int(triples * 2 * ntn), uniform_int(singles * ntn)};
+  float end = 0.f;
+  if (tail_slices_considered(kinds[0] + kinds[1] + kinds[2], g.compute_units)) {
+    WaveSim sim;
+    end = simulate_launch(sim, kinds, (float)((int64_t)g.block_rows * g.width) / (float)lines, g.compute_units, uniform_int(wave) + 1);
+  }
+  if (lane == 0) s.ends[wave] = end;
+  __syncthreads();
+  if (tid == 0) {
+    const float all[kMaxTailSlices] = {s.ends[0], s.ends[1], s.ends[2], s.ends[3]};
+    uint8_t* h = g.plan + plan_slices_offset(g.block_rows, block_cols) + (cols ? kPlanHintBytes : 0);
+    h[column] = (uint8_t)choose_tail_slices(all);
   }
 }
 
@@ -382,9 +398,16 @@ __global__ __launch_bounds__(256) void dmoe_plan_kernel(DmoeArgs g) {
       for (int e = 1; e <= g.experts; e++) s.first[e] = max(s.first[e], s.first[e - 1]);
     __syncthreads();
   }
-  const int64_t thread = blockIdx.x * (int64_t)256 + threadIdx.x, threads = (int64_t)gridDim.x * 256;
+  // The workgroups in front simulate, the others write the arrays and the lists beside them.  One behind the other in the same
+  // workgroups: 128 slots over 64 experts of 32 block columns 16.7 us, 15.4 like this; 16 384 slots 19.1 and 16.7 us.
+  if (blockIdx.x < kSimulations) {
+    dmoe_simulation<FOURS>(g, s, blockIdx.x);
+    return;
+  }
+  const int group = (int)blockIdx.x - kSimulations;
+  const int64_t thread = group * (int64_t)256 + threadIdx.x, threads = (int64_t)(gridDim.x - kSimulations) * 256;
   dmoe_arrays<IDX>(g, [&](int e) { return s.first[e]; }, thread, threads);
-  dmoe_plan<FOURS>(g, s, thread, threads);
+  dmoe_plan<FOURS>(g, s, group, thread, threads);
 }
 
 // Without a plan: any number of experts, the bins read where they are.
@@ -442,9 +465,7 @@ extern "C" int stk_dmoe_topology_plan(const int32_t* padded_bins, int64_t num_ex
   g.plan = plan + plan_sdd_bytes(block_rows, nnz);
   g.max_sdd_tiles = sdd_max_tiles(block_rows, nnz);
   g.compute_units = compute_units();
-  // (at least a workgroup per simulated launch)
-  const int64_t least = 2 * kTailSliceColumns;
-  const dim3 grid((unsigned)(groups < least ? least : groups < 1024 ? groups : 1024));
+  const dim3 grid((unsigned)(kSimulations + (groups < 1024 ? groups : 1024)));
   const size_t lds = DmoeLds::bytes((int)num_experts);
 #define STK_DMOE_CASE(I32, T, FOURS)                                                                    \
   if ((index_dtype == STK_I32) == I32 && (blocking == 64) == FOURS) {                                   \
