@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define STK_AMD_ABI_VERSION 19
+#define STK_AMD_ABI_VERSION 20
 
 /* status codes */
 #define STK_OK 0
@@ -549,7 +549,10 @@ int stk_padded_scatter_weight_gradient(const void* x, int64_t padded_rows, int64
  * rows to zeros).  Bit-identical to the two calls it replaces.  128-blocks only, and the token rows must span less
  * than 4 GiB; STK_ERR_UNSUPPORTED otherwise (callers then make the two calls).  No counterpart in the reference,
  * whose callers gather with their own kernels (see stk_route) in front of sdd, stk/backend/sputnik.py:206-237.
+ * stk_sdd_gather_reads_plan(m, k, num_tokens * top_k): 0 where the block rows hold few slots each, whose kernels make no use of
+ * plan, 1 elsewhere.
  */
+int stk_sdd_gather_reads_plan(int64_t m, int64_t k, int64_t slots);
 int stk_sdd_gather(const void* tokens, int64_t num_tokens, int64_t token_stride, const int32_t* row_slots, int top_k,
                    const void* rhs, int64_t rhs_stride_k, int64_t rhs_stride_n, int64_t m, int64_t k, int64_t n,
                    void* out, const int32_t* offsets, const void* row_indices, const void* column_indices, int64_t nnz,

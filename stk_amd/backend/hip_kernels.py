@@ -450,13 +450,20 @@ def padded_scatter_weight_gradient(x, grad, slot_rows, top_k):
     return _lib.native().padded_scatter_weight_gradient(x, grad, slot_rows, top_k)
 
 
+def sdd_gather_reads_plan(x, top_k, shape):
+    """Whether sdd_gather of these token rows makes use of a plan: not where the block rows hold few slots each."""
+    return x.dim() != 2 or bool(_lib.native().sdd_gather_reads_plan(shape[0], x.shape[1], x.shape[0] * top_k))
+
+
 def sdd_gather(x, row_slots, top_k, rhs, shape, out, offsets, row_indices, column_indices, activation=None):
     """out = act(sdd(padded_gather(x, row_slots, top_k), rhs)) on the topology without the padded copy of x
     (stk_sdd_gather); bit-identical to padded_gather followed by sdd_fused.  False, with nothing launched, when
     the library has no such kernel for this case (the caller then makes the two calls); True otherwise."""
     if out.shape[-1] != 128 or activation not in ACTIVATIONS or ACTIVATIONS[activation] > ACTIVATIONS["silu"] or not FUSION:
         return False
-    plan = fusion_plan(offsets, column_indices, blocking=128) if offsets is not None and out.shape[0] > 0 else None
+    plan = None
+    if offsets is not None and out.shape[0] > 0 and sdd_gather_reads_plan(x, top_k, shape):
+        plan = fusion_plan(offsets, column_indices, blocking=128)
     return _lib.native().sdd_gather(x, row_slots, top_k, rhs, *shape, out, offsets, row_indices, column_indices, plan, ACTIVATIONS[activation])
 
 

@@ -616,6 +616,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("padded_scatter", &padded_scatter, py::call_guard<py::gil_scoped_release>());
   m.def("padded_scatter_weight_gradient", &padded_scatter_weight_gradient, py::call_guard<py::gil_scoped_release>());
   m.def("sdd_gather", &sdd_gather, py::call_guard<py::gil_scoped_release>());
+  m.def("sdd_gather_reads_plan", &stk_sdd_gather_reads_plan);
   m.def("dsd_scatter_few", &dsd_scatter_few, py::call_guard<py::gil_scoped_release>());
   m.def("dsd_scatter", &dsd_scatter, py::call_guard<py::gil_scoped_release>());
 }

@@ -64,6 +64,8 @@ static void launch_gather(const SddArgs& g, bool bk, bool stream_rhs, hipStream_
 
 }  // namespace stk
 
+extern "C" int stk_sdd_gather_reads_plan(int64_t m, int64_t k, int64_t slots) { return !(stk::few_rows(slots, m / 128) && k > 0 && k % 64 == 0); }
+
 extern "C" int stk_sdd_gather(const void* tokens, int64_t num_tokens, int64_t token_stride, const int32_t* row_slots, int top_k,
                               const void* rhs, int64_t rhs_stride_k, int64_t rhs_stride_n, int64_t m, int64_t k, int64_t n,
                               void* out, const int32_t* offsets, const void* row_indices, const void* column_indices, int64_t nnz,
@@ -87,7 +89,7 @@ extern "C" int stk_sdd_gather(const void* tokens, int64_t num_tokens, int64_t to
   g.top_k = top_k;
   g.slots = (int)(num_tokens * top_k);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (few_rows(g.slots, m / 128) && k > 0 && k % 64 == 0) {
+  if (!stk_sdd_gather_reads_plan(m, k, g.slots)) {
     sdd_few(g, problem.bk, dtype == STK_BF16, s);
     return check_launch(who);
   }

@@ -98,7 +98,8 @@ def gather_sdd(x, route, rhs, topo, activation=None):
     if x.is_cuda and not _wants_grad(x, rhs):
         out = torch.empty_like(topo.data)
         # (one plan for both directions: the product that follows on the same topology walks it the other way)
-        hip_kernels.prepare_plan(topo.data, topo.offsets, topo.column_indices, topo.offsets_t, topo.column_indices_t)
+        if hip_kernels.sdd_gather_reads_plan(x, route.top_k, topo.size()):
+            hip_kernels.prepare_plan(topo.data, topo.offsets, topo.column_indices, topo.offsets_t, topo.column_indices_t)
         if hip_kernels.sdd_gather(x, route.row_slots, route.top_k, rhs, topo.size(), out, topo.offsets, topo.row_indices, topo.column_indices,
                                   activation):
             return Matrix(topo.size(), out, topo.row_indices, topo.column_indices, topo.offsets,

@@ -98,3 +98,20 @@ def test_dsd_scatter_few_with_columns_that_are_no_multiple_of_128():
     want = (dense.double() @ w2.double())[r.slot_rows.long()]
     # one rounding of the result, fp32 sums
     assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
+
+
+@pytest.mark.parametrize("counts,reads", ((COUNTS[0], False), ((100, 128, 90, 128), True)))
+def test_a_plan_is_built_for_the_gathered_product_only_where_it_is_read(monkeypatch, counts, reads):
+    # (under inference mode, which caches none, every product that asks for a plan builds one)
+    built = []
+    plan = hip_kernels.fusion_plan
+    monkeypatch.setattr(hip_kernels, "fusion_plan", lambda *a, **k: built.append(1) or plan(*a, **k))
+    with torch.inference_mode():
+        x, _, r, topo, w1, _ = _layer(counts, 128, 1280, 1, torch.bfloat16)
+        stk.ops.gather_sdd(x, r, w1, topo)
+    assert bool(built) == reads
+    with torch.no_grad():
+        x, _, r, topo, w1, _ = _layer(counts, 128, 1280, 1, torch.bfloat16)
+        del topo.offsets._stk_plan, built[:]
+        stk.ops.gather_sdd(x, r, w1, topo)
+    assert bool(built) == reads
