@@ -391,11 +391,12 @@ static void launch_dsd_scatter(const DsdArgs& g, const PlanLists& plan, const Ta
 
 // The sliced last round of a dsd launch, if this one gets one: for launches of a few rounds of tiles (with many
 // rounds the last one matters little and the plain kernel is used as it is); the plan says whether and how the last
-// round is cut.  STK_OK with *sliced set or cleared.
-static int tail_of(const char* who, const DsdArgs& g, int64_t n, int64_t nnz, int blocking, const uint8_t* plan, void* workspace,
+// round is cut.  STK_OK with *sliced set or cleared.  Only on the extents on which stk_dsd takes the wide tiles: the scattered
+// product, which takes them on others too, leaves the sums whole where stk_dsd does.
+static int tail_of(const char* who, const DsdArgs& g, bool ta, int64_t n, int64_t nnz, int blocking, const uint8_t* plan, void* workspace,
                    int64_t workspace_bytes, TailArgs* tail, bool* sliced) {
   *sliced = false;
-  if (!(workspace && plan && blocking == 128 && edge_tiles(n, 256) && nnz > 0 && !g.small)) return STK_OK;
+  if (!(workspace && plan && blocking == 128 && edge_pays(!ta, g.block_rows, n) && nnz > 0 && !g.small)) return STK_OK;
   const int workgroups = compute_units();
   if (workgroups <= 0 || (int64_t)g.block_rows * (n / 128) / 3 >= 8 * (int64_t)workgroups) return STK_OK;
   if (reinterpret_cast<uintptr_t>(workspace) & 255u) return fail(STK_ERR_WORKSPACE, "%s: the workspace must be 256-byte aligned", who);
@@ -499,7 +500,7 @@ extern "C" int stk_dsd(int64_t m, int64_t k, int64_t n,
   const bool ta = problem.ta, bk = problem.bk, stream_rhs = problem.stream_rhs;
   TailArgs tail{};
   bool sliced = false;
-  const int tail_rc = tail_of("stk_dsd", g, n, nnz, blocking, plan, workspace, workspace_bytes, &tail, &sliced);
+  const int tail_rc = tail_of("stk_dsd", g, ta, n, nnz, blocking, plan, workspace, workspace_bytes, &tail, &sliced);
   if (tail_rc != STK_OK) return tail_rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define STK_DSD_CASE(BF, BLK, TA, BK)                                                          \
@@ -537,7 +538,7 @@ extern "C" int stk_dsd_scatter(int64_t m, int64_t k, int64_t n, const void* data
   g.out_rows = (int)num_tokens;
   TailArgs tail{};
   bool sliced = false;
-  const int tail_rc = tail_of(who, g, n, nnz, blocking, plan, workspace, workspace_bytes, &tail, &sliced);
+  const int tail_rc = tail_of(who, g, false, n, nnz, blocking, plan, workspace, workspace_bytes, &tail, &sliced);
   if (tail_rc != STK_OK) return tail_rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const TailArgs* t = sliced ? &tail : nullptr;

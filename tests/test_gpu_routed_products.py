@@ -143,6 +143,17 @@ def test_dsd_scatter_is_dsd_then_scatter(tokens, hidden, experts, ffn, dtype, we
     hip_kernels.release_workspaces()
 
 
+@pytest.mark.parametrize("hidden", (384, 512))
+def test_dsd_scatter_cuts_its_last_round_where_dsd_does(hidden):
+    # 384 columns: dsd runs on 128 x 128 tiles and cuts none of them, the scattered product has wide tiles only
+    x, r, topo, _, w2 = _layer(8000, hidden, 16, 8192, 1, torch.bfloat16, 3)
+    h = stk.Matrix(topo.size(), torch.randn(topo.data.shape, device=DEV).to(torch.bfloat16), topo.row_indices, topo.column_indices, topo.offsets,
+                   topo.column_indices_t, topo.offsets_t, topo.block_offsets_t)
+    out = torch.empty(8000, hidden, dtype=torch.bfloat16, device=DEV)
+    assert hip_kernels.dsd_scatter(h.size(), h.data, h.offsets, h.column_indices, h.offsets_t, h.column_indices_t, w2, r.row_slots, None, out)
+    assert _same_bits(out, stk.ops.padded_scatter(stk.ops.dsd(h, w2), r))
+
+
 def test_dsd_scatter_falls_back_where_it_has_no_kernel():
     # little work (four-wavefront tiles in stk_dsd), top-2, a transposed operand, gradients: the two steps run
     x, r, topo, w1, w2 = _layer(700, 256, 4, 256, 1, torch.bfloat16, 2)
