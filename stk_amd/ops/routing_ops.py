@@ -84,10 +84,6 @@ def padded_scatter(x, route, weights=None):
     return _PaddedScatter.apply(x, route, weights)
 
 
-def _wants_grad(*tensors):
-    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
-
-
 def gather_sdd(x, route, rhs, topo, activation=None):
     """stk.ops.sdd_fused(padded_gather(x, route), rhs, topo, activation) in one launch: the sampled product reads the
     token rows where they lie, and the padded copy of x is never made.  The result is bit-identical to the two steps.
@@ -95,7 +91,7 @@ def gather_sdd(x, route, rhs, topo, activation=None):
     has the kernel (128-blocks); otherwise the two steps run."""
     from stk_amd.ops import linear_ops
     assert isinstance(topo, Matrix) and topo.is_contiguous()
-    if x.is_cuda and not _wants_grad(x, rhs):
+    if x.is_cuda and not applies(x, rhs):
         out = torch.empty_like(topo.data)
         # (one plan for both directions: the product that follows on the same topology walks it the other way)
         if hip_kernels.sdd_gather_reads_plan(x, route.top_k, topo.size()):
@@ -120,7 +116,7 @@ def dsd_scatter(a, rhs, route, weights=None):
         out = hip_kernels.dsd_scatter_few(a.size(), a.data, a.offsets, a.column_indices, rhs, route.row_slots, route.slot_rows, route.top_k, weights)
         if out is not None:
             return out
-    if route.top_k == 1 and a.is_contiguous() and a.data.is_cuda and not _wants_grad(a.data, rhs, weights):
+    if route.top_k == 1 and a.is_contiguous() and a.data.is_cuda and not applies(a.data, rhs, weights):
         tokens = route.slot_rows.numel()
         out = torch.empty((tokens, rhs.shape[1]), dtype=a.dtype, device=a.data.device)
         if hip_kernels.dsd_scatter(a.size(), a.data, a.offsets, a.column_indices, a.offsets_t, a.column_indices_t, rhs,

@@ -110,6 +110,22 @@ def test_sdd_gather_refuses_what_it_has_no_kernel_for():
     assert _same_bits(gx, x.grad) and _same_bits(gw, w1.grad)
 
 
+@pytest.mark.parametrize("tokens,hidden,experts,ffn", ((30, 256, 4, 256), (8192, 1024, 8, 2560)))
+def test_forward_mode_and_transforms_are_refused_as_by_the_two_steps(tokens, hidden, experts, ffn):
+    # a tangent that the kernels do not carry on is not dropped without a word
+    from torch.autograd import forward_ad
+    x, r, topo, w1, w2 = _layer(tokens, hidden, experts, ffn, 1, torch.bfloat16, 2)
+    h = stk.ops.sdd(stk.ops.padded_gather(x, r), w1, topo)
+    weights = torch.rand(tokens, 1, device=DEV)
+    calls = ((lambda t: stk.ops.gather_sdd(t, r, w1, topo).data, x), (lambda t: stk.ops.gather_sdd(x, r, t, topo).data, w1),
+             (lambda t: stk.ops.dsd_scatter(h, t, r), w2), (lambda t: stk.ops.dsd_scatter(h, w2, r, t), weights))
+    for call, t in calls:
+        with forward_ad.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
+            call(forward_ad.make_dual(t, torch.ones_like(t)))
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(call)(t[None])
+
+
 # (tokens, hidden, experts, ffn per expert): enough blocks x columns for the eight-wavefront tiles
 SCATTER_SIZES = (
     (8192, 1024, 8, 2560),
