@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define STK_AMD_ABI_VERSION 20
+#define STK_AMD_ABI_VERSION 21
 
 /* status codes */
 #define STK_OK 0
@@ -583,8 +583,7 @@ int stk_dsd_scatter(int64_t m, int64_t k, int64_t n, const void* data, const int
  * up per token.
  *   out[t] = sum over j of (weights[s] *) round((S * rhs)[slot_rows[s]]),  s = t * top_k + j
  * with stk_padded_scatter's products, order and rounding; row_slots and slot_rows are those of one routing (stk_route), and
- * slots without a row in [0, m) are left out.  The sums are cut into slices along k, whose number depends on m, n and nnz
- * only: results are repeatable, and differ from the two calls by the order of the fp32 sums.
+ * slots without a row in [0, m) are left out.  Bit-identical to stk_dsd without a workspace and stk_padded_scatter.
  * stk_dsd_scatter_few_bytes(m, n, nnz, num_tokens * top_k) is the size of the workspace (16-byte aligned, nothing in it is
  * read before it is written), 0 where this call is not for the sizes: then, and for other than 128-blocks,
  * STK_ERR_UNSUPPORTED (callers make the two calls).  No counterpart in the reference (see stk_route).
@@ -595,6 +594,17 @@ int stk_dsd_scatter_few(int64_t m, int64_t k, int64_t n, const void* data, const
                         const int32_t* slot_rows, const float* weights, int top_k, int64_t num_tokens, void* out,
                         int64_t out_stride_m, int64_t nnz, int blocking, int dtype, int index_dtype, void* workspace,
                         int64_t workspace_bytes, stk_stream_t stream);
+/*
+ * The same with the bits of a stk_dsd that gets a workspace of dsd_workspace_bytes (none is needed here) and the plan `plan`, built
+ * with the block columns: where that one cuts a tile of its last round into slices along k, the sums are cut alike.
+ * stk_dsd_cuts(m, n, nnz, dsd_workspace_bytes): whether it may; where it is 0 the plan is not read.
+ */
+int stk_dsd_scatter_few_as_cut(int64_t m, int64_t k, int64_t n, const void* data, const int32_t* offsets, const void* column_indices,
+                               const void* rhs, int64_t rhs_stride_k, int64_t rhs_stride_n, const int32_t* row_slots,
+                               const int32_t* slot_rows, const float* weights, int top_k, int64_t num_tokens, void* out,
+                               int64_t out_stride_m, int64_t nnz, int blocking, int dtype, int index_dtype, void* workspace,
+                               int64_t workspace_bytes, const uint8_t* plan, int64_t dsd_workspace_bytes, stk_stream_t stream);
+int stk_dsd_cuts(int64_t m, int64_t n, int64_t nnz, int64_t workspace_bytes);
 
 #ifdef __cplusplus
 }

@@ -12,7 +12,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), "libstk_amd.so")
 NATIVE_PATH = os.path.join(os.path.dirname(_HERE), "_native.so")
 
-ABI_VERSION = 20
+ABI_VERSION = 21
 STK_OK, STK_ERR_DIMS, STK_ERR_UNSUPPORTED, STK_ERR_HIP, STK_ERR_WORKSPACE = 0, 1, 2, 3, 4
 STK_F16, STK_BF16, STK_F32 = 0, 1, 2
 STK_I16, STK_I32 = 0, 1
@@ -66,7 +66,9 @@ SIGNATURES = {
     "stk_sdd_gather": (_int, [_p, _i64, _i64, _p, _int, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _i64, _int, _int, _int, _p, _int, _p]),
     "stk_sdd_gather_reads_plan": (_int, [_i64, _i64, _i64]),
     "stk_dsd_scatter_few_bytes": (_i64, [_i64, _i64, _i64, _i64]),
+    "stk_dsd_cuts": (_int, [_i64, _i64, _i64, _i64]),
     "stk_dsd_scatter_few": (_int, [_i64, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _p, _p, _p, _int, _i64, _p, _i64, _i64, _int, _int, _int, _p, _i64, _p]),
+    "stk_dsd_scatter_few_as_cut": (_int, [_i64, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _p, _p, _p, _int, _i64, _p, _i64, _i64, _int, _int, _int, _p, _i64, _p, _i64, _p]),
     "stk_dsd_scatter": (_int, [_i64, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _p, _p, _i64, _p, _i64, _i64, _int, _int, _int, _p, _p, _i64, _p]),
 }
 

@@ -485,8 +485,18 @@ def dsd_scatter(shape, data, offsets, column_indices, offsets_t, column_indices_
     return True
 
 
-def dsd_scatter_few(shape, data, offsets, column_indices, rhs, row_slots, slot_rows, top_k, weights):
-    """padded_scatter(sparse @ rhs, top_k, weights) from the rows that hold a slot alone (stk_dsd_scatter_few); None, with
-    nothing launched, when the library has no such kernel for this case (the block rows hold many slots, other than 128-blocks
-    of 16-bit values)."""
-    return _lib.native().dsd_scatter_few(*shape, data, offsets, column_indices, rhs, row_slots, slot_rows, top_k, weights)
+def dsd_scatter_few(shape, data, offsets, column_indices, rhs, row_slots, slot_rows, top_k, weights, offsets_t=None, column_indices_t=None):
+    """padded_scatter(sparse @ rhs, top_k, weights) from the rows that hold a slot alone (stk_dsd_scatter_few_as_cut); bit-identical
+    to dsd followed by padded_scatter (without the transpose metadata: to a dsd without its workspace).  None, with nothing
+    launched, when the library has no such kernel for this case (the block rows hold many slots, other than 128-blocks of 16-bit
+    values; the caller then makes the two calls)."""
+    if data.shape[-1] != 128 or data.dtype == torch.float32 or not FUSION or rhs.dim() != 2:
+        return None
+    m, k = shape
+    # the workspace of that dsd, if it may cut its last round: the plan then says where, and the sums here are cut alike
+    partial_tiles = DSD_WORKSPACE_SLOTS if SLICE_LAST_ROUND and offsets_t is not None else 0
+    dsd_workspace = _lib.native().dsd_scatter_few_case(m, rhs.shape[1], data.shape[0], slot_rows.numel(), partial_tiles)
+    if dsd_workspace < 0:
+        return None
+    plan = fusion_plan(offsets, column_indices, offsets_t, column_indices_t, 128) if dsd_workspace else None
+    return _lib.native().dsd_scatter_few(m, k, data, offsets, column_indices, rhs, row_slots, slot_rows, top_k, weights, plan, dsd_workspace)

@@ -229,58 +229,23 @@ __global__ __launch_bounds__(512, 2) void dsd_sliced_kernel(DsdArgs g, PlanLists
   extern __shared__ __align__(16) char smem[];
   __shared__ int flag;
   static_assert(Fused::TN == Single::TN && Fused::TN == 2 * Triple::TN, "same column tiling");
-  const int ntn = (g.n + Fused::TN - 1) / Fused::TN, narrow = (g.n + Triple::TN - 1) / Triple::TN;
-  const int pair_tiles = const_ints(plan.counts)[kTallPairs] * ntn;
-  const int triple_tiles = const_ints(plan.counts)[kTallTriples] * narrow;
-  const int single_tiles = const_ints(plan.counts)[kTallSingles] * ntn;
-  const int tiles = pair_tiles + triple_tiles + single_tiles;
-  int slices = uniform(plan.hints[(ntn < kTailSliceColumns ? ntn : kTailSliceColumns) - 1]);
-  const bool spread = (const_ints(plan.hints)[kSpreadHint / 4] & 0xff) != 0;
-  if (slices < 1 || slices > kMaxTailSlices) slices = 1;
-  // whole rounds first; the rest (all of it when there is less than one round) is the last round
-  int whole = (slices > 1 && tiles > 0) ? (tiles - 1) / t.workgroups * t.workgroups : tiles;
-  if (slices > 1 && (tiles - whole) * slices > t.capacity) {
-    // a workspace smaller than the plan would like: fewer slices, or none
-    slices = t.capacity / (tiles - whole);
-    if (slices < 2) slices = 1, whole = tiles;
-  }
-  int item = blockIdx.x, slice = 0;
-  if (item >= whole) {
+  static_assert(Fused::TN == kTailTile, "the tiles of tail_round()");
+  const TailRound round = tail_round(plan, g.n, t.workgroups, t.capacity);
+  int item = blockIdx.x, slice = 0, slices = 1;
+  if (item >= round.whole) {
     // last round: blocks of kTailBlock tiles, slice by slice, so that neighbouring tiles (which share
     // the sparse operand in the L2 of their compute die) work on the same stretch of k at the same time
-    const int j = item - whole, r = j % (kTailBlock * slices);
+    slices = round.slices;
+    const int j = item - round.whole, r = j % (kTailBlock * slices);
     slice = r / kTailBlock;
-    item = whole + j / (kTailBlock * slices) * kTailBlock + r % kTailBlock;
-    if (item >= tiles) return;
-  } else {
-    slices = 1;
+    item = round.whole + j / (kTailBlock * slices) * kTailBlock + r % kTailBlock;
+    if (item >= round.tiles) return;
   }
-  const int ordinal = item - whole;  // among the tiles of the last round: 0 .. workgroups - 1
-  if (item < pair_tiles) {
-    const int i = xcd_share(item, pair_tiles, spread);
-    dsd_slice<Fused, TRANS_A, 2, SCATTER>(g, t, const_ints(plan.list(kTallPairs))[i / ntn], i % ntn, slice, slices, ordinal, smem, &flag);
-    return;
-  }
-  item -= pair_tiles;
-  if (item < triple_tiles) {
-    const int i = xcd_share(item, triple_tiles, spread);
-    dsd_slice<Triple, TRANS_A, 3, SCATTER>(g, t, const_ints(plan.list(kTallTriples))[i / narrow], i % narrow, slice, slices, ordinal, smem, &flag);
-    return;
-  }
-  item -= triple_tiles;
-  // (in order of length: no contiguous shares.)  When the plan says that the lone lines share little, the lines whose tiles all
-  // lie in the whole rounds, where a workgroup's id is its item, are dealt by stripes of the dense operand (xcd_lines; the
-  // list must start at a multiple of the eight dies, so that every line's tiles stay among themselves); what is left
-  // of the list is taken in order.
-  const int from = (plan.stripe_from(true) + 1) >> 1, lead = pair_tiles + triple_tiles;
-  int i;
-  if (from != 0 && ntn >= from && !(ntn & 7) && !(lead & 7)) {
-    const int striped = whole > lead ? (whole - lead) / ntn * ntn : 0;
-    i = item < striped ? xcd_lines(item, striped, ntn, from) : item;
-  } else {
-    i = xcd_grouped(item, single_tiles);
-  }
-  dsd_slice<Single, TRANS_A, 1, SCATTER>(g, t, const_ints(plan.list(kTallSingles))[i / ntn], i % ntn, slice, slices, ordinal, smem, &flag);
+  const int ordinal = item - round.whole;  // among the tiles of the last round: 0 .. workgroups - 1
+  const LineTile tile = tail_round_tile(plan, g.n, round, item);
+  if (tile.lines == 2) dsd_slice<Fused, TRANS_A, 2, SCATTER>(g, t, tile.line, tile.column, slice, slices, ordinal, smem, &flag);
+  else if (tile.lines == 3) dsd_slice<Triple, TRANS_A, 3, SCATTER>(g, t, tile.line, tile.column, slice, slices, ordinal, smem, &flag);
+  else dsd_slice<Single, TRANS_A, 1, SCATTER>(g, t, tile.line, tile.column, slice, slices, ordinal, smem, &flag);
 }
 
 template <class Cfg, int BLK, bool TRANS_A, bool FULL>
@@ -389,24 +354,20 @@ static void launch_dsd_scatter(const DsdArgs& g, const PlanLists& plan, const Ta
   hipLaunchKernelGGL((dsd_fused_kernel<Fused, Triple, Single, false, true>), dim3(g.block_rows * ((g.n + Fused::TN - 1) / Fused::TN)), dim3(512), lds, stream, g, plan);
 }
 
-// The sliced last round of a dsd launch, if this one gets one: for launches of a few rounds of tiles (with many
-// rounds the last one matters little and the plain kernel is used as it is); the plan says whether and how the last
-// round is cut.  STK_OK with *sliced set or cleared.  Only on the extents on which stk_dsd takes the wide tiles: the scattered
-// product, which takes them on others too, leaves the sums whole where stk_dsd does.
+// The sliced last round of a dsd launch, if this one gets one (tail_capacity()); the plan says whether and how the last
+// round is cut.  STK_OK with *sliced set or cleared.
 static int tail_of(const char* who, const DsdArgs& g, bool ta, int64_t n, int64_t nnz, int blocking, const uint8_t* plan, void* workspace,
                    int64_t workspace_bytes, TailArgs* tail, bool* sliced) {
   *sliced = false;
-  if (!(workspace && plan && blocking == 128 && edge_pays(!ta, g.block_rows, n) && nnz > 0 && !g.small)) return STK_OK;
-  const int workgroups = compute_units();
-  if (workgroups <= 0 || (int64_t)g.block_rows * (n / 128) / 3 >= 8 * (int64_t)workgroups) return STK_OK;
+  if (!(workspace && plan && blocking == 128)) return STK_OK;
+  const int capacity = tail_capacity(ta, g.block_rows, n, nnz, workspace_bytes);
+  if (capacity == 0) return STK_OK;
   if (reinterpret_cast<uintptr_t>(workspace) & 255u) return fail(STK_ERR_WORKSPACE, "%s: the workspace must be 256-byte aligned", who);
-  const int64_t capacity = (workspace_bytes - (int64_t)tail_counter_bytes(workgroups)) / (int64_t)(sizeof(float) * kSlotFloats);
-  if (capacity < 2) return STK_OK;
   *sliced = true;
   tail->counters = static_cast<int32_t*>(workspace);
-  tail->slots = reinterpret_cast<float*>(static_cast<char*>(workspace) + tail_counter_bytes(workgroups));
-  tail->workgroups = workgroups;
-  tail->capacity = (int)(capacity < kMaxTailSlices * (int64_t)workgroups ? capacity : kMaxTailSlices * (int64_t)workgroups);
+  tail->workgroups = compute_units();
+  tail->slots = reinterpret_cast<float*>(static_cast<char*>(workspace) + tail_counter_bytes(tail->workgroups));
+  tail->capacity = capacity;
   return STK_OK;
 }
 

@@ -143,4 +143,73 @@ __device__ __forceinline__ bool dsd_plan_tile(const DsdArgs& g, const PlanLists&
   return false;
 }
 
+// The last round of a dsd launch over the plan's lists whose tiles fill the compute units a few times only (dsd.hip): the
+// tiles from `whole` on, in the order of the lists, are computed in `slices` slices along k, each an fp32 sum of its own; the
+// partial sums are then added up in the order of the slices.  workgroups: tiles per round; capacity: partial tiles that the
+// workspace holds, the round is cut no further than fits.
+struct TailRound {
+  int pair_tiles, triple_tiles, single_tiles, tiles, whole, slices;
+  bool spread;
+};
+constexpr int kTailTile = 256;   // columns of a tile of pairs and of lone rows; threes take half as many
+__device__ __forceinline__ TailRound tail_round(const PlanLists& plan, int n, int workgroups, int capacity) {
+  TailRound t;
+  const int ntn = (n + kTailTile - 1) / kTailTile, narrow = (n + kTailTile / 2 - 1) / (kTailTile / 2);
+  t.pair_tiles = const_ints(plan.counts)[kTallPairs] * ntn;
+  t.triple_tiles = const_ints(plan.counts)[kTallTriples] * narrow;
+  t.single_tiles = const_ints(plan.counts)[kTallSingles] * ntn;
+  t.tiles = t.pair_tiles + t.triple_tiles + t.single_tiles;
+  t.slices = uniform(plan.hints[(ntn < kTailSliceColumns ? ntn : kTailSliceColumns) - 1]);
+  t.spread = (const_ints(plan.hints)[kSpreadHint / 4] & 0xff) != 0;
+  if (t.slices < 1 || t.slices > kMaxTailSlices) t.slices = 1;
+  // whole rounds first; the rest (all of it when there is less than one round) is the last round
+  t.whole = (t.slices > 1 && t.tiles > 0) ? (t.tiles - 1) / workgroups * workgroups : t.tiles;
+  if (t.slices > 1 && (t.tiles - t.whole) * t.slices > capacity) {
+    // a workspace smaller than the plan would like: fewer slices, or none
+    t.slices = capacity / (t.tiles - t.whole);
+    if (t.slices < 2) t.slices = 1, t.whole = t.tiles;
+  }
+  return t;
+}
+// Tile `item` of such a launch: `lines` block rows from `line` on, the column-th tile of columns.
+struct LineTile {
+  int lines, line, column;
+};
+__device__ __forceinline__ LineTile tail_round_tile(const PlanLists& plan, int n, const TailRound& t, int item) {
+  const int ntn = (n + kTailTile - 1) / kTailTile, narrow = (n + kTailTile / 2 - 1) / (kTailTile / 2);
+  if (item < t.pair_tiles) {
+    const int i = xcd_share(item, t.pair_tiles, t.spread);
+    return {2, const_ints(plan.list(kTallPairs))[i / ntn], i % ntn};
+  }
+  item -= t.pair_tiles;
+  if (item < t.triple_tiles) {
+    const int i = xcd_share(item, t.triple_tiles, t.spread);
+    return {3, const_ints(plan.list(kTallTriples))[i / narrow], i % narrow};
+  }
+  item -= t.triple_tiles;
+  // (in order of length: no contiguous shares.)  When the plan says that the lone lines share little, the lines whose tiles all
+  // lie in the whole rounds, where a workgroup's id is its item, are dealt by stripes of the dense operand (xcd_lines; the
+  // list must start at a multiple of the eight dies, so that every line's tiles stay among themselves); what is left
+  // of the list is taken in order.
+  const int from = (plan.stripe_from(true) + 1) >> 1, lead = t.pair_tiles + t.triple_tiles;
+  int i;
+  if (from != 0 && ntn >= from && !(ntn & 7) && !(lead & 7)) {
+    const int striped = t.whole > lead ? (t.whole - lead) / ntn * ntn : 0;
+    i = item < striped ? xcd_lines(item, lead + item, striped, ntn, from) : item;
+  } else {
+    i = xcd_grouped(item, t.single_tiles);
+  }
+  return {1, const_ints(plan.list(kTallSingles))[i / ntn], i % ntn};
+}
+
+// Whether a dsd of `lines` block rows of 128 (of op(S): ta, transposed) with this workspace may cut its last round, its partial
+// tiles then `capacity` (common to every launch that has to give the bits of that dsd).
+inline int tail_capacity(bool ta, int64_t lines, int64_t n, int64_t nnz, int64_t workspace_bytes) {
+  const int64_t units = compute_units();
+  // (with many rounds the last one matters little and the plain kernel is used as it is)
+  if (units <= 0 || nnz <= 0 || !edge_pays(!ta, lines, n) || stk_dsd_is_small(nnz, n) || lines * (n / 128) / 3 >= 8 * units) return 0;
+  const int64_t room = (workspace_bytes - stk_dsd_workspace_counter_bytes()) / stk_dsd_workspace_slot_bytes();
+  return room < 2 ? 0 : (int)(room < kMaxTailSlices * units ? room : kMaxTailSlices * units);
+}
+
 }  // namespace stk

@@ -562,10 +562,19 @@ int dsd_scatter(int64_t m, int64_t k, const Tensor& data, const Tensor& offsets,
                          stream_of(out));
 }
 
+// Whether dsd_scatter_few is for these sizes (-1: no), and the size of the workspace, with room for `partial_tiles`, of the
+// stk_dsd whose bits it gives, 0 if that one cuts no tile.
+int64_t dsd_scatter_few_case(int64_t m, int64_t n, int64_t nnz, int64_t slots, int64_t partial_tiles) {
+  if (stk_dsd_scatter_few_bytes(m, n, nnz, slots) == 0) return -1;
+  const int64_t bytes = partial_tiles > 0 ? stk_dsd_workspace_counter_bytes() + partial_tiles * stk_dsd_workspace_slot_bytes() : 0;
+  return stk_dsd_cuts(m, n, nnz, bytes) ? bytes : 0;
+}
+
 // padded_scatter(sparse @ rhs, top_k, weights) where the block rows hold few slots each; nothing, with nothing launched, when the
 // library has no kernel for this case
 OptTensor dsd_scatter_few(int64_t m, int64_t k, const Tensor& data, const Tensor& offsets, const Tensor& column_indices, const Tensor& rhs_,
-                          const Tensor& row_slots, const Tensor& slot_rows, int top_k, const OptTensor& weights) {
+                          const Tensor& row_slots, const Tensor& slot_rows, int top_k, const OptTensor& weights, const OptTensor& plan,
+                          int64_t dsd_workspace_bytes) {
   // (what the two calls refuse is left to them)
   if (rhs_.dim() != 2 || k != rhs_.size(0) || top_k < 1) return {};
   const int64_t n = rhs_.size(1), b = data.size(-1), slots = slot_rows.numel(), nnz = data.size(0);
@@ -584,9 +593,10 @@ OptTensor dsd_scatter_few(int64_t m, int64_t k, const Tensor& data, const Tensor
   const Tensor ci = index(column_indices), offs = offsets32(offsets);
   Tensor out = at::empty({slots / top_k, n}, rhs.options());
   const Tensor sums = at::empty({bytes / 4}, rhs.options().dtype(at::kFloat));
-  const int status = stk_dsd_scatter_few(m, k, n, ptr<void>(data), ptr<int32_t>(offs), ptr<void>(ci), ptr<void>(rhs), rhs.stride(0), rhs.stride(1),
+  const int status = stk_dsd_scatter_few_as_cut(m, k, n, ptr<void>(data), ptr<int32_t>(offs), ptr<void>(ci), ptr<void>(rhs), rhs.stride(0), rhs.stride(1),
                                          ptr<int32_t>(row_slots), ptr<int32_t>(slot_rows), ptr<float>(w), top_k, slots / top_k, ptr<void>(out), n, nnz,
-                                         (int)b, value_dtype(rhs), index_dtype(ci.scalar_type()), ptr<void>(sums), bytes, stream_of(rhs));
+                                         (int)b, value_dtype(rhs), index_dtype(ci.scalar_type()), ptr<void>(sums), bytes,
+                                                ptr<uint8_t>(plan), dsd_workspace_bytes, stream_of(rhs));
   if (status == STK_ERR_UNSUPPORTED) return {};
   check(status);
   return out;
@@ -617,6 +627,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("padded_scatter_weight_gradient", &padded_scatter_weight_gradient, py::call_guard<py::gil_scoped_release>());
   m.def("sdd_gather", &sdd_gather, py::call_guard<py::gil_scoped_release>());
   m.def("sdd_gather_reads_plan", &stk_sdd_gather_reads_plan);
+  m.def("dsd_scatter_few_case", &dsd_scatter_few_case);
   m.def("dsd_scatter_few", &dsd_scatter_few, py::call_guard<py::gil_scoped_release>());
   m.def("dsd_scatter", &dsd_scatter, py::call_guard<py::gil_scoped_release>());
 }

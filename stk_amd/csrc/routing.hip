@@ -402,12 +402,11 @@ __global__ __launch_bounds__(256) void padded_scatter_kernel(const uint16_t* __r
   }
 }
 
-// scatter_sums (few_rows.h): a thread per token and four columns.  A few thousand threads, bound by latency: the loads of a
-// thread's slices are independent of each other.
+// scatter_sums (few_rows.h): a thread per token and four columns.
 template <int DTYPE, bool WEIGHTED>
-__global__ __launch_bounds__(256) void scatter_sums_kernel(const float* __restrict__ sums, int slices, int64_t slots, int64_t n,
-                                                           const int32_t* __restrict__ slot_rows, int64_t rows, const float* __restrict__ weights,
-                                                           int top_k, int64_t tokens, uint16_t* __restrict__ out, int64_t out_stride) {
+__global__ __launch_bounds__(256) void scatter_sums_kernel(const float* __restrict__ sums, int64_t n, const int32_t* __restrict__ slot_rows, int64_t rows,
+                                                           const float* __restrict__ weights, int top_k, int64_t tokens, uint16_t* __restrict__ out,
+                                                           int64_t out_stride) {
   const int64_t per = n / 4, i = (int64_t)blockIdx.x * 256 + threadIdx.x, t = i / per, c = i % per;
   if (t >= tokens) return;
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
@@ -417,12 +416,7 @@ __global__ __launch_bounds__(256) void scatter_sums_kernel(const float* __restri
     const int row = slot_rows[s];
     if (row < 0 || row >= rows) continue;
     const float w = WEIGHTED ? weights[s] : 1.0f;
-    const float4* from = reinterpret_cast<const float4*>(sums + s * n) + c;
-    float4 v = from[0];
-    for (int j = 1; j < slices; j++) {
-      const float4 u = from[j * slots * per];
-      v.x += u.x, v.y += u.y, v.z += u.z, v.w += u.w;
-    }
+    const float4 v = reinterpret_cast<const float4*>(sums + s * n)[c];
     const float row_sums[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -438,19 +432,19 @@ __global__ __launch_bounds__(256) void scatter_sums_kernel(const float* __restri
 }
 
 template <int DTYPE>
-static void launch_scatter_sums(const float* sums, int slices, int64_t slots, int64_t n, const int32_t* slot_rows, int64_t rows, const float* weights,
-                                int top_k, int64_t tokens, void* out, int64_t out_stride, hipStream_t stream) {
+static void launch_scatter_sums(const float* sums, int64_t n, const int32_t* slot_rows, int64_t rows, const float* weights, int top_k, int64_t tokens,
+                                void* out, int64_t out_stride, hipStream_t stream) {
   const dim3 grid((unsigned)((tokens * (n / 4) + 255) / 256));
   uint16_t* to = static_cast<uint16_t*>(out);
-  if (weights) hipLaunchKernelGGL((scatter_sums_kernel<DTYPE, true>), grid, dim3(256), 0, stream, sums, slices, slots, n, slot_rows, rows, weights, top_k, tokens, to, out_stride);
-  else hipLaunchKernelGGL((scatter_sums_kernel<DTYPE, false>), grid, dim3(256), 0, stream, sums, slices, slots, n, slot_rows, rows, weights, top_k, tokens, to, out_stride);
+  if (weights) hipLaunchKernelGGL((scatter_sums_kernel<DTYPE, true>), grid, dim3(256), 0, stream, sums, n, slot_rows, rows, weights, top_k, tokens, to, out_stride);
+  else hipLaunchKernelGGL((scatter_sums_kernel<DTYPE, false>), grid, dim3(256), 0, stream, sums, n, slot_rows, rows, weights, top_k, tokens, to, out_stride);
 }
 
-int scatter_sums(const float* sums, int slices, int64_t slots, int64_t n, const int32_t* slot_rows, int64_t rows, const float* weights, int top_k,
-                 int64_t tokens, void* out, int64_t out_stride, int dtype, hipStream_t stream) {
+int scatter_sums(const float* sums, int64_t slots, int64_t n, const int32_t* slot_rows, int64_t rows, const float* weights, int top_k, int64_t tokens,
+                 void* out, int64_t out_stride, int dtype, hipStream_t stream) {
   if (tokens * (n / 4) / 256 >= INT32_MAX) return fail(STK_ERR_UNSUPPORTED, "scatter of sums: size exceeds 32-bit range");
-  if (dtype == STK_BF16) launch_scatter_sums<STK_BF16>(sums, slices, slots, n, slot_rows, rows, weights, top_k, tokens, out, out_stride, stream);
-  else launch_scatter_sums<STK_F16>(sums, slices, slots, n, slot_rows, rows, weights, top_k, tokens, out, out_stride, stream);
+  if (dtype == STK_BF16) launch_scatter_sums<STK_BF16>(sums, n, slot_rows, rows, weights, top_k, tokens, out, out_stride, stream);
+  else launch_scatter_sums<STK_F16>(sums, n, slot_rows, rows, weights, top_k, tokens, out, out_stride, stream);
   return check_launch("scatter of sums");
 }
 

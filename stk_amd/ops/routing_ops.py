@@ -104,16 +104,16 @@ def gather_sdd(x, route, rhs, topo, activation=None):
 
 
 def dsd_scatter(a, rhs, route, weights=None):
-    """padded_scatter(stk.ops.dsd(a, rhs), route, weights) in one launch for top_k = 1: the product's store writes
-    every row to its token's place (times its weight), and the padded result is never made.  The result is
-    bit-identical to the two steps.  Used when nothing needs a gradient, the routing is top-1 and the library has the
-    kernel (128-blocks, at least 256 columns, enough work for the eight-wavefront tiles); otherwise the two steps
-    run.  Where the block rows hold few tokens each, only the rows of tokens are computed, for any top_k; the result then
-    differs from the two steps' by the order of the fp32 sums."""
+    """padded_scatter(stk.ops.dsd(a, rhs), route, weights) without the padded result; bit-identical to the two steps.  For
+    top_k = 1 the product's store writes every row to its token's place (times its weight), where the library has the
+    kernel (128-blocks, at least 256 columns, enough work for the eight-wavefront tiles).  Where the block rows hold few tokens
+    each, only the rows of tokens are computed, for any top_k (128-blocks of 16-bit values).  Used when nothing needs a gradient;
+    otherwise the two steps run."""
     from stk_amd.ops import linear_ops
     assert isinstance(a, Matrix)
     if a.is_contiguous() and a.data.is_cuda and a.data.shape[0] > 0 and not applies(a.data, rhs, weights) and not torch.is_autocast_enabled():
-        out = hip_kernels.dsd_scatter_few(a.size(), a.data, a.offsets, a.column_indices, rhs, route.row_slots, route.slot_rows, route.top_k, weights)
+        out = hip_kernels.dsd_scatter_few(a.size(), a.data, a.offsets, a.column_indices, rhs, route.row_slots, route.slot_rows, route.top_k, weights,
+                                          a.offsets_t, a.column_indices_t)
         if out is not None:
             return out
     if route.top_k == 1 and a.is_contiguous() and a.data.is_cuda and not applies(a.data, rhs, weights):

@@ -1,5 +1,5 @@
-"""The routed products on block rows with few tokens each: stk_sdd_gather's small tiles bit for bit against the two calls
-(same sums in the same order), stk_dsd_scatter_few against the two calls' arithmetic in fp32.
+"""The routed products on block rows with few tokens each, stk_sdd_gather's small tiles and stk_dsd_scatter_few: bit for bit against
+the two calls (same sums in the same order, cut where stk_dsd cuts its last round), and against float64.
 
 Rows in use per block row are chosen at the edges of the tiles (1, 31 .. 33, 64, 65, 128, none)."""
 import pytest
@@ -115,3 +115,93 @@ def test_a_plan_is_built_for_the_gathered_product_only_where_it_is_read(monkeypa
         del topo.offsets._stk_plan, built[:]
         stk.ops.gather_sdd(x, r, w1, topo)
     assert bool(built) == reads
+
+
+# (slots of the experts, hidden, ffn, top_k, spare block rows, whether dsd cuts a tile of its last round): tiles of 64 and of 128 columns;
+# one round of tiles, all of them cut, and a second one of 28; pairs and threes of block rows in the lists; no cut
+SLICED = [([8] * 16, 2048, 8192, 2, 0, True), ([16] * 64, 1024, 4096, 1, 7, True), ([290, 190] + [5] * 6, 2048, 8192, 1, 0, True),
+          ([4] * 8, 1024, 9088, 1, 2, False)]
+
+
+def _random_layer(counts, hidden, ffn, top_k, spare, dtype=torch.bfloat16):
+    _, top, r, topo, _, _ = _layer(counts, 128, 128, top_k, dtype, spare)
+    topo = stk.ops.dmoe_topology(r.padded_bins, 128, r.row_slots.numel() // 128, ffn // 128, dtype=dtype)
+    topo.data.normal_()
+    w2 = torch.empty(len(counts) * ffn, hidden, dtype=dtype, device=DEV).normal_()
+    return r, topo, w2, torch.rand(top.shape, device=DEV) + 0.5
+
+
+@pytest.mark.parametrize("counts,hidden,ffn,top_k,spare,cut", SLICED)
+def test_dsd_scatter_of_few_rows_is_dsd_then_scatter(monkeypatch, counts, hidden, ffn, top_k, spare, cut):
+    r, m, w2, weights = _random_layer(counts, hidden, ffn, top_k, spare)
+    args = (m.size(), m.data, m.offsets, m.column_indices, w2, r.row_slots, r.slot_rows, top_k, weights, m.offsets_t, m.column_indices_t)
+    wants = []
+    for sliced in (True, False):
+        monkeypatch.setattr(hip_kernels, "SLICE_LAST_ROUND", sliced)
+        wants.append(stk.ops.padded_scatter(stk.ops.dsd(m, w2), r, weights))
+        got = hip_kernels.dsd_scatter_few(*args)
+        assert got is not None and torch.equal(_bits(got), _bits(wants[-1])), sliced
+        assert torch.equal(_bits(stk.ops.dsd_scatter(m, w2, r, weights)), _bits(got))
+    assert torch.equal(*map(_bits, wants)) != cut
+    # a K-major second weight, int32 indices, less room for partial tiles
+    monkeypatch.setattr(hip_kernels, "SLICE_LAST_ROUND", True)
+    monkeypatch.setattr(hip_kernels, "DSD_WORKSPACE_SLOTS", 100)
+    m = stk.Matrix(m.size(), m.data, m.row_indices.int(), m.column_indices.int(), m.offsets.clone(), m.column_indices_t.int(), m.offsets_t, m.block_offsets_t)
+    w2 = w2.t().contiguous().t()
+    assert torch.equal(_bits(stk.ops.dsd_scatter(m, w2, r, weights)), _bits(stk.ops.padded_scatter(stk.ops.dsd(m, w2), r, weights)))
+    hip_kernels.release_workspaces()
+    monkeypatch.setattr(hip_kernels, "FUSION", False)
+    assert hip_kernels.dsd_scatter_few(*args) is None
+
+
+def test_dsd_scatter_of_few_rows_without_some_slots():
+    # slots without a row, and rows of the layout behind the matrix: left out, like in the scatter
+    r, m, w2, weights = _random_layer(COUNTS[1], 256, 2048, 2, 1)
+    slot_rows, row_slots = r.slot_rows.clone(), r.row_slots.clone()
+    gone = torch.arange(0, slot_rows.numel(), 3, device=DEV)
+    row_slots[slot_rows[gone].long()] = -1
+    slot_rows[gone] = -1
+    slot_rows[1] = m.size()[0]
+    row_slots[r.slot_rows[1].long()] = -1
+    r = r._replace(slot_rows=slot_rows, row_slots=row_slots)
+    assert hip_kernels.dsd_scatter_few(m.size(), m.data, m.offsets, m.column_indices, w2, r.row_slots, r.slot_rows, 2, weights) is not None
+    assert torch.equal(_bits(stk.ops.dsd_scatter(m, w2, r, weights)), _bits(stk.ops.padded_scatter(stk.ops.dsd(m, w2), r, weights)))
+
+
+def test_a_layer_of_few_rows_on_a_stream_under_autocast_and_in_a_graph():
+    tokens, experts, hidden, ffn, dtype = 96, 16, 256, 4096, torch.bfloat16
+    capacity = stk.ops.route_capacity(2 * tokens, experts, 128)
+    x = torch.randn(tokens, hidden, device=DEV).to(dtype)
+    w1, w2 = (torch.randn(*shape, device=DEV).to(dtype) * 0.05 for shape in ((hidden, experts * ffn), (experts * ffn, hidden)))
+    weights, top = torch.rand(tokens, 2, device=DEV), torch.zeros(tokens, 2, dtype=torch.int32, device=DEV)
+    choose = lambda seed: top.copy_(torch.rand(tokens, experts, generator=torch.Generator().manual_seed(seed)).topk(2).indices)
+
+    def layer(routed):
+        r = stk.ops.route(top, experts, 128, capacity)
+        topo = stk.ops.dmoe_topology(r.padded_bins, 128, capacity // 128, ffn // 128, dtype=dtype)
+        if routed:
+            return stk.ops.dsd_scatter(stk.ops.gather_sdd(x, r, w1, topo, "silu"), w2, r, weights)
+        h = stk.ops.sdd_fused(stk.ops.padded_gather(x, r), w1, topo, "silu")
+        return stk.ops.padded_scatter(stk.ops.dsd(h, w2), r, weights)
+
+    with torch.no_grad():
+        choose(0)
+        assert torch.equal(_bits(layer(True)), _bits(layer(False)))
+        r, h, rhs, wts = _random_layer([4] * 8, 256, 1024, 1, 0)
+        with torch.autocast("cuda", dtype=torch.float16):     # casts the product's operands
+            got, want = stk.ops.dsd_scatter(h, rhs, r, wts), stk.ops.padded_scatter(stk.ops.dsd(h, rhs), r, wts)
+        assert got.dtype == want.dtype == torch.float16 and torch.equal(_bits(got), _bits(want))
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            got = layer(True)
+        torch.cuda.current_stream().wait_stream(side)
+        assert torch.equal(_bits(got), _bits(layer(False)))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out = layer(True)
+        for seed in (1, 2, 3):
+            choose(seed)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(_bits(out), _bits(layer(False))), seed
