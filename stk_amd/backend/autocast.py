@@ -24,6 +24,11 @@ def _cast_tree(x, dtype):
     return x
 
 
+def casts(*tensors):
+    """Whether a function wrapped by custom_fwd would be called on other tensors than these."""
+    return torch.is_autocast_enabled() and any(_castable(t) and t.dtype != torch.get_autocast_gpu_dtype() for t in tensors)
+
+
 def custom_fwd(fwd):
     @functools.wraps(fwd)
     def wrapper(*args, **kwargs):

@@ -8,7 +8,7 @@ from collections import namedtuple
 
 import torch
 
-from stk_amd.backend import hip_kernels
+from stk_amd.backend import autocast, hip_kernels
 from stk_amd.backend.autograd import applies
 from stk_amd.matrix import Matrix
 
@@ -87,11 +87,11 @@ def padded_scatter(x, route, weights=None):
 def gather_sdd(x, route, rhs, topo, activation=None):
     """stk.ops.sdd_fused(padded_gather(x, route), rhs, topo, activation) in one launch: the sampled product reads the
     token rows where they lie, and the padded copy of x is never made.  The result is bit-identical to the two steps.
-    Used when nothing needs a gradient (the backward pass of the product needs the padded copy anyway) and the library
-    has the kernel (128-blocks); otherwise the two steps run."""
+    Used when nothing needs a gradient (the backward pass of the product needs the padded copy anyway), autocast does not cast
+    the operands and the library has the kernel (128-blocks); otherwise the two steps run."""
     from stk_amd.ops import linear_ops
     assert isinstance(topo, Matrix) and topo.is_contiguous()
-    if x.is_cuda and not applies(x, rhs):
+    if x.is_cuda and not applies(x, rhs) and not autocast.casts(x, rhs):
         out = torch.empty_like(topo.data)
         # (one plan for both directions: the product that follows on the same topology walks it the other way)
         if hip_kernels.sdd_gather_reads_plan(x, route.top_k, topo.size()):
@@ -107,16 +107,17 @@ def dsd_scatter(a, rhs, route, weights=None):
     """padded_scatter(stk.ops.dsd(a, rhs), route, weights) without the padded result; bit-identical to the two steps.  For
     top_k = 1 the product's store writes every row to its token's place (times its weight), where the library has the
     kernel (128-blocks, at least 256 columns, enough work for the eight-wavefront tiles).  Where the block rows hold few tokens
-    each, only the rows of tokens are computed, for any top_k (128-blocks of 16-bit values).  Used when nothing needs a gradient;
-    otherwise the two steps run."""
+    each, only the rows of tokens are computed, for any top_k (128-blocks of 16-bit values).  Used when nothing needs a gradient and
+    autocast does not cast the operands; otherwise the two steps run."""
     from stk_amd.ops import linear_ops
     assert isinstance(a, Matrix)
-    if a.is_contiguous() and a.data.is_cuda and a.data.shape[0] > 0 and not applies(a.data, rhs, weights) and not torch.is_autocast_enabled():
+    here = a.is_contiguous() and a.data.is_cuda and not applies(a.data, rhs, weights) and not autocast.casts(a.data, rhs)
+    if here and a.data.shape[0] > 0:
         out = hip_kernels.dsd_scatter_few(a.size(), a.data, a.offsets, a.column_indices, rhs, route.row_slots, route.slot_rows, route.top_k, weights,
                                           a.offsets_t, a.column_indices_t)
         if out is not None:
             return out
-    if route.top_k == 1 and a.is_contiguous() and a.data.is_cuda and not applies(a.data, rhs, weights):
+    if here and route.top_k == 1:
         tokens = route.slot_rows.numel()
         out = torch.empty((tokens, rhs.shape[1]), dtype=a.dtype, device=a.data.device)
         if hip_kernels.dsd_scatter(a.size(), a.data, a.offsets, a.column_indices, a.offsets_t, a.column_indices_t, rhs,

@@ -187,10 +187,10 @@ def test_a_layer_of_few_rows_on_a_stream_under_autocast_and_in_a_graph():
     with torch.no_grad():
         choose(0)
         assert torch.equal(_bits(layer(True)), _bits(layer(False)))
-        r, h, rhs, wts = _random_layer([4] * 8, 256, 1024, 1, 0)
-        with torch.autocast("cuda", dtype=torch.float16):     # casts the product's operands
-            got, want = stk.ops.dsd_scatter(h, rhs, r, wts), stk.ops.padded_scatter(stk.ops.dsd(h, rhs), r, wts)
-        assert got.dtype == want.dtype == torch.float16 and torch.equal(_bits(got), _bits(want))
+        for autocast in (torch.float16, dtype):               # casts the products' operands, or leaves them
+            with torch.autocast("cuda", dtype=autocast):
+                got, want = layer(True), layer(False)
+            assert got.dtype == want.dtype == autocast and torch.equal(_bits(got), _bits(want))
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):

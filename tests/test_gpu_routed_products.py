@@ -170,6 +170,16 @@ def test_dsd_scatter_cuts_its_last_round_where_dsd_does(hidden):
     assert _same_bits(out, stk.ops.padded_scatter(stk.ops.dsd(h, w2), r))
 
 
+def test_autocast_casts_the_operands_of_both():
+    x, r, topo, w1, w2 = _layer(8192, 1024, 8, 2560, 1, torch.bfloat16, 4)
+    h = stk.ops.sdd(stk.ops.padded_gather(x, r), w1, topo)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        got, want = stk.ops.gather_sdd(x, r, w1, topo).data, stk.ops.sdd(stk.ops.padded_gather(x, r), w1, topo).data
+        assert got.dtype == want.dtype == torch.float16 and _same_bits(got, want)
+        got, want = stk.ops.dsd_scatter(h, w2, r), stk.ops.padded_scatter(stk.ops.dsd(h, w2), r)
+        assert got.dtype == want.dtype == torch.float16 and _same_bits(got, want)
+
+
 def test_dsd_scatter_falls_back_where_it_has_no_kernel():
     # little work (four-wavefront tiles in stk_dsd), top-2, a transposed operand, gradients: the two steps run
     x, r, topo, w1, w2 = _layer(700, 256, 4, 256, 1, torch.bfloat16, 2)
