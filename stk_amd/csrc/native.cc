@@ -469,6 +469,7 @@ Tensor rows16(const Tensor& x_) {
 int64_t row_stride(const Tensor& x) { return x.numel() && x.size(0) > 1 ? x.stride(0) : std::max<int64_t>(x.size(1), 1); }
 OptTensor weights32(const OptTensor& weights, int64_t slots) {
   if (!weights) return {};
+  if (weights->numel() > 0) need_gpu(*weights);   // (a kernel reads them: an address in host memory would be a fault)
   Tensor w = weights->detach().reshape({-1}).to(at::kFloat).contiguous();
   if (w.numel() != slots)
     raise(PyExc_AssertionError, "one weight per slot: " + std::to_string(w.numel()) + " weights for " + std::to_string(slots) + " slots");

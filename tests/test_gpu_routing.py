@@ -227,6 +227,21 @@ def test_empty_and_errors():
         stk.ops.padded_scatter(torch.zeros(16, 16, dtype=torch.bfloat16, device=DEV), r, torch.ones(3, device=DEV))
 
 
+def test_weights_in_host_memory_are_refused():
+    # 4 slots: the few-row product, 9000: the scattered one (or the two steps)
+    for tokens, experts, hidden, ffn in ((4, 4, 128, 128), (9000, 8, 1024, 2560)):
+        r = stk.ops.route(torch.randint(0, experts, (tokens, 1), dtype=torch.int32, device=DEV), experts, 128)
+        rows = r.row_slots.numel()
+        m = stk.ops.dmoe_topology(r.padded_bins, 128, rows // 128, ffn // 128, dtype=torch.bfloat16)
+        x = torch.zeros(tokens, hidden, dtype=torch.bfloat16, device=DEV)
+        rhs = torch.zeros(m.size()[1], hidden, dtype=torch.bfloat16, device=DEV)
+        weights = torch.ones(tokens, 1)
+        for call in (lambda: stk.ops.dsd_scatter(m, rhs, r, weights), lambda: stk.ops.padded_scatter(stk.ops.padded_gather(x, r), r, weights),
+                     lambda: hip_kernels.padded_gather(x, r.row_slots, 1, weights)):
+            with pytest.raises(RuntimeError, match="ROCm GPU only"):
+                call()
+
+
 def test_routed_layer_gradients_against_dense_autograd():
     """Backward of route -> gather -> sdd -> dsd -> weighted scatter against torch autograd on the same layer written
     with per-expert dense fp32 products.  The HIP path rounds four intermediate tensors to bf16 (2^-9 relative each), the
