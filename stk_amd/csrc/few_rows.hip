@@ -5,11 +5,12 @@
 // wavefronts, with a ring of 80 KB and two workgroups per compute unit: one's start and stores lie under the other's stream, and
 // the many short tiles leave no long last round.  On 32 rows that is three 16 KB stages of weights in flight per workgroup, on
 // 64 two, on 128 one (four of 32-deep K-tiles instead: 118 -> 140 us for the second product of 4096 tokens over 64 experts).
-// 64 tokens top-2 over 64 experts (1024 x 4096, bf16, 466 MB of weights a product): the wide tiles take 110 us for the first
-// product and 104 for the second with its scatter, these 94 (with the 59 MB of its result 5.6 TB/s) and 83 (5.6 TB/s); 300 tokens
-// over 16 experts (2048 x 8192) 101 and 128 us, these 101 and 94; 16 tokens 27 and 67 us, these 23 and 30.  Row-major weights
-// are loaded non-temporally (without the hint: 109 us for the first product), K-major ones are not.  Workgroups of the first
-// product in plain order: 95 us.
+// 128 tokens over 58 of 64 experts (1024 x 4096, bf16, 487 MB of weights a product): the wide tiles take 114 us for the first
+// product and 104 for the second with its scatter, these 100 (with the 61 MB of its result 5.5 TB/s) and 82 (5.9 TB/s); 300 tokens
+// top-2 over 16 experts (2048 x 8192) 105 and 128 us, these 104 and 94; 16 tokens top-2 over 8 experts (1024 x 4096) 20 and
+// 65 us, these 15 and 24.  Row-major weights are loaded non-temporally (without the hint the first product takes 15 us more), K-major
+// ones are not.  With the workgroups in plain order the second product takes 9 us more; in eight contiguous shares of the list
+// as long, but 70 instead of 46 us where four experts share the block rows unevenly.
 #include "dsd_tile.h"
 #include "few_rows.h"
 #include "sdd_tile.h"
