@@ -38,7 +38,9 @@ __device__ __forceinline__ void wait_younger(int younger) {
 }
 
 // Four wavefronts on a tile of 32 IM rows and TN columns, TN / 32 of them side by side, the others below with their share of
-// the rows (with 32 rows of 64 columns two of them only load).
+// the rows (with 32 rows of 64 columns two of them only load).  On 64 columns four more do the loading: issuing the transfers
+// takes as long as multiplying, and a workgroup that has a compute unit to itself would do one behind the other (second product of
+// 4 experts of 256 x 8192 41 -> 34 us, 16 of 256 x 4096 24 -> 20, 8 of 1024 x 4096 the same).
 template <int IM, int TN, bool BK>
 struct FewTile {
   using OpA = Operand<32 * IM, true, kFewKT, kFewThreads>;
@@ -46,11 +48,15 @@ struct FewTile {
   static constexpr int kAcross = TN / 32, kDown = 4 / kAcross, kMine = IM < kDown ? 1 : IM / kDown;   // row strips of 32 a wavefront
   static constexpr int kStage = OpA::kBytes + OpB::kBytes, kStages = kFewLds / kStage, kLoads = IM + OpB::kSlicesPerWave;
   static_assert(OpA::kSlicesPerWave == IM && kStages >= 2 && (kStages - 2) * kLoads < 64, "the ring");
-  int lane, wave, column, strip;   // of this wavefront: first column, first strip
-  bool multiplies;
+  static constexpr bool kLoaders = TN == 64;
+  static constexpr int kThreads = kLoaders ? 512 : 256;
+  int lane, wave, column, strip;   // of this wavefront: its number among the four, first column, first strip
+  bool loads, multiplies;
   __device__ __forceinline__ FewTile() {
-    lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
-    column = 32 * (wave % kAcross), strip = wave / kAcross * kMine, multiplies = strip < IM;
+    lane = threadIdx.x & 63;
+    const int all = uniform(threadIdx.x >> 6);
+    wave = all & 3, loads = !kLoaders || all >= 4;
+    column = 32 * (wave % kAcross), strip = wave / kAcross * kMine, multiplies = all < 4 && strip < IM;
   }
 };
 
@@ -77,13 +83,14 @@ __device__ __forceinline__ void few_rows_loop(const Tile& w, f32x16_t (&acc)[Til
 #pragma unroll
     for (int i = 0; i < OpA::kSlicesPerWave; i++) dma16(ga, offa[i], stage + (i * 4 + w.wave) * 1024);
   };
-  for (int t = 0; t < S - 1 && t < ntiles; t++) issue();
+  if (w.loads)
+    for (int t = 0; t < S - 1 && t < ntiles; t++) issue();
   for (int t = 0; t < ntiles; t++) {
     // K-tile t has landed; up to S - 2 younger ones stay in flight
-    wait_younger<S - 2, Tile::kLoads>(ntiles - 1 - t);
+    if (w.loads) wait_younger<S - 2, Tile::kLoads>(ntiles - 1 - t);
     // every wavefront's part of it is visible, and every wavefront has read K-tile t - 1, whose stage is refilled now
     __syncthreads();
-    if (t + S - 1 < ntiles) issue();
+    if (w.loads && t + S - 1 < ntiles) issue();
     const char* stage = smem + use * Tile::kStage;
     use = use + 1 == S ? 0 : use + 1;
     if (w.multiplies) {
@@ -237,7 +244,7 @@ __device__ __forceinline__ void dsd_few_tile(const DsdFewArgs& g, int r, int row
 }
 
 template <int TN, bool BK, bool BF16>
-__global__ __launch_bounds__(kFewThreads, 2) void dsd_few_kernel(DsdFewArgs g) {
+__global__ __launch_bounds__((FewTile<1, TN, BK>::kThreads), (FewTile<1, TN, BK>::kThreads / 128)) void dsd_few_kernel(DsdFewArgs g) {
   extern __shared__ __align__(16) char smem[];
   const int bid = xcd_grouped<8>(blockIdx.x, gridDim.x), r = bid / g.tiles, n0 = bid % g.tiles * TN;
   const int rows = uniform(rows_in_use(g.row_slots, g.slots, r, threadIdx.x & 63));
@@ -251,7 +258,7 @@ template <int TN, bool BK, bool BF16>
 static void launch_dsd_few(const DsdFewArgs& g, hipStream_t stream) {
   static const int once = (set_lds_limit(&dsd_few_kernel<TN, BK, BF16>, kFewLds), 0);
   (void)once;
-  hipLaunchKernelGGL((dsd_few_kernel<TN, BK, BF16>), dim3(g.block_rows * g.tiles), dim3(kFewThreads), kFewLds, stream, g);
+  hipLaunchKernelGGL((dsd_few_kernel<TN, BK, BF16>), dim3(g.block_rows * g.tiles), dim3(FewTile<1, TN, BK>::kThreads), kFewLds, stream, g);
 }
 template <int TN>
 static void launch_dsd_few(const DsdFewArgs& g, bool bk, bool bf16, hipStream_t stream) {
@@ -263,9 +270,9 @@ static void launch_dsd_few(const DsdFewArgs& g, bool bk, bool bf16, hipStream_t 
 // what a workgroup moves per K-tile is the token rows, which wider tiles share.  us with 128 / 64 columns, and where the work
 // allows it two steps: 64 tiles of 128 (8 experts, 1024 columns, 4096 deep) 31 / 24, two steps 65; 128 tiles (16 experts)
 // 34 / 30, 68; 216 (27 of 32 experts) 41 / 50, 76; 240 (15 experts, 2048 columns, 8192 deep) 85 / 100, 120.  32 columns are as
-// slow as 64 or slower everywhere: a compute unit takes in about one 128-byte line in 6 cycles.  The sums of a tile cannot be
-// split over k between workgroups without another order: with up to eight slices 8 experts of 1024 x 4096 took 20 us, 4 of
-// 256 x 8192 21, now 41 (two steps 112).
+// slow as 64 or slower everywhere.  The sums of a tile cannot be split over k between workgroups without another order, and a
+// compute unit by itself takes in 40 - 60 GB/s: with up to eight slices 8 experts of 1024 x 4096 took 20 us, 8 of
+// 512 x 8192 23, now 40 (two steps 117), 4 of 256 x 8192 21, now 34 (112).
 static int few_columns(int64_t block_rows, int64_t n) { return n % 128 == 0 && block_rows * (n / 128) >= compute_units() * 3 / 4 ? 128 : 64; }
 
 }  // namespace stk
