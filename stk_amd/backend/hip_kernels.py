@@ -450,9 +450,10 @@ def padded_scatter_weight_gradient(x, grad, slot_rows, top_k):
     return _lib.native().padded_scatter_weight_gradient(x, grad, slot_rows, top_k)
 
 
-def sdd_gather_reads_plan(x, top_k, shape):
-    """Whether sdd_gather of these token rows makes use of a plan: not where the block rows hold few slots each."""
-    return x.dim() != 2 or bool(_lib.native().sdd_gather_reads_plan(shape[0], x.shape[1], x.shape[0] * top_k))
+def sdd_gather_reads_plan(x, top_k, shape, blocking=128):
+    """Whether sdd_gather of these token rows, or what runs where it has no kernel, makes use of a plan: not where block rows of
+    128 hold few slots each."""
+    return blocking != 128 or x.dim() != 2 or bool(_lib.native().sdd_gather_reads_plan(shape[0], x.shape[1], x.shape[0] * top_k))
 
 
 def sdd_gather(x, row_slots, top_k, rhs, shape, out, offsets, row_indices, column_indices, activation=None):

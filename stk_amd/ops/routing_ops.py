@@ -94,7 +94,7 @@ def gather_sdd(x, route, rhs, topo, activation=None):
     if x.is_cuda and not applies(x, rhs) and not autocast.casts(x, rhs):
         out = torch.empty_like(topo.data)
         # (one plan for both directions: the product that follows on the same topology walks it the other way)
-        if hip_kernels.sdd_gather_reads_plan(x, route.top_k, topo.size()):
+        if hip_kernels.sdd_gather_reads_plan(x, route.top_k, topo.size(), topo.blocking):
             hip_kernels.prepare_plan(topo.data, topo.offsets, topo.column_indices, topo.offsets_t, topo.column_indices_t)
         if hip_kernels.sdd_gather(x, route.row_slots, route.top_k, rhs, topo.size(), out, topo.offsets, topo.row_indices, topo.column_indices,
                                   activation):

@@ -117,6 +117,20 @@ def test_a_plan_is_built_for_the_gathered_product_only_where_it_is_read(monkeypa
     assert bool(built) == reads
 
 
+def test_one_plan_for_a_layer_of_64_blocks():
+    # (which has no gathered product: the first of its two steps finds the plan that the second will ask for)
+    top = torch.arange(8, dtype=torch.int32, device=DEV).view(-1, 1)
+    r = stk.ops.route(top, 8, 64)
+    m = stk.ops.dmoe_topology(r.padded_bins, 64, 8, 4, dtype=torch.bfloat16)
+    m = stk.Matrix(m.size(), m.data, m.row_indices, m.column_indices, m.offsets.clone(), m.column_indices_t, m.offsets_t, m.block_offsets_t)
+    x = torch.randn(8, 128, device=DEV).to(torch.bfloat16)
+    w1 = torch.randn(128, m.size()[1], device=DEV).to(torch.bfloat16)
+    with torch.no_grad():
+        stk.ops.gather_sdd(x, r, w1, m)
+    plan = m.offsets._stk_plan[1]
+    assert hip_kernels.fusion_plan(m.offsets, m.column_indices, m.offsets_t, m.column_indices_t, blocking=64) is plan
+
+
 # (slots of the experts, hidden, ffn, top_k, spare block rows, whether dsd cuts a tile of its last round): tiles of 64 and of 128 columns;
 # one round of tiles, all of them cut, and a second one of 28; pairs and threes of block rows in the lists; no cut
 SLICED = [([8] * 16, 2048, 8192, 2, 0, True), ([16] * 64, 1024, 4096, 1, 7, True), ([290, 190] + [5] * 6, 2048, 8192, 1, 0, True),
